@@ -1337,8 +1337,70 @@ const TileCfg kTiles[] = {
     {144, 128, launch_big<144, 128, 3, 2, 3>},                            // 15: 3 stages
     {144, 128, launch_big<144, 128, 3, 2, 4>},                            // 16: 4 stages
     {288, 128, launch_big<288, 128, 2, 4, 3>},                            // 17: 3 stages
+    // above 320 tokens (kCosts picks among these and tiles 2-4 and 9-12): wave tiles of 48 x 32 to
+    // 96 x 64 on 6 to 16 waves, sized so that some tile fills one round of 256 CUs at any row count;
+    // the two-stage ones of 64 and 56 KB run two workgroups per CU
+    {144, 128, launch_big<144, 128, 3, 4, 3>},                            // 18: 12 waves
+    {192, 128, launch_big<192, 128, 4, 2, 2>},                            // 19
+    {192, 128, launch_big<192, 128, 4, 2, 3>},                            // 20
+    {144, 256, launch_big<144, 256, 3, 4, 3>},                            // 21: 12 waves
+    {192, 192, launch_big<192, 192, 4, 3, 2>},                            // 22: 12 waves
+    {96, 128, launch_big<96, 128, 2, 4, 4>},                              // 23
+    {96, 128, launch_big<96, 128, 2, 4, 2>},                              // 24
+    {128, 128, launch_big<128, 128, 2, 4, 3>},                            // 25
+    {256, 256, launch_big<256, 256, 4, 4, 2>},                            // 26: 16 waves
+    {288, 256, launch_big<288, 256, 2, 8, 2>},                            // 27: 16 waves
+    {256, 128, launch_big<256, 128, 4, 4, 3>},                            // 28: 16 waves
+    {144, 96, launch_big<144, 96, 3, 3, 4>},                              // 29: 9 waves
 };
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
+
+// Fitted costs (tile_cost) of the tiles used above 320 tokens: c, a and b for the plain and GELU
+// stores, QKV + RoPE, and the fp32 residual and partial-sum epilogues.
+const TileCost kCosts[] = {
+    {2, {{0.25f, 0.374f, 0.00f}, {3.80f, 0.300f, 0.00f}, {3.71f, 0.235f, 1.04f}}},  // 96 x 64
+    {3, {{1.35f, 0.287f, 0.00f}, {0.20f, 0.298f, 0.00f}, {3.45f, 0.181f, 0.79f}}},  // 64 x 64
+    {4, {{2.48f, 0.555f, 0.00f}, {2.15f, 0.722f, 0.00f}, {1.48f, 0.375f, 3.43f}}},  // 144 x 64
+    {9, {{0.00f, 0.173f, 0.00f}, {3.31f, 0.129f, 0.00f}, {1.26f, 0.090f, 1.12f}}},  // 48 x 32
+    {10, {{2.85f, 0.271f, 0.00f}, {2.44f, 0.279f, 0.00f}, {1.48f, 0.147f, 2.28f}}},  // 48 x 64
+    {11, {{2.53f, 0.319f, 0.00f}, {1.89f, 0.324f, 0.00f}, {1.47f, 0.172f, 2.71f}}},  // 64 x 64
+    {12, {{-3.05f, 0.287f, 0.00f}, {2.48f, 0.211f, 0.00f}, {1.45f, 0.113f, 1.86f}}},  // 32 x 64
+    {18, {{2.19f, 0.787f, 0.00f}, {1.10f, 0.811f, 0.00f}, {0.79f, 0.528f, 5.23f}}},  // 144 x 128
+    {19, {{8.94f, 0.644f, 0.00f}, {6.75f, 0.668f, 0.00f}, {3.35f, 0.684f, 3.14f}}},  // 192 x 128
+    {20, {{0.78f, 1.029f, 0.00f}, {0.37f, 1.208f, 0.00f}, {0.74f, 0.626f, 6.26f}}},  // 192 x 128
+    {21, {{-0.16f, 1.402f, 0.00f}, {-0.84f, 1.527f, 0.00f}, {-0.86f, 0.838f, 9.16f}}},  // 144 x 256
+    {22, {{2.68f, 1.270f, 0.00f}, {-0.48f, 1.319f, 0.00f}, {-0.25f, 0.866f, 7.63f}}},  // 192 x 192
+    {23, {{2.59f, 0.602f, 0.00f}, {3.17f, 0.724f, 0.00f}, {1.61f, 0.429f, 3.57f}}},  // 96 x 128
+    {24, {{8.86f, 0.396f, 0.00f}, {6.93f, 0.372f, 0.00f}, {5.18f, 0.459f, 0.89f}}},  // 96 x 128
+    {25, {{1.63f, 0.753f, 0.00f}, {1.38f, 0.918f, 0.00f}, {1.14f, 0.490f, 4.60f}}},  // 128 x 128
+    {26, {{-2.32f, 2.061f, 0.00f}, {-1.76f, 1.971f, 0.00f}, {-2.81f, 1.197f, 13.58f}}},  // 256 x 256
+    {27, {{-1.88f, 2.319f, 0.00f}, {-1.23f, 2.289f, 0.00f}, {-4.66f, 1.369f, 16.58f}}},  // 288 x 256
+    {28, {{-0.66f, 1.286f, 0.00f}, {-0.80f, 1.360f, 0.00f}, {-0.57f, 0.702f, 9.04f}}},  // 256 x 128
+    {29, {{2.27f, 0.703f, 0.00f}, {2.06f, 0.813f, 0.00f}, {1.31f, 0.467f, 4.25f}}},  // 144 x 96
+};
+
+// the K / splits a tile can run (as gemm_launch_cfg checks it)
+bool tile_takes_k(const TileCfg& t, int64_t kslice) {
+  return kslice % t.k_gran == 0 && kslice <= t.k_max &&
+         (t.k_gran == 64 || ((kslice / t.k_gran) & (kslice / t.k_gran - 1)) == 0);
+}
+
+// the cheapest tile above 320 tokens; *us (optional) its cost
+int cheapest_tile(int64_t M, int64_t N, int64_t K, int splits, int kind, float* us) {
+  int best = 2;
+  float best_us = kNever;
+  for (const TileCost& c : kCosts) {
+    const TileCfg& t = kTiles[c.tile];
+    if (!tile_takes_k(t, K / splits) || (t.no_fp8_epi && kind == OASIS_EPI_GELU_TANH_FP8)) continue;
+    const float cost = tile_cost(c, t.bm, t.bn, M, N, K / splits / 64, splits, kind);
+    if (cost < best_us) {
+      best_us = cost;
+      best = c.tile;
+    }
+  }
+  if (us) *us = best_us;
+  return best;
+}
 
 }  // namespace
 
@@ -1346,43 +1408,48 @@ namespace oasis {
 
 // Default tile per shape, from timings of each projection on MI355X with cold weights (hipGraphs
 // of 100 launches over rotating weight sets):
-//   - 2048+ tokens: the 8-wave tall tiles, the width that fills the last round of 256 workgroups best;
+//   - above 320 tokens the cheapest tile by kCosts;
 //   - below, where the K slice suits the wave-split kernel (256, 512, 1024 or 2048 long):
 //       FC1 (GELU): 48 x 64 (tile 10) at one 144-token frame, 80-row tiles every 72 rows x 64
 //       (tile 8) up to 320 tokens (8.51 us at 288 against 9.36 on 96 x 64 tiles);
-//       split-K partials of K <= 1024 (O): 48 x 32 (tile 9) up to 320 tokens, 48 x 64 (tile 10) above;
+//       split-K partials of K <= 1024 (O): 48 x 32 (tile 9);
 //       split-K partials of longer K (FC2): tile 10 at one frame, tile 8 up to 320 tokens;
 //       other epilogues (QKV + RoPE): 32 x 64 (tile 12) at one frame, 64 x 64 (tile 11) up to 320;
-//   - otherwise the shared-ring kernels: FC1 on 144 x 64 six-wave tiles (tile 4) from 512 tokens (the
-//     VAE's 576) and 96 x 64 (tile 2) else; split-K partials on 32 x 64 (tile 0) for short slices up to
-//     320 tokens and tile 2 else; other epilogues on 32 x 64 (tile 1), 64 x 64 (tile 3) from 512 tokens.
+//   - otherwise the shared-ring kernels: FC1 on 64 x 64 (tile 3) at one frame and 96 x 64 (tile 2)
+//     else; split-K partials on 32 x 64 (tile 0) for short slices and tile 2 else; other epilogues on
+//     32 x 64 (tile 1).
 int auto_tile(int64_t M, int64_t N, int64_t K, int splits, int kind) {
-  if (M >= 2048) return large_token_tile(M, N, kind != OASIS_EPI_GELU_TANH_FP8, 5, 6, 7);
+  if (M > 320) return cheapest_tile(M, N, K, splits, kind, nullptr);
   const int64_t Kslice = K / splits;
   const bool wave_k = Kslice % 256 == 0 && Kslice <= 2048 && ((Kslice / 256) & (Kslice / 256 - 1)) == 0;
   const bool gelu = kind == OASIS_EPI_GELU_TANH || kind == OASIS_EPI_GELU_ERF || kind == OASIS_EPI_GELU_TANH_FRAG;
-  if (wave_k && M <= 320) {
+  if (wave_k) {
     if (gelu) return M <= 160 ? 10 : 8;
     if (kind == OASIS_EPI_PARTIAL_F32) return K <= 1024 ? 9 : (M <= 160 ? 10 : 8);
     if (kind != OASIS_EPI_GELU_TANH_FP8) return M <= 160 ? 12 : 11;
   }
-  if (wave_k && kind == OASIS_EPI_PARTIAL_F32 && K <= 1024) return 10;
-  if (gelu) return M <= 160 ? 3 : (M >= 512 ? 4 : 2);
-  if (kind == OASIS_EPI_PARTIAL_F32) {
-    if (M <= 160) return Kslice <= 256 ? 0 : 2;
-    return M <= 320 && Kslice <= 512 ? 0 : 2;
-  }
-  return M >= 512 ? 3 : 1;
+  if (gelu) return M <= 160 ? 3 : 2;
+  if (kind == OASIS_EPI_PARTIAL_F32) return Kslice <= (M <= 160 ? 256 : 512) ? 0 : 2;
+  return 1;
 }
 
-// Split-K count for the default tile of a large-token split-K product: K slices until the
-// launch has at least 256 workgroups (one per CU), within max_splits and whole 64-wide K tiles.
+// Split-K count above 320 tokens: 1 (the residual in the epilogue), 2, 4 or 8 K slices, within
+// max_splits and whole 64-wide K tiles, whichever the fitted costs of the GEMM and of the slices'
+// reads make cheapest.
 int gemm_auto_splits(int64_t M, int64_t N, int64_t K, int max_splits) {
-  const TileCfg& t = kTiles[auto_tile(M, N, K, 1, OASIS_EPI_PARTIAL_F32)];
-  const int64_t tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-  int s = 1;
-  while (tiles * s < 256 && 2 * s <= max_splits && 2 * s <= 8 && (K / 64) % (2 * s) == 0) s *= 2;
-  return s;
+  int best = 1;
+  float best_us = kNever;
+  for (int s = 1; s <= std::min(max_splits, 8); s *= 2) {
+    if ((K / 64) % s != 0) break;
+    float us;
+    cheapest_tile(M, N, K, s, OASIS_EPI_PARTIAL_F32, &us);
+    if (s > 1) us += split_cost(M, N, s);
+    if (us < best_us) {
+      best_us = us;
+      best = s;
+    }
+  }
+  return best;
 }
 
 int gemm_launch_cfg(const bf16* A, int64_t lda, const bf16* B, int64_t ldb, int64_t M, int64_t N, int64_t K,
@@ -1410,9 +1477,7 @@ int gemm_launch_cfg(const bf16* A, int64_t lda, const bf16* B, int64_t ldb, int6
   const TileCfg& t = kTiles[tile];
   OASIS_REQUIRE(!(t.no_fp8_epi && e.kind == OASIS_EPI_GELU_TANH_FP8), OASIS_ERR_ARG,
                 "gemm: tile config %d cannot run the GELU_TANH_FP8 epilogue", tile);
-  OASIS_REQUIRE((K / splits) % t.k_gran == 0 && K / splits <= t.k_max &&
-                    (t.k_gran == 64 || ((K / splits / t.k_gran) & (K / splits / t.k_gran - 1)) == 0),
-                OASIS_ERR_SHAPE, "gemm: tile config %d needs K/splits=%lld to be %s of %d up to %d", tile,
+  OASIS_REQUIRE(tile_takes_k(t, K / splits), OASIS_ERR_SHAPE, "gemm: tile config %d needs K/splits=%lld to be %s of %d up to %d", tile,
                 (long long)(K / splits), t.k_gran == 64 ? "a multiple" : "a power-of-two multiple", t.k_gran, t.k_max);
   const hipError_t err = t.fn(A, lda, B, ldb, (int)M, (int)N, (int)K, splits, e, s);
   if (err != hipSuccess) {

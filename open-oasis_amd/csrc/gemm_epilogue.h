@@ -85,27 +85,36 @@ __device__ __forceinline__ void grouped_tile(int pid, int Mt, int Nt, int GN, in
   nt = first + (r - mt * gsz);
 }
 
-// Large-token tile choice among 288 x 256, 288 x 192 (only when allow192) and 288 x 128 (ids
-// t256, t192, t128): among the widths that divide N, the one whose tile count fills its last
-// round of 256 workgroups best (ties: the wider tile); 288 x 128 when none divides N.
-inline int large_token_tile(int64_t M, int64_t N, bool allow192, int t256, int t192, int t128) {
-  const int64_t mt = (M + 287) / 288;
-  const int widths[3] = {256, 192, 128};
-  const int ids[3] = {t256, t192, t128};
-  int best = t128;
-  double best_fill = -1.0;
-  for (int i = 0; i < 3; ++i) {
-    if (N % widths[i] != 0 || (widths[i] == 192 && !allow192)) continue;
-    const int64_t tiles = mt * (N / widths[i]);
-    const int64_t rounds = (tiles + 255) / 256;
-    const double fill = (double)tiles / (double)(rounds * 256);
-    if (fill > best_fill + 1e-9) {
-      best_fill = fill;
-      best = ids[i];
-    }
-  }
-  return best;
+// Tile choice by measured cost. A launch of `tiles` workgroups puts W = ceil(tiles / 256) of them on
+// the busiest CU, one after another or side by side, and takes about
+//     c + W * (a * nk + b)  microseconds,  nk = K tiles of a workgroup's K slice,
+// with c, a and b of a tile and an epilogue class fitted (least squares of the relative error) to
+// hipGraphs of 32 launches over cold weights at 24 row counts from 432 to 9216 (fp8: from 144) and the
+// DiT's four projections. It is what the width alone could not say: 1440 x 4096 in 144 x 64 tiles is
+// 640 workgroups, three rounds of 256 of which the last is half empty (29.8 us), in 192 x 128 tiles
+// 256 workgroups (19.0 us). Over those shapes the tile it picks takes 1.02 times the fastest of all
+// tiles (mean; 1.2 at worst).
+enum { COST_STORE = 0, COST_QKV = 1, COST_RES = 2 };  // plain and GELU stores; QKV + RoPE; fp32 residual / partials
+struct TileCost {
+  int tile;
+  struct {
+    float c, a, b;
+  } k[3];
+};
+constexpr float kNever = 1e9f;  // class not run on this tile
+inline int cost_class(int kind) {
+  if (kind == OASIS_EPI_QKV_ROPE) return COST_QKV;
+  return kind == OASIS_EPI_PARTIAL_F32 || kind == OASIS_EPI_GATED_RES || kind == OASIS_EPI_RESIDUAL ? COST_RES : COST_STORE;
 }
+// microseconds of an M x N product in bm x bn tiles and nk K tiles per workgroup
+inline float tile_cost(const TileCost& t, int bm, int bn, int64_t M, int64_t N, int64_t nk, int splits, int kind) {
+  const auto& k = t.k[cost_class(kind)];
+  const int64_t tiles = (M + bm - 1) / bm * ((N + bn - 1) / bn) * splits;
+  return k.c + (float)((tiles + 255) / 256) * (k.a * (float)nk + k.b);
+}
+// What a split-K product's slices cost the residual_ln that adds them: its reads of M x N fp32
+// slices against a residual added in the GEMM's epilogue (measured at 288 to 4608 rows, N = 1024).
+inline float split_cost(int64_t M, int64_t N, int splits) { return 0.1f + 0.6e-6f * (float)M * (float)N / 1.024f * (float)splits; }
 
 // 16 (or 4) bytes per lane from global memory straight into LDS at lds + 16 * lane (4 * lane);
 // lds is wave-uniform.

@@ -526,18 +526,64 @@ const Tile8 kTiles8[] = {
     OASIS_T8_BIG(288, 64, 2, 4, 1, 2),     // 9
     OASIS_T8_BIG(144, 128, 3, 2, 0, 3),    // 10 (three stages)
     OASIS_T8_BIG(144, 128, 3, 2, 0, 4),    // 11 (four stages)
+    // with 5, 10 and 4 what kCosts8 picks from (fp8 A): 32 x 32 to 96 x 64 wave tiles on 4 to 16 waves
+    OASIS_T8_BIG(64, 64, 2, 2, 0, 4),      // 12
+    OASIS_T8_BIG(96, 64, 2, 2, 0, 3),      // 13
+    OASIS_T8_BIG(96, 128, 2, 4, 0, 3),     // 14
+    OASIS_T8_BIG(144, 128, 3, 4, 0, 3),    // 15
+    OASIS_T8_BIG(144, 64, 3, 2, 0, 3),     // 16
+    OASIS_T8_BIG(192, 128, 4, 2, 0, 3),    // 17
+    OASIS_T8_BIG(192, 192, 4, 3, 0, 2),    // 18
+    OASIS_T8_BIG(64, 128, 2, 4, 0, 3),     // 19
+    OASIS_T8_BIG(144, 256, 3, 4, 0, 3),    // 20
+    OASIS_T8_BIG(192, 256, 4, 4, 0, 2),    // 21
+    OASIS_T8_BIG(288, 192, 3, 4, 1, 2),    // 22
+    OASIS_T8_BIG(256, 128, 4, 2, 0, 3),    // 23
 };
 #undef OASIS_T8
 #undef OASIS_T8_BIG
 constexpr int kNumTiles8 = sizeof(kTiles8) / sizeof(kTiles8[0]);
 
-// Default tile per shape, from sweeps of the DiT projections at M = 4608 on MI355X: with fp8 A
-// from 2048 tokens up the 8-wave 288-row tiles (as the bf16 GEMM picks them).
-int auto_tile8(int64_t M, int64_t N, bool aq, int kind) {
-  if (M >= 2048 && aq) return large_token_tile(M, N, kind != OASIS_EPI_GELU_TANH_FP8, 5, 6, 7);
-  if (M >= 2048) return 2;
-  if (M >= 256) return 3;
-  return 4;
+// Fitted costs (tile_cost, 128-wide K tiles) of the tiles for fp8 A: c, a and b for the plain and
+// GELU stores, QKV + RoPE, and the fp32 residual and partial-sum epilogues.
+const TileCost kCosts8[] = {
+    {4, {{2.96f, 0.254f, 0.00f}, {4.03f, 0.224f, 0.00f}, {3.33f, 0.212f, 0.36f}}},  // 32 x 64
+    {5, {{0.04f, 3.364f, 0.00f}, {0.22f, 3.304f, 0.00f}, {-5.24f, 1.520f, 15.95f}}},  // 288 x 256
+    {10, {{1.81f, 1.299f, 0.00f}, {2.19f, 1.551f, 0.00f}, {0.33f, 0.719f, 5.47f}}},  // 144 x 128
+    {12, {{3.15f, 0.405f, 0.00f}, {3.61f, 0.419f, 0.00f}, {2.63f, 0.365f, 1.09f}}},  // 64 x 64
+    {13, {{4.28f, 0.414f, 0.00f}, {4.56f, 0.437f, 0.00f}, {3.44f, 0.409f, 1.09f}}},  // 96 x 64
+    {14, {{1.50f, 0.960f, 0.00f}, {1.70f, 0.971f, 0.00f}, {0.37f, 0.698f, 3.96f}}},  // 96 x 128
+    {15, {{0.82f, 1.270f, 0.00f}, {1.05f, 1.412f, 0.00f}, {-0.94f, 0.821f, 6.04f}}},  // 144 x 128
+    {16, {{1.87f, 0.881f, 0.00f}, {1.92f, 0.886f, 0.00f}, {0.78f, 0.578f, 3.62f}}},  // 144 x 64
+    {17, {{1.21f, 1.412f, 0.00f}, {1.13f, 1.630f, 0.00f}, {-0.86f, 0.786f, 6.93f}}},  // 192 x 128
+    {18, {{0.61f, 1.918f, 0.00f}, {-0.26f, 1.928f, 0.00f}, {-1.76f, 1.109f, 8.54f}}},  // 192 x 192
+    {19, {{3.06f, 0.598f, 0.00f}, {3.08f, 0.622f, 0.00f}, {kNever, 0.0f, 0.0f}}},  // 64 x 128
+    {20, {{0.63f, 1.949f, 0.00f}, {-0.03f, 2.121f, 0.00f}, {-2.70f, 1.183f, 9.80f}}},  // 144 x 256
+    {21, {{-1.13f, 2.549f, 0.00f}, {-0.65f, 2.346f, 0.00f}, {-3.86f, 1.419f, 11.80f}}},  // 192 x 256
+    {22, {{kNever, 0.0f, 0.0f}, {-0.31f, 3.001f, 0.00f}, {-2.06f, 1.362f, 11.77f}}},  // 288 x 192
+    {23, {{1.01f, 1.758f, 0.00f}, {0.44f, 1.971f, 0.00f}, {-1.64f, 0.870f, 8.72f}}},  // 256 x 128
+};
+
+int cheapest_tile8(int64_t M, int64_t N, int64_t K, int splits, int kind, float* us) {
+  int best = 4;
+  float best_us = kNever;
+  for (const TileCost& c : kCosts8) {
+    const Tile8& t = kTiles8[c.tile];
+    if (t.no_fp8_epi && kind == OASIS_EPI_GELU_TANH_FP8) continue;
+    const float cost = tile_cost(c, t.bm, t.bn, M, N, K / splits / BK8, splits, kind);
+    if (cost < best_us) {
+      best_us = cost;
+      best = c.tile;
+    }
+  }
+  if (us) *us = best_us;
+  return best;
+}
+
+// Default tile: with fp8 A the cheapest by kCosts8, with bf16 A the 4-wave tiles.
+int auto_tile8(int64_t M, int64_t N, int64_t K, int splits, bool aq, int kind) {
+  if (aq) return cheapest_tile8(M, N, K, splits, kind, nullptr);
+  return M >= 2048 ? 2 : (M >= 256 ? 3 : 4);
 }
 
 // Per-row quantization of a bf16 [N, K] weight: scale[n] = max|W[n, :]| / 448,
@@ -592,6 +638,22 @@ __global__ __launch_bounds__(256) void quant_act_kernel(const bf16* __restrict__
 
 namespace oasis {
 
+int gemm_fp8_auto_splits(int64_t M, int64_t N, int64_t K, int max_splits) {
+  int best = 1;
+  float best_us = kNever;
+  for (int s = 1; s <= (max_splits < 8 ? max_splits : 8); s *= 2) {
+    if ((K / BK8) % s != 0) break;
+    float us;
+    cheapest_tile8(M, N, K, s, OASIS_EPI_PARTIAL_F32, &us);
+    if (s > 1) us += split_cost(M, N, s);
+    if (us < best_us) {
+      best_us = us;
+      best = s;
+    }
+  }
+  return best;
+}
+
 int gemm_fp8_launch(const void* A, int64_t lda, const uint8_t* A_scale, int64_t lds, const uint8_t* B, int64_t ldb,
                     const float* w_scale, int64_t M, int64_t N, int64_t K, const oasis_epilogue_t& ex, int tile,
                     int splits, hipStream_t s) {
@@ -615,7 +677,7 @@ int gemm_fp8_launch(const void* A, int64_t lda, const uint8_t* A_scale, int64_t 
                 splits);
   const Epi e = to_epi(ex);
   if (const int rc = check_epilogue(e, M, N, splits)) return rc;
-  if (tile < 0) tile = auto_tile8(M, N, aq, e.kind);
+  if (tile < 0) tile = auto_tile8(M, N, K, splits, aq, e.kind);
   OASIS_REQUIRE(tile < kNumTiles8, OASIS_ERR_ARG, "gemm_fp8: tile config %d out of range", tile);
   const Tile8& t = kTiles8[tile];
   OASIS_REQUIRE(!(t.no_fp8_epi && e.kind == OASIS_EPI_GELU_TANH_FP8), OASIS_ERR_ARG,

@@ -84,20 +84,16 @@ struct Plan {
   // a word every 256 bytes is slower than none (step 1.4876, frame 5.952 ms), and every 32 or 16
   // bytes slower again (frame 5.68 and 6.02 ms).
   int pf_line[3];
-  // Large-token passes whose unsplit 144 x 128 tiles fill the 256 CUs (4465+ tokens at D = 1024):
-  // the O and FC2 projections (N = D) unsplit on these tiles (bf16 kTiles id, fp8 kTiles8 id) with
+  // Passes of 1024 tokens up: the O and FC2 projections (N = D) run unsplit with
   // the bias + gated residual into x in their epilogue, so that no split-K partials are written and
-  // read back and the LayerNorm + modulate after them runs alone. OASIS_O_UNSPLIT and
-  // OASIS_FC2_UNSPLIT = "bf16_tile,fp8_tile" (-1: split-K partials + residual_ln). The defaults
-  // are the fastest measured on MI355X (one box, two reps each), against split-K on 288 x 128:
-  //  - bf16 tile 16 (144 x 128, 6 waves, 4 stages), fp8 tile 10 (the same, 3 stages): the config-2
-  //    sub-block 0.204 -> 0.188 ms, the config-4 step 6.31 -> 5.91 ms (bf16) and 5.61 -> 5.22 ms (fp8);
-  //  - two stages (bf16 tile 13, fp8 8): 6.59 / 5.65 ms with FC2 unsplit; O alone 6.22 / 5.44 ms;
-  //  - 8 waves of 144 x 16 on 288 x 64 (bf16 14, fp8 9): O alone 6.53 / 5.65 ms;
-  //  - FC1 or QKV on the 144 x 128 tiles too (four rounds of 256 tiles): 6.52-7.04 / 5.52-5.99 ms.
+  // read back and the LayerNorm + modulate after them runs alone, wherever the measured tile costs make
+  // one K slice cheapest (gemm_auto_splits; kAutoUnsplit, the default). OASIS_O_UNSPLIT and OASIS_FC2_UNSPLIT =
+  // "bf16_tile,fp8_tile" force a tile (kTiles / kTiles8 id) from 256 tiles of 144 x 128 up (4465+
+  // tokens at D = 1024) and split-K partials + residual_ln below; -1: partials + residual_ln always.
   int o_unsplit[2];
   int fc2_unsplit[2];
 };
+constexpr int kAutoUnsplit = -2;
 
 enum { PF_NONE = 0, PF_LN = 1, PF_ATTN = 2, PF_QKVG = 3, PF_OG = 4, PF_FC1G = 5, PF_FC2G = 6 };
 // where each host runs in a sub-block, and where each of the four weights is read: a host that runs
@@ -184,8 +180,7 @@ const Plan& plan() {
         q.pf_host[i / 4][i % 4] = (v >= PF_LN && v <= PF_FC2G) ? v : PF_NONE;
       }
     }
-    q.o_unsplit[0] = q.fc2_unsplit[0] = 16;
-    q.o_unsplit[1] = q.fc2_unsplit[1] = 10;
+    q.o_unsplit[0] = q.o_unsplit[1] = q.fc2_unsplit[0] = q.fc2_unsplit[1] = kAutoUnsplit;
     if (const char* env = getenv("OASIS_O_UNSPLIT")) sscanf(env, "%d,%d", &q.o_unsplit[0], &q.o_unsplit[1]);
     if (const char* env = getenv("OASIS_FC2_UNSPLIT")) sscanf(env, "%d,%d", &q.fc2_unsplit[0], &q.fc2_unsplit[1]);
     q.frag1 = FRAG_O | FRAG_FC2 | FRAG_LN;
@@ -395,16 +390,31 @@ extern "C" int oasis_dit_conditioning_noalloc(const oasis_dit_weights_t* w, cons
 
 namespace {
 
-// Split-K count of a partial-sum projection (O: K = D, FC2: K = 4D) below 2048 tokens, from timings
-// on MI355X of gemm.hip's default tiles: O in 2 slices at one 144-token frame and whole above (the
-// wave-split tiles fill the CUs without slicing), FC2 in 4; fewer when max_splits or whole 64-wide K
-// tiles per slice require it. From 2048 tokens up the GEMM's own large-token tiles decide.
-int choose_splits(int64_t M, int64_t N, int64_t K, int64_t max_splits) {
-  (void)N;
-  if (M >= 2048) return oasis::gemm_auto_splits(M, N, K, (int)std::min<int64_t>(max_splits, 8));
+// Split-K count of a residual projection (O: K = D, FC2: K = 4D): above 320 tokens and with fp8 weights
+// the measured tile costs decide; else, from timings on MI355X of gemm.hip's default tiles, O in 2
+// slices at one 144-token frame and whole above (the wave-split tiles fill the CUs without slicing),
+// FC2 in 4, fewer when max_splits or whole 64-wide K tiles per slice require it.
+int choose_splits(bool fp8, int64_t M, int64_t N, int64_t K, int64_t max_splits) {
+  const int cap = (int)std::min<int64_t>(max_splits, 8);
+  if (fp8) return oasis::gemm_fp8_auto_splits(M, N, K, cap);
+  if (M > 320) return oasis::gemm_auto_splits(M, N, K, cap);
   int s = K > 1024 ? 4 : (M <= 160 ? 2 : 1);
   while (s > 1 && (s > max_splits || (K / 64) % s != 0)) s /= 2;
   return s;
+}
+
+// Whether a residual projection of `splits` K slices runs unsplit with its residual in the epilogue,
+// by the plan's tiles (o_unsplit / fc2_unsplit) for bf16 or fp8 weights; *tile: the tile (-1: default).
+// A role placed by OASIS_GEMM_PLAN / OASIS_GEMM_PLAN8 (planned) keeps split-K partials.
+bool unsplit_residual(const int (&tiles)[2], bool fp8, bool planned, int64_t M, int64_t N, int splits, int* tile) {
+  const int t = tiles[fp8 ? 1 : 0];
+  *tile = t >= 0 ? t : -1;
+  if (planned) return false;
+  // below ~1000 rows the residual's loads in the epilogue cost more than the partial that residual_ln
+  // then reads (O at 576 rows: GEMM 6.9 against 6.0 us, residual_ln 4.9 against 5.0; at 1440 rows 9.5
+  // against 9.0 and 5.2 against 5.9)
+  if (t == kAutoUnsplit) return splits == 1 && M >= 1024;
+  return t >= 0 && (M + 143) / 144 * ((N + 127) / 128) >= 256;
 }
 
 // A residual that has been computed as split-K partials but not yet added to x.
@@ -519,10 +529,11 @@ int dit_blocks(const oasis_dit_weights_t* w, const oasis_dit_buffers_t* buf, int
   const int64_t M = B * T * P;
   hipStream_t s = (hipStream_t)stream;
   const Plan& pl = plan();
+  const bool fp8 = w->weight_format == OASIS_WEIGHTS_FP8;
   const int so = pl.splits[ROLE_O] > 0 ? std::min<int>(pl.splits[ROLE_O], buf->max_splits)
-                                       : choose_splits(M, D, D, buf->max_splits);
+                                       : choose_splits(fp8, M, D, D, buf->max_splits);
   int sf = pl.splits[ROLE_FC2] > 0 ? std::min<int>(pl.splits[ROLE_FC2], buf->max_splits)
-                                   : choose_splits(M, D, Dm, buf->max_splits);
+                                   : choose_splits(fp8, M, D, Dm, buf->max_splits);
   // fragment order (the FRAG_* bits of the plan): the producer of each chosen operand (residual_ln,
   // the attention kernels, FC1's GELU epilogue) writes it in MFMA fragment order and its projection
   // runs on gemm_frag (O unsplit, FC2 in slices of 1024)
@@ -539,16 +550,12 @@ int dit_blocks(const oasis_dit_weights_t* w, const oasis_dit_buffers_t* buf, int
   qkv.n_heads = (int)H;
   qkv.rows_per_frame = P;
   qkv.frames_per_stream = T;
-  const bool fp8 = w->weight_format == OASIS_WEIGHTS_FP8;
-  // O and FC2 unsplit with their gated residual in the epilogue where 144 x 128 tiles fill the CUs
-  // (unless OASIS_GEMM_PLAN / OASIS_GEMM_PLAN8 place that role themselves)
-  const bool unsplit_fill = (M + 143) / 144 * ((D + 127) / 128) >= 256;
-  auto unsplit = [&](int role, const int (&tiles)[2]) {
-    return unsplit_fill && pl.splits[role] <= 0 && (fp8 ? tiles[1] >= 0 && pl.tile8[role] < 0
-                                                           : tiles[0] >= 0 && pl.tile[role] < 0);
-  };
-  const bool o_res = !f_o && !f_ln && !f_fc1 && unsplit(ROLE_O, pl.o_unsplit);
-  const bool fc2_res = !f_fc2 && unsplit(ROLE_FC2, pl.fc2_unsplit);
+  // O and FC2 unsplit with their gated residual in the epilogue
+  auto planned = [&](int role) { return pl.splits[role] > 0 || (fp8 ? pl.tile8[role] : pl.tile[role]) >= 0; };
+  int o_tile, fc2_tile;
+  const bool o_res =
+      unsplit_residual(pl.o_unsplit, fp8, planned(ROLE_O), M, D, so, &o_tile) && !f_o && !f_ln && !f_fc1;
+  const bool fc2_res = unsplit_residual(pl.fc2_unsplit, fp8, planned(ROLE_FC2), M, D, sf, &fc2_tile) && !f_fc2;
   oasis_epilogue_t gelu = epi_zero();
   gelu.kind = fp8 ? OASIS_EPI_GELU_TANH_FP8 : (f_fc2 ? OASIS_EPI_GELU_TANH_FRAG : OASIS_EPI_GELU_TANH);
   gelu.out_bf16 = buf->mlp;
@@ -694,8 +701,7 @@ int dit_blocks(const oasis_dit_weights_t* w, const oasis_dit_buffers_t* buf, int
     } else if (o_res) {
       // O unsplit with bias + gated residual into x in its epilogue, then LN + modulate alone
       OASIS_TRY(proj(w, ROLE_O, j, fp8 ? (const void*)a8 : buf->attn, D, a8s, M, D, D,
-                     gated_res_epi(buf->x, D, w->out_b[j], a + 2 * D, fs, P), pl.o_unsplit[0], 1, s, nullptr,
-                     pl.o_unsplit[1]));
+                     gated_res_epi(buf->x, D, w->out_b[j], a + 2 * D, fs, P), o_tile, 1, s, nullptr, o_tile));
       OASIS_TRY(oasis::residual_ln(buf->x, M, D, buf->partial, 0, M * D, nullptr, nullptr, fs, P, a + 4 * D, a + 3 * D,
                                    fs, (void*)ln_out, fp8 ? a8 : nullptr, a8s, kLnEps, s, f_fc1));
       OASIS_TRY(proj(w, ROLE_FC1, j, fp8 ? (const void*)a8 : buf->h, D, a8s, M, Dm, D, gelu, pl.tile[ROLE_FC1], 1, s,
@@ -718,8 +724,7 @@ int dit_blocks(const oasis_dit_weights_t* w, const oasis_dit_buffers_t* buf, int
     }
     if (fc2_res) {  // FC2 unsplit: its gated residual lands in x, nothing stays pending
       OASIS_TRY(proj(w, ROLE_FC2, j, mlp_in, Dm, mlp_sc, M, D, Dm,
-                     gated_res_epi(buf->x, D, w->fc2_b[j], a + 5 * D, fs, P), pl.fc2_unsplit[0], 1, s, nullptr,
-                     pl.fc2_unsplit[1]));
+                     gated_res_epi(buf->x, D, w->fc2_b[j], a + 5 * D, fs, P), fc2_tile, 1, s, nullptr, fc2_tile));
       *pend = Pending();
       continue;
     }
@@ -883,9 +888,9 @@ int vae_decode(const oasis_vae_weights_t* w, const oasis_vae_buffers_t* buf, int
   hipStream_t s = (hipStream_t)stream;
   const Plan& pl = plan();
   const int sp = pl.splits[ROLE_VO] > 0 ? std::min<int>(pl.splits[ROLE_VO], buf->max_splits)
-                                        : choose_splits(L, D, D, buf->max_splits);
+                                        : choose_splits(false, L, D, D, buf->max_splits);
   const int sf = pl.splits[ROLE_VFC2] > 0 ? std::min<int>(pl.splits[ROLE_VFC2], buf->max_splits)
-                                          : choose_splits(L, D, Dm, buf->max_splits);
+                                          : choose_splits(false, L, D, Dm, buf->max_splits);
   OASIS_TRY(oasis_small_linear(latent, w->latent_dim, L, w->latent_dim, w->pq_w, OASIS_BF16, 0, D, w->pq_b, buf->x, D,
                                stream));
 
@@ -908,10 +913,12 @@ int vae_decode(const oasis_vae_weights_t* w, const oasis_vae_buffers_t* buf, int
   gelu.out_bf16 = buf->mlp;
   gelu.ld_out = Dm;
   const oasis_epilogue_t part = partial_epi(buf->partial, L, D);
-  // batched decodes whose unsplit 144 x 128 tiles fill the CUs: O and FC2 unsplit (as dit_blocks)
-  const bool unsplit_fill = (L + 143) / 144 * ((D + 127) / 128) >= 256;
-  const bool o_res = unsplit_fill && pl.tile[ROLE_VO] < 0 && pl.splits[ROLE_VO] <= 0 && pl.o_unsplit[0] >= 0;
-  const bool fc2_res = unsplit_fill && pl.tile[ROLE_VFC2] < 0 && pl.splits[ROLE_VFC2] <= 0 && pl.fc2_unsplit[0] >= 0;
+  // O and FC2 unsplit with the residual in the epilogue (as dit_blocks)
+  int o_tile, fc2_tile;
+  const bool o_res = unsplit_residual(pl.o_unsplit, false, pl.tile[ROLE_VO] >= 0 || pl.splits[ROLE_VO] > 0, L, D, sp,
+                                      &o_tile);
+  const bool fc2_res = unsplit_residual(pl.fc2_unsplit, false, pl.tile[ROLE_VFC2] >= 0 || pl.splits[ROLE_VFC2] > 0, L, D,
+                                        sf, &fc2_tile);
 
   Pending pend;
   const int64_t wbytes[4] = {3 * D * D * 2, D * D * 2, Dm * D * 2, D * Dm * 2};
@@ -932,7 +939,7 @@ int vae_decode(const oasis_vae_weights_t* w, const oasis_vae_buffers_t* buf, int
     OASIS_TRY(oasis::attention(buf->q, buf->k, buf->v, buf->attn, B, Lf, H, kAttnScale, s, false, &pf_attn));
     if (o_res) {  // unsplit, the residual added in the epilogue (as the DiT's large-token passes)
       OASIS_TRY(oasis::gemm_launch_cfg((const bf16*)buf->attn, D, (const bf16*)w->proj_w[i], D, L, D, D,
-                                       residual_epi(buf->x, D, w->proj_b[i]), pl.o_unsplit[0], 1, s));
+                                       residual_epi(buf->x, D, w->proj_b[i]), o_tile, 1, s));
       OASIS_TRY(oasis_residual_ln(buf->x, L, D, nullptr, 0, L * D, nullptr, nullptr, 0, L, w->n2_w[i], w->n2_b[i], 0,
                                   buf->h, kLnEps, stream));
     } else {
@@ -946,7 +953,7 @@ int vae_decode(const oasis_vae_weights_t* w, const oasis_vae_buffers_t* buf, int
                                      pl.tile[ROLE_VFC1], 1, s));
     if (fc2_res) {
       OASIS_TRY(oasis::gemm_launch_cfg((const bf16*)buf->mlp, Dm, (const bf16*)w->fc2_w[i], Dm, L, D, Dm,
-                                       residual_epi(buf->x, D, w->fc2_b[i]), pl.fc2_unsplit[0], 1, s));
+                                       residual_epi(buf->x, D, w->fc2_b[i]), fc2_tile, 1, s));
       pend = Pending();
     } else {
       OASIS_TRY(oasis::gemm_launch_cfg((const bf16*)buf->mlp, Dm, (const bf16*)w->fc2_w[i], Dm, L, D, Dm, part,
