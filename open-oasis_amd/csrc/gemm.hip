@@ -15,8 +15,6 @@
 //   - gemm_wave_kernel: 4 waves split each workgroup's K slice four ways, each over its own LDS
 //     ring with no workgroup barrier in the K loop; the default below 320 tokens (QKV + RoPE, O,
 //     FC1, FC2) and for the VAE's O projection.
-//   - gemm_bf16_kernel: global -> registers -> LDS, for the reference-surface oasis_linear with
-//     its [K, N] weight layout (the weights transposed into LDS).
 // After the K loop the fp32 tile is staged through LDS so each thread handles 8 consecutive
 // columns of one row: coalesced 16/32-byte stores and in-register RoPE pair swaps.
 //
@@ -33,183 +31,7 @@ namespace {
 
 constexpr int BK = 64;            // K granularity every configuration supports
 
-// BKN = false: B is [N, K] (weights as stored by this library); true: B is [K, N]
-// (the reference's transposed weight layout, used by the linear_k32 surface only).
-// STAGES K-tiles are in flight per workgroup: a register ring of STAGES global-load
-// slots feeds a double-buffered LDS tile pair. With `splits` > 1 the K range is cut
-// into equal slices, one per workgroup, and the epilogue must be PARTIAL_F32.
-template <int BM, int BN, int WM, int WN, int STAGES, bool BKN, int BKT>
-__global__ __launch_bounds__(256) void gemm_bf16_kernel(const bf16* __restrict__ A, int64_t lda,
-                                                        const bf16* __restrict__ B, int64_t ldb,
-                                                        int M, int N, int K, int splits, Epi e) {
-  static_assert(WM * WN == 4, "4 waves");
-  constexpr int TM = BM / WM, TN = BN / WN;
-  constexpr int FM = TM / 16, FN = TN / 16;
-  static_assert(FM * 16 == TM && FN * 16 == TN, "wave tile must be a multiple of 16");
-  constexpr int BK = BKT;                  // K per pipeline step
-  constexpr int LDS_PITCH = BK + 8;        // bf16 per LDS row (16 B pad: conflict-free b128 reads)
-  constexpr int CPR = BK / 8;              // 16-byte chunks per tile row
-  constexpr int A_CHUNKS = BM * CPR;       // 16-byte chunks per A tile
-  constexpr int B_CHUNKS = BN * CPR;
-  // every thread loads whole chunks: no per-thread guards, so the compiler can keep
-  // STAGES tiles of loads in flight (a divergent guard forces a full vmcnt(0) wait)
-  static_assert(A_CHUNKS % 256 == 0 && B_CHUNKS % 256 == 0, "BM and BN must be multiples of 32");
-  constexpr int A_PER = A_CHUNKS / 256;
-  constexpr int B_PER = B_CHUNKS / 256;
-  constexpr int AB_BYTES = 2 * (BM + BN) * LDS_PITCH * 2;
-  constexpr int C_PITCH = BN + 4;
-  constexpr int C_BYTES = BM * C_PITCH * 4;
-  constexpr int SMEM = AB_BYTES > C_BYTES ? AB_BYTES : C_BYTES;
-  __shared__ __attribute__((aligned(16))) char smem[SMEM];
-  bf16* As = reinterpret_cast<bf16*>(smem);                    // [2][BM][LDS_PITCH]
-  bf16* Bs = As + 2 * BM * LDS_PITCH;                          // [2][BN][LDS_PITCH]
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave % WM, wn = wave / WM;
-  const int Mt = (M + BM - 1) / BM, Nt = (N + BN - 1) / BN;
-  // (n tile, split, m tile) with m fastest: consecutive ids share one weight slice
-  const int pid = xcd_remap(blockIdx.x, Mt * Nt * splits);
-  const int mt = pid % Mt;
-  const int rest = pid / Mt;
-  const int split = rest % splits, nt = rest / splits;
-  const int m0 = mt * BM, n0 = nt * BN;
-  const int nk = K / BK / splits;  // the host guarantees nk % STAGES == 0
-  const int kb = split * nk * BK;
-
-  const bf16* a_src[A_PER];
-  int a_dst[A_PER];
-#pragma unroll
-  for (int i = 0; i < A_PER; ++i) {
-    const int c = tid + i * 256;
-    const int row = c / CPR, col = (c % CPR) * 8;
-    const int gr = min(m0 + row, M - 1);
-    a_src[i] = A + (int64_t)gr * lda + kb + col;
-    a_dst[i] = row * LDS_PITCH + col;
-  }
-  const bf16* b_src[B_PER];
-  int b_dst[B_PER];
-#pragma unroll
-  for (int i = 0; i < B_PER; ++i) {
-    const int c = tid + i * 256;
-    if (!BKN) {
-      const int row = c / CPR, col = (c % CPR) * 8;
-      const int gr = min(n0 + row, N - 1);
-      b_src[i] = B + (int64_t)gr * ldb + kb + col;
-      b_dst[i] = row * LDS_PITCH + col;
-    } else {  // chunk = 8 consecutive n of one k row; stored transposed into [n][k]
-      const int krow = c / (BN / 8), nc = (c % (BN / 8)) * 8;
-      const int gn = min(n0 + nc, N - 8);
-      b_src[i] = B + (int64_t)(kb + krow) * ldb + gn;
-      b_dst[i] = nc * LDS_PITCH + krow;
-    }
-  }
-
-  i32x4 ra[STAGES][A_PER], rb[STAGES][B_PER];
-  auto gload = [&](int slot, int kt) {
-    const int64_t ka = (int64_t)kt * BK;
-#pragma unroll
-    for (int i = 0; i < A_PER; ++i) ra[slot][i] = *reinterpret_cast<const i32x4*>(a_src[i] + ka);
-#pragma unroll
-    for (int i = 0; i < B_PER; ++i)
-      rb[slot][i] = *reinterpret_cast<const i32x4*>(b_src[i] + (BKN ? ka * ldb : ka));
-  };
-  auto lstore = [&](int slot, int buf) {
-    bf16* as = As + buf * BM * LDS_PITCH;
-    bf16* bs = Bs + buf * BN * LDS_PITCH;
-#pragma unroll
-    for (int i = 0; i < A_PER; ++i) *reinterpret_cast<i32x4*>(as + a_dst[i]) = ra[slot][i];
-#pragma unroll
-    for (int i = 0; i < B_PER; ++i) {
-      if (!BKN) {
-        *reinterpret_cast<i32x4*>(bs + b_dst[i]) = rb[slot][i];
-      } else {
-        const bf16x8 t = __builtin_bit_cast(bf16x8, rb[slot][i]);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) bs[b_dst[i] + j * LDS_PITCH] = t[j];
-      }
-    }
-  };
-
-  f32x4 acc[FM][FN];
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int lr = lane & 15, lk = (lane >> 4) * 8;
-  auto compute = [&](int buf) {
-    const bf16* as = As + buf * BM * LDS_PITCH + (wm * TM + lr) * LDS_PITCH + lk;
-    const bf16* bs = Bs + buf * BN * LDS_PITCH + (wn * TN + lr) * LDS_PITCH + lk;
-#pragma unroll
-    for (int ks = 0; ks < BK / 32; ++ks) {
-      bf16x8 af[FM], bfr[FN];
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-        af[i] = *reinterpret_cast<const bf16x8*>(as + i * 16 * LDS_PITCH + ks * 32);
-#pragma unroll
-      for (int j = 0; j < FN; ++j)
-        bfr[j] = *reinterpret_cast<const bf16x8*>(bs + j * 16 * LDS_PITCH + ks * 32);
-#pragma unroll
-      for (int i = 0; i < FM; ++i)
-#pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = mfma16(af[i], bfr[j], acc[i][j]);
-    }
-  };
-
-  // Prologue: tiles 0..STAGES-1 in flight, tile 0 in LDS. Tile indices past the end are
-  // clamped to the last tile (a redundant L2 hit) instead of branched around, so the
-  // loop body is straight-line and the waits before each LDS store count only the
-  // STAGES-1 younger tiles.
-#pragma unroll
-  for (int s = 0; s < STAGES; ++s) gload(s, min(s, nk - 1));
-  lstore(0, 0);
-  __syncthreads();
-  for (int k0 = 0; k0 < nk; k0 += STAGES) {
-#pragma unroll
-    for (int s = 0; s < STAGES; ++s) {
-      const int k = k0 + s;
-      gload(s, min(k + STAGES, nk - 1));     // slot s held tile k, already in LDS
-      compute(k & 1);
-      lstore((s + 1) % STAGES, (k + 1) & 1);  // tile k+1 (a copy of the last tile at the end)
-      __syncthreads();
-    }
-  }
-
-  // stage the fp32 tile through LDS (the A/B ring is free after the last barrier)
-  float* Cs = reinterpret_cast<float*>(smem);
-#pragma unroll
-  for (int i = 0; i < FM; ++i)
-#pragma unroll
-    for (int j = 0; j < FN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        Cs[(wm * TM + i * 16 + (lane >> 4) * 4 + r) * C_PITCH + wn * TN + j * 16 + lr] = acc[i][j][r];
-  __syncthreads();
-
-  constexpr int UNITS = BM * (BN / 8);
-  for (int u = tid; u < UNITS; u += 256) {
-    const int r = u / (BN / 8), c8 = (u % (BN / 8)) * 8;
-    const int gm = m0 + r, gn = n0 + c8;
-    if (gm >= M || gn >= N) continue;
-    float v[8];
-    const f32x4 c0 = *reinterpret_cast<const f32x4*>(Cs + r * C_PITCH + c8);
-    const f32x4 c1 = *reinterpret_cast<const f32x4*>(Cs + r * C_PITCH + c8 + 4);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      v[j] = c0[j];
-      v[j + 4] = c1[j];
-    }
-    if (e.kind == OASIS_EPI_PARTIAL_F32) {
-      float* d = e.out_f32 + (int64_t)split * e.split_stride + (int64_t)gm * e.ld_out + gn;
-      *reinterpret_cast<f32x4*>(d) = c0;
-      *reinterpret_cast<f32x4*>(d + 4) = c1;
-    } else {
-      epilogue8(e, gm, gn, v);
-    }
-  }
-}
-
-// Same product with the global -> LDS copies done by the memory pipeline itself
+// The global -> LDS copies are done by the memory pipeline itself
 // (global_load_lds_dwordx4: each lane's 16 bytes land at LDS base + 16 * lane), so tiles
 // take no VGPRs or LDS-store instructions in flight and STAGES K tiles can be queued per
 // workgroup. LDS rows are unpadded 128-byte rows of 16-byte chunks stored XOR-swizzled
@@ -1286,16 +1108,6 @@ hipError_t launch_lds(const bf16* A, int64_t lda, const bf16* B, int64_t ldb, in
   return hipGetLastError();
 }
 
-template <int BM, int BN, int WM, int WN, int STAGES, bool BKN = false, int BKT = 64>
-hipError_t launch_cfg(const bf16* A, int64_t lda, const bf16* B, int64_t ldb, int M, int N, int K,
-                      int splits, const Epi& e, hipStream_t s) {
-  if ((K / splits) % BKT != 0) return hipErrorInvalidConfiguration;
-  const int Mt = (M + BM - 1) / BM, Nt = (N + BN - 1) / BN;
-  hipLaunchKernelGGL((gemm_bf16_kernel<BM, BN, WM, WN, STAGES, BKN, BKT>), dim3(Mt * Nt * splits), dim3(256), 0, s,
-                     A, lda, B, ldb, M, N, K, splits, e);
-  return hipGetLastError();
-}
-
 // Tile configurations (id -> BM x BN, wave grid, prefetch depth): the ones the default choice
 // below uses, for the shapes of the DiT step, the frame, the VAE and the large-token batches.
 typedef hipError_t (*launch_fn)(const bf16*, int64_t, const bf16*, int64_t, int, int, int, int, const Epi&,
@@ -1555,35 +1367,6 @@ int gemm_launch(const bf16* A, int64_t lda, const bf16* B, int64_t ldb, int64_t 
 }
 
 }  // namespace oasis
-
-extern "C" int oasis_linear(const void* x, const void* w, void* out, int64_t M, int64_t K, int64_t N,
-                            int w_layout, int out_dtype, oasis_stream_t stream) {
-  OASIS_REQUIRE(x && w && out, OASIS_ERR_NULL, "linear: null pointer");
-  OASIS_REQUIRE(oasis_aligned(16, x, w, out), OASIS_ERR_ARG, "linear: pointers must be 16-byte aligned");
-  OASIS_REQUIRE(M > 0 && N > 0 && K > 0 && K % BK == 0 && N % 8 == 0 && M < (1ll << 31) && N < (1ll << 31),
-                OASIS_ERR_SHAPE, "linear: need K %% 64 == 0 and N %% 8 == 0");
-  OASIS_REQUIRE(w_layout == 0 || w_layout == 1, OASIS_ERR_ARG, "linear: w_layout must be 0 ([K,N]) or 1 ([N,K])");
-  OASIS_REQUIRE(out_dtype == OASIS_F32 || out_dtype == OASIS_BF16, OASIS_ERR_DTYPE, "linear: bad out dtype %d",
-                out_dtype);
-  oasis_epilogue_t ex;
-  memset(&ex, 0, sizeof(ex));
-  ex.kind = out_dtype == OASIS_F32 ? OASIS_EPI_STORE_F32 : OASIS_EPI_STORE_BF16;
-  ex.out_f32 = static_cast<float*>(out);
-  ex.out_bf16 = out;
-  ex.ld_out = N;
-  if (w_layout == 1)
-    return oasis::gemm_launch(static_cast<const bf16*>(x), K, static_cast<const bf16*>(w), K, M, N, K, ex,
-                              static_cast<hipStream_t>(stream));
-  const Epi e = to_epi(ex);
-  const hipError_t err = launch_cfg<32, 64, 1, 4, 1, true>(static_cast<const bf16*>(x), K, static_cast<const bf16*>(w),
-                                                           N, (int)M, (int)N, (int)K, 1, e,
-                                                           static_cast<hipStream_t>(stream));
-  if (err != hipSuccess) {
-    oasis::set_error("linear launch failed: %s", hipGetErrorString(err));
-    return OASIS_ERR_LAUNCH;
-  }
-  return OASIS_OK;
-}
 
 extern "C" int oasis_gemm_bf16_config(const void* A, int64_t lda, const void* B, int64_t ldb, int64_t M,
                                       int64_t N, int64_t K, const oasis_epilogue_t* epi, int tile, int splits,
