@@ -93,6 +93,40 @@ __device__ __forceinline__ void store_fp8x4(uint8_t* q, uint8_t* sc, const float
   if (sc) *sc = (uint8_t)sb;
 }
 
+// One query's output in the O^T accumulators of its 4 lanes (o[dt][i]: dim 16 dt + 4 g + i of the head, times
+// inv), at row-major element offset off: as T, in fragment order, or as fp8 activation blocks. Called by all 4
+// lanes (the ones that share lane % 16) of a query together.
+template <typename T>
+__device__ __forceinline__ void store_head(T* O, int64_t off, const f32x4 (&o)[4], float inv, int g, int frag_ks,
+                                           uint8_t* o8, uint8_t* o8s) {
+  if (o8) {
+    // dims 0..31 of the head are o[0..1] of the 4 lanes (lane groups g), 32..63 o[2..3]
+    float r[4][4], m[2] = {0.f, 0.f};
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        r[dt][i] = bf2f(f2bf(o[dt][i] * inv));
+        m[dt >> 1] = fmaxf(m[dt >> 1], fabsf(r[dt][i]));
+      }
+#pragma unroll
+    for (int h2 = 0; h2 < 2; ++h2) m[h2] = max_xor32(max_xor16(m[h2]));
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) {
+      const int64_t e = off + dt * 16 + 4 * g;
+      store_fp8x4(o8 + e, (g == 0 && (dt & 1) == 0) ? o8s + e / 32 : nullptr, r[dt], m[dt >> 1]);
+    }
+    return;
+  }
+  const int64_t ocols = (int64_t)frag_ks * 32, orow = frag_ks ? off / ocols : 0;
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt) {
+    const int d = dt * 16 + 4 * g;
+    T* dst = frag_ks ? O + frag_index(orow, off - orow * ocols + d, frag_ks) : O + off + d;
+    store4<T>(dst, o[dt][0] * inv, o[dt][1] * inv, o[dt][2] * inv, o[dt][3] * inv);
+  }
+}
+
 // KS keys are staged in LDS at a time (K rows and V^T columns; KS >= Lk stages the whole
 // sequence once, with no barrier in the key loop) and consumed in KC-key chunks.
 // V^T is built from 8x8 blocks: a thread loads 8 key rows x 8 dims and transposes them in
@@ -286,32 +320,7 @@ __global__ __launch_bounds__(NW * KSPLIT * 64) void flash_kernel(const T* __rest
   const int f = bh / a.H, h = bh - f * a.H;
   const int fo = f / a.f_inner, fi = f - fo * a.f_inner;
   const int64_t off = fo * a.o_sfo + fi * a.o_sf + h * a.o_sh + (int64_t)my_q * a.o_si;
-  const int64_t ocols = (int64_t)a.frag_ks * 32, orow = a.frag_ks ? off / ocols : 0;
-  if (a.o8) {
-    // dims 0..31 of the head are o[0..1] of the 4 lanes sharing lr (lane groups g), 32..63 o[2..3]
-    float r[4][4], m[2] = {0.f, 0.f};
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        r[dt][i] = bf2f(f2bf(o[dt][i] * inv));
-        m[dt >> 1] = fmaxf(m[dt >> 1], fabsf(r[dt][i]));
-      }
-#pragma unroll
-    for (int h2 = 0; h2 < 2; ++h2) m[h2] = max_xor32(max_xor16(m[h2]));
-#pragma unroll
-    for (int dt = 0; dt < 4; ++dt) {
-      const int64_t e = off + dt * 16 + 4 * g;
-      store_fp8x4(a.o8 + e, (g == 0 && (dt & 1) == 0) ? a.o8s + e / 32 : nullptr, r[dt], m[dt >> 1]);
-    }
-    return;
-  }
-#pragma unroll
-  for (int dt = 0; dt < 4; ++dt) {
-    const int d = dt * 16 + 4 * g;
-    T* dst = a.frag_ks ? O + frag_index(orow, off - orow * ocols + d, a.frag_ks) : O + off + d;
-    store4<T>(dst, o[dt][0] * inv, o[dt][1] * inv, o[dt][2] * inv, o[dt][3] * inv);
-  }
+  store_head<T>(O, off, o, inv, g, a.frag_ks, a.o8, a.o8s);
 }
 
 // PLAIN variants (no bias, not causal) exist for bf16, the dtype of the DiT and VAE paths
@@ -379,7 +388,10 @@ int flash_launch(const T* q, const T* k, const T* v, T* o, int64_t n_bh, const A
 }
 
 // q,k,v: [B][P][H][T][64] bf16; out: token-major [(b*T + t)*P + p][h*64 + d], row-major or
-// (fks = 2H) in MFMA fragment order
+// (fks = 2H) in MFMA fragment order. TW >= 3: windows of TW frames, every row loaded up front (the general loop
+// loads a key and a value row per (query, key) pair, a dependent chain of round trips: T = 3 at 432 tokens 4.0 us,
+// T = 5 at 1440 10.1, T = 7 at 3024 15.7; with the loads ahead 3.0, 6.2 and 9.1)
+template <int TW>
 __global__ __launch_bounds__(256) void temporal_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k,
                                                        const bf16* __restrict__ v, bf16* __restrict__ out,
                                                        int64_t G, int T, int P, int H, float scale_log2, int qf,
@@ -411,6 +423,36 @@ __global__ __launch_bounds__(256) void temporal_kernel(const bf16* __restrict__ 
     bf16* dst = fks ? out + frag_index(row, col, fks) : out + row * (int64_t)(H * 64) + col;
     *reinterpret_cast<bf16x4*>(dst) = bf16x4{f2bf(a0), f2bf(a1), f2bf(a2), f2bf(a3)};
   };
+  if constexpr (TW >= 3) {
+    bf16x4 qr[TW], kr[TW], vr[TW];
+#pragma unroll
+    for (int t = 0; t < TW; ++t) {
+      qr[t] = *reinterpret_cast<const bf16x4*>(q + base + t * 64);
+      kr[t] = *reinterpret_cast<const bf16x4*>(k + base + t * 64);
+      vr[t] = *reinterpret_cast<const bf16x4*>(v + base + t * 64);
+    }
+#pragma unroll
+    for (int t = 0; t < TW; ++t) {
+      float m = -INFINITY, l = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s <= t; ++s) {
+        float dot = bf2f(qr[t][0]) * bf2f(kr[s][0]) + bf2f(qr[t][1]) * bf2f(kr[s][1]) +
+                    bf2f(qr[t][2]) * bf2f(kr[s][2]) + bf2f(qr[t][3]) * bf2f(kr[s][3]);
+        dot = row16_sum(dot);
+        const float x = dot * scale_log2;
+        const float m_new = fmaxf(m, x);
+        const float alpha = exp2f(m - m_new);
+        const float pexp = exp2f(x - m_new);
+        l = l * alpha + pexp;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[i] = acc[i] * alpha + pexp * bf2f(vr[s][i]);
+        m = m_new;
+      }
+      const float inv = 1.0f / l;
+      put((b * TW + t) * P + p, acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
+    }
+    return;
+  }
   // qf >= 0: only query frame qf is computed, written as the single frame of a T=1 output
   // (out row b*P + p); the K/V cache path runs the current frame against cached context K/V.
   if (T == 2) {  // the DiT's 2-frame window: one round trip for all six rows
@@ -460,6 +502,144 @@ __global__ __launch_bounds__(256) void temporal_kernel(const bf16* __restrict__ 
     const float inv = 1.0f / l;
     const int64_t frame = qf < 0 ? b * T + t : b;
     put(frame * P + p, acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
+  }
+}
+
+// Causal windows of 8 to 32 frames: one wave per tile of NT x 16 consecutive rows of the [group][T][64] layout
+// (NT = 1: floor(16 / T) whole groups; NT = 2: one group of up to 32 frames), no barrier and no shared staging.
+// Q and K rows go straight into the MFMA operands of S^T = K Q^T; V rows go to the wave's own LDS as they lie
+// (32-byte groups XOR-swizzled by (row / 2) % 4, so that half a wave's 8 rows fall in distinct banks) and
+// ds_read_b64_tr_b16 transposes them into the operand of O^T = V^T P^T: k-slot j of lane group g is key 4g + j
+// (j < 4) and 16 + 4g + j - 4. Memory-bound: 4 x 18.9 MB at 9216 tokens. flash_kernel ran a two-wave workgroup per
+// group there, one wave without queries up to 16 frames: 34.6 us at 8 streams x 8 frames, 22.6 at 4 x 16, 17.1 at
+// 2 x 24, 10.6 at 1 x 32; here 19.3, 19.3, 16.4 and 10.1.
+// A masked key's probability is 0, but 0 x inf is not: where a tile's V holds a non-finite value the wave adds
+// the unmasked products one key at a time, so that frames and groups stay independent.
+template <int NT>
+__global__ __launch_bounds__(256) void temporal_tile_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k,
+                                                            const bf16* __restrict__ v, bf16* __restrict__ out,
+                                                            int64_t rows, int T, int tile_rows, int P, int H,
+                                                            float scale_log2, int fks, uint8_t* __restrict__ out8,
+                                                            uint8_t* __restrict__ out8s, oasis::Prefetch pf) {
+  __shared__ __attribute__((aligned(1024))) char vs_all[4 * NT * 2048];
+  if (blockIdx.z) {  // the prefetching slice
+    prefetch_lines(pf);
+    return;
+  }
+  const int lane = threadIdx.x & 63, lr = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t r0 = ((int64_t)blockIdx.x * 4 + wave) * tile_rows;
+  if (r0 >= rows) return;
+  const int n = (int)(rows - r0 < tile_rows ? rows - r0 : tile_rows);
+  char* vs = vs_all + wave * NT * 2048;
+  const __amdgpu_buffer_rsrc_t Qrs = buffer_rsrc(q + r0 * 64), Krs = buffer_rsrc(k + r0 * 64), Vrs = buffer_rsrc(v + r0 * 64);
+  // rows past the tile read its last row; what they give is masked or not stored
+#pragma unroll
+  for (int b = 0; b < NT * 2; ++b) {
+    const int r = b * 8 + (lane >> 3), s = lane & 7;
+    const int col = ((((s >> 1) ^ ((r >> 1) & 3)) << 1) | (s & 1)) * 8;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(Vrs, (__attribute__((address_space(3))) void*)(vs + b * 1024), 16,
+                                             (min(r, n - 1) * 64 + col) * 2, 0, 0, 0);
+  }
+  bf16x8 qf[NT][2], kf[NT][2];
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int r = min(t * 16 + lr, n - 1) * 64 + g * 8;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      kf[t][h] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(Krs, (r + h * 32) * 2, 0, 0));
+      qf[t][h] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(Qrs, (r + h * 32) * 2, 0, 0));
+    }
+  }
+  float p[NT][NT][4], inv[NT];  // [query tile][key tile]
+#pragma unroll
+  for (int qt = 0; qt < NT; ++qt) {
+    const int my_q = qt * 16 + lr, first = NT == 1 ? my_q - my_q % T : 0;  // the query's group starts at row `first`
+    float mx = -INFINITY;
+#pragma unroll
+    for (int kt = 0; kt <= qt; ++kt) {
+      f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+      acc = mfma16(kf[kt][0], qf[qt][0], acc);
+      acc = mfma16(kf[kt][1], qf[qt][1], acc);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int key = kt * 16 + 4 * g + i;
+        p[qt][kt][i] = key <= my_q && key >= first ? acc[i] * scale_log2 : -INFINITY;
+        mx = fmaxf(mx, p[qt][kt][i]);
+      }
+    }
+    mx = max_xor32(max_xor16(mx));
+    const float m_use = mx == -INFINITY ? 0.f : mx;
+    float ps = 0.f;
+#pragma unroll
+    for (int kt = 0; kt <= qt; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        p[qt][kt][i] = __builtin_amdgcn_exp2f(p[qt][kt][i] - m_use);
+        ps += p[qt][kt][i];
+      }
+    inv[qt] = 1.0f / sum_xor32(sum_xor16(ps));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xF << 8));  // vmcnt(0): the wave's V rows are in its LDS
+  __builtin_amdgcn_sched_barrier(0);
+  typedef short i16x4 __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) i16x4* lds4;
+  bf16x8 va[4];
+  bool finite = true;
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt) {
+    i16x4 t[2] = {i16x4{0, 0, 0, 0}, i16x4{0, 0, 0, 0}};
+#pragma unroll
+    for (int kt = 0; kt < NT; ++kt) {
+      const int r = kt * 16 + 4 * g + (lr >> 2);
+      t[kt] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(vs + r * 128 + ((dt ^ ((r >> 1) & 3)) << 5) + (lr & 3) * 8));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) finite &= (t[kt][i] & 0x7F80) != 0x7F80;
+    }
+    va[dt] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(t[0], t[1], 0, 1, 2, 3, 4, 5, 6, 7));
+  }
+  const bool all_finite = __builtin_amdgcn_ballot_w64(!finite) == 0;
+#pragma unroll
+  for (int qt = 0; qt < NT; ++qt) {
+    f32x4 o[4];
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int my_q = qt * 16 + lr;
+    if (all_finite) {
+      bf16x8 pb;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        pb[i] = f2bf(p[qt][0][i]);
+        pb[4 + i] = qt > 0 ? f2bf(p[qt][NT - 1][i]) : f2bf(0.f);
+      }
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) o[dt] = mfma16(va[dt], pb, o[dt]);
+    } else {
+      const int first = NT == 1 ? my_q - my_q % T : 0;
+#pragma unroll
+      for (int kt = 0; kt <= qt; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int kg = 0; kg < 4; ++kg) {
+            const int key = kt * 16 + 4 * kg + i;
+            const float pk = bf2f(f2bf(__shfl(p[qt][kt][i], kg * 16 + lr, 64)));
+            if (key > my_q || key < first) continue;
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                const bf16* row = reinterpret_cast<const bf16*>(vs + key * 128 + ((dt ^ ((key >> 1) & 3)) << 5));
+                o[dt][e] += pk * bf2f(row[4 * g + e]);
+              }
+          }
+    }
+    if (my_q >= n) continue;  // the 4 lanes of a query leave together
+    const int64_t row = r0 + my_q, grp = row / T;
+    const int t = (int)(row - grp * T), h = (int)(grp % H);
+    const int64_t bp = grp / H, b = bp / P, pos = bp - b * P;
+    store_head<bf16>(out, ((b * T + t) * P + pos) * (int64_t)(H * 64) + h * 64, o, inv[qt], g, fks, out8, out8s);
   }
 }
 
@@ -561,10 +741,28 @@ int temporal_attention(const void* q, const void* k, const void* v, void* out, i
                 "temporal_attention: bad shape");
   OASIS_REQUIRE(q_frame < T, OASIS_ERR_ARG, "temporal_attention: q_frame must be < T");
   const int64_t G = B * P * n_heads;
+  const bf16 *qp = static_cast<const bf16*>(q), *kp = static_cast<const bf16*>(k), *vp = static_cast<const bf16*>(v);
+  bf16* op = static_cast<bf16*>(out);
+  const float sl = scale * LOG2E;
+  const int fks = out_frag ? (int)(n_heads * 2) : 0;
+  const unsigned gz = prefetch_any(pf) ? 2 : 1;
+  const Prefetch pfv = prefetch_or_none(pf);
   if (T >= 8 && q_frame < 0) {
-    // long causal windows on the MFMA flash kernel: each (stream, position, head) group is a
-    // contiguous [T][64] block; outputs land token-major at row (b*T + t)*P + p
+    // long causal windows: each (stream, position, head) group is a contiguous [T][64] block; outputs land
+    // token-major at row (b*T + t)*P + p. Up to 32 frames a wave per tile of rows, beyond on flash_kernel.
     OASIS_REQUIRE(G <= 65535, OASIS_ERR_SHAPE, "temporal_attention: too many (stream, position, head) groups");
+    if (T <= 32) {
+      const int tile_rows = T <= 16 ? (int)(16 / T * T) : (int)T;
+      const int64_t tiles = (G * T + tile_rows - 1) / tile_rows;
+      const dim3 grid((unsigned)((tiles + 3) / 4), 1, gz);
+      if (T <= 16)
+        hipLaunchKernelGGL((temporal_tile_kernel<1>), grid, dim3(256), 0, stream, qp, kp, vp, op, G * T, (int)T, tile_rows,
+                           (int)P, (int)n_heads, sl, fks, out8, out8_scale, pfv);
+      else
+        hipLaunchKernelGGL((temporal_tile_kernel<2>), grid, dim3(256), 0, stream, qp, kp, vp, op, G * T, (int)T, tile_rows,
+                           (int)P, (int)n_heads, sl, fks, out8, out8_scale, pfv);
+      return check_launch("temporal_attention");
+    }
     AttnArgs a;
     a.Lq = a.Lk = (int)T;
     a.q_bh = a.kv_bh = T * 64;
@@ -584,10 +782,20 @@ int temporal_attention(const void* q, const void* k, const void* v, void* out, i
     return flash_launch<bf16>(static_cast<const bf16*>(q), static_cast<const bf16*>(k), static_cast<const bf16*>(v),
                               static_cast<bf16*>(out), G, a, stream);
   }
-  hipLaunchKernelGGL(temporal_kernel, dim3((unsigned)((G + 15) / 16), 1, prefetch_any(pf) ? 2 : 1), dim3(256), 0,
-                     stream, static_cast<const bf16*>(q), static_cast<const bf16*>(k), static_cast<const bf16*>(v),
-                     static_cast<bf16*>(out), G, (int)T, (int)P, (int)n_heads, scale * LOG2E, q_frame < 0 ? -1 : q_frame,
-                     out_frag ? (int)(n_heads * 2) : 0, prefetch_or_none(pf), out8, out8_scale);
+  const dim3 grid((unsigned)((G + 15) / 16), 1, gz);
+  const int qfr = q_frame < 0 ? -1 : q_frame;
+#define OASIS_TEMPORAL(TWV)                                                                                           \
+  hipLaunchKernelGGL((temporal_kernel<TWV>), grid, dim3(256), 0, stream, qp, kp, vp, op, G, (int)T, (int)P, (int)n_heads, \
+                     sl, qfr, fks, pfv, out8, out8_scale)
+  switch (q_frame < 0 ? T : 0) {
+    case 3: OASIS_TEMPORAL(3); break;
+    case 4: OASIS_TEMPORAL(4); break;
+    case 5: OASIS_TEMPORAL(5); break;
+    case 6: OASIS_TEMPORAL(6); break;
+    case 7: OASIS_TEMPORAL(7); break;
+    default: OASIS_TEMPORAL(0);
+  }
+#undef OASIS_TEMPORAL
   return check_launch("temporal_attention");
 }
 
