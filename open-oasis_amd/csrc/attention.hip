@@ -7,8 +7,11 @@
 //   belong to one query (lane & 15): the running max/sum and the rescale of the output
 //   accumulators need only lane-group reductions, and the probabilities feed the
 //   P V product (as O^T = V^T P^T) straight from registers without an LDS round trip.
-//   Used for spatial attention (144 tokens per frame), the VAE (576 tokens) and the
-//   reference's sdpa / sdpa_causal surface (optional additive bias, causal mask).
+//   Used for sequences of up to 64 and for the reference's sdpa / sdpa_causal surface with an additive
+//   bias, a causal mask or fp32 operands.
+//
+// flash_ring_kernel: the same products without bias and mask on bf16, K and V staged as they lie:
+//   spatial attention (144 tokens per frame), the VAE (576 tokens) and the sdpa surface.
 //
 // temporal_kernel: causal attention over the T frames of one (stream, position, head)
 //   group. At T=2 each group is 2 queries x 2 keys, far below an MFMA tile, so it is a
@@ -97,7 +100,7 @@ __device__ __forceinline__ void store_fp8x4(uint8_t* q, uint8_t* sc, const float
 // inv), at row-major element offset off: as T, in fragment order, or as fp8 activation blocks. Called by all 4
 // lanes (the ones that share lane % 16) of a query together.
 template <typename T>
-__device__ __forceinline__ void store_head(T* O, int64_t off, const f32x4 (&o)[4], float inv, int g, int frag_ks,
+__device__ __forceinline__ void store_head(T* O, int64_t off, const f32x4* o, float inv, int g, int frag_ks,
                                            uint8_t* o8, uint8_t* o8s) {
   if (o8) {
     // dims 0..31 of the head are o[0..1] of the 4 lanes (lane groups g), 32..63 o[2..3]
@@ -323,18 +326,205 @@ __global__ __launch_bounds__(NW * KSPLIT * 64) void flash_kernel(const T* __rest
   store_head<T>(O, off, o, inv, g, a.frag_ks, a.o8, a.o8s);
 }
 
-// PLAIN variants (no bias, not causal) exist for bf16, the dtype of the DiT and VAE paths
+// PLAIN variants (no bias, not causal) exist for bf16 sequences of up to 64; longer ones run flash_ring_kernel
 template <int NW, int KC, int KS, typename T, int KSPLIT = 1>
 void flash_go(dim3 g, const T* q, const T* k, const T* v, T* o, const AttnArgs& a, hipStream_t s) {
   const dim3 b(NW * KSPLIT * 64);
   if (oasis::prefetch_any(&a.pf)) g.z = 2;
-  if constexpr (std::is_same<T, bf16>::value) {
+  if constexpr (std::is_same<T, bf16>::value && KS <= 64) {
     if (!a.bias && !a.causal) {
       hipLaunchKernelGGL((flash_kernel<NW, KC, KS, T, KSPLIT, true>), g, b, 0, s, q, k, v, o, a);
       return;
     }
   }
   hipLaunchKernelGGL((flash_kernel<NW, KC, KS, T, KSPLIT, false>), g, b, 0, s, q, k, v, o, a);
+}
+
+// Attention without bias or causal mask on bf16 (every spatial and VAE call). K and V rows go to LDS as they lie,
+// by direct-to-LDS loads into a ring of ST stages of KS keys (ST = 1: the whole sequence), and V is transposed on
+// the way out by ds_read_b64_tr_b16, so nothing passes through registers and stages are small enough for two or
+// three workgroups per CU: flash_kernel stages K and V^T at once (158 KB at 576 keys, one workgroup per CU) and
+// its time stepped with rounds of 256 workgroups. Rows are XOR-swizzled against bank repeats: a K row's 16-byte
+// units by row % 8, a V row's 32-byte groups by (row / 2) % 4. A stage is consumed in chunks of CT 16-key tiles;
+// KSPLIT = 2: two waves per query block, each half of every stage. The sum of the probabilities is a product with
+// ones on the matrix cores: the sum of what the products take, so that rounding to bf16 largely cancels.
+// FINE: what that rounding leaves goes through the products as a second bf16 (one stage, one chunk): chunks of 9 or
+// 10 tiles round more probabilities than the 32-key chunks of flash_kernel did, where every chunk's largest is 1.
+// Relative rms error against fp64 at 144 keys: 1.70e-3 there, 1.75e-3 without FINE, 1.66e-3 (the output's own
+// rounding) with it, for 0.3-0.9 us.
+// Measured, before -> now: 576 tokens x 1, 2, 3, 4, 8 latents 9.9, 19.3, 20.1, 28.2, 44.8 -> 9.3, 14.3, 14.8, 18.7,
+// 29.2 us; 144 tokens x 1, 8, 12, 32, 64 frames 5.1, 8.1, 11.7, 15.8, 33.1 -> 4.8, 7.0, 8.5, 11.5, 23.7 (64 frames: 75 MB,
+// 3.2 TB/s).
+template <int NW, int KSPLIT, int KS, int ST, int CT, bool FINE = false>
+__global__ __launch_bounds__(NW * KSPLIT * 64) void flash_ring_kernel(const bf16* __restrict__ Q,
+                                                                      const bf16* __restrict__ K,
+                                                                      const bf16* __restrict__ V, bf16* __restrict__ O,
+                                                                      AttnArgs a) {
+  constexpr int W = NW * KSPLIT, KT = KS / KSPLIT / 16;   // 16-key tiles of a wave in a stage
+  constexpr int BLKS = KS / 4, LPW = (BLKS + W - 1) / W;  // 1 KB blocks of 8 rows, K's then V's
+  constexpr int STAGE = KS * 256, MERGE = KSPLIT > 1 ? NW * 64 * 18 * 4 : 0;
+  constexpr int SMEM = ST * STAGE > MERGE ? ST * STAGE : MERGE;
+  constexpr int VM = ST > 1 ? (ST - 2) * LPW : 0;
+  constexpr int WAIT = (VM & 15) | ((VM >> 4) << 14) | (0x7 << 4) | (0xF << 8);
+  static_assert(KT * 16 * KSPLIT == KS && KS % 8 == 0 && SMEM <= 160 * 1024 && VM <= 63, "stages");
+  static_assert(!FINE || (ST == 1 && KSPLIT == 1 && CT == KT), "the remainders are not rescaled");
+  static_assert((KSPLIT == 1 || KSPLIT == 2) && (CT % 2 == 0 || CT == KT) && CT <= KT, "key split, chunks");
+  __shared__ __attribute__((aligned(1024))) char smem[SMEM];
+  if (blockIdx.z) {  // the prefetching slice
+    prefetch_lines(a.pf);
+    return;
+  }
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wq = wave % NW, wk = wave / NW;  // query block, key half of each stage
+  const int nqb = gridDim.x, wid = xcd_remap(blockIdx.y * nqb + blockIdx.x, nqb * gridDim.y);
+  const int bh = wid / nqb, q0 = ((wid - bh * nqb) * NW + wq) * 16;
+  const int lr = lane & 15, g = lane >> 4, my_q = q0 + lr;
+  const bf16* qp = Q + (int64_t)bh * a.q_bh + (int64_t)min(my_q, a.Lq - 1) * 64 + g * 8;
+  const bf16x8 qf0 = load8_bf16<bf16>(qp), qf1 = load8_bf16<bf16>(qp + 32);
+  const __amdgpu_buffer_rsrc_t Krs = buffer_rsrc(K + (int64_t)bh * a.kv_bh), Vrs = buffer_rsrc(V + (int64_t)bh * a.kv_bh);
+
+  const int n = (a.Lk + KS - 1) / KS;
+  auto issue = [&](int st, int buf) {  // rows past Lk are the last key's; masked below
+    char* base = smem + buf * STAGE;
+#pragma unroll
+    for (int u = 0; u < LPW; ++u) {
+      const int blk = min(wave * LPW + u, BLKS - 1);
+      const bool isv = blk >= KS / 8;
+      const int r = (isv ? blk - KS / 8 : blk) * 8 + (lane >> 3), s = lane & 7;
+      const int unit = isv ? ((((s >> 1) ^ ((r >> 1) & 3)) << 1) | (s & 1)) : s ^ (r & 7);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(isv ? Vrs : Krs, (__attribute__((address_space(3))) void*)(base + blk * 1024),
+                                               16, (uint32_t)min(st * KS + r, a.Lk - 1) * 128u + unit * 16, 0, 0, 0);
+    }
+  };
+#pragma unroll
+  for (int st = 0; st < (ST > 1 ? ST - 1 : 1); ++st) issue(min(st, n - 1), st);
+
+  float m = -INFINITY;
+  f32x4 o[5];  // o[4]: the sum of the probabilities as the products take them (ones in V's place)
+#pragma unroll
+  for (int dt = 0; dt < 5; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 ol[4];  // FINE: the products of the remainders, apart: against an infinite value they are not finite
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt) ol[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const bf16 one = f2bf(1.f);
+  const bf16x8 ones = {one, one, one, one, one, one, one, one};
+  for (int st = 0; st < n; ++st) {
+    __builtin_amdgcn_s_waitcnt(WAIT);
+    __builtin_amdgcn_s_barrier();
+    if constexpr (ST > 1) issue(min(st + ST - 1, n - 1), (st + ST - 1) % ST);  // into the buffer read at st - 1
+    if (q0 >= a.Lq) continue;
+    const char* kb = smem + (ST > 1 ? st % ST : 0) * STAGE + wk * KT * 16 * 128;
+    const char* vb = kb + KS * 128;
+    const int key0 = st * KS + wk * KT * 16;
+#pragma unroll
+    for (int c = 0; c < KT; c += CT) {
+      const int nt = KT - c < CT ? KT - c : CT;  // tiles of this chunk, known at compile time
+      // S^T: s[kt][i] = score(key key0 + (c + kt) * 16 + 4g + i, query my_q)
+      float s[CT][4], mx = -INFINITY;
+#pragma unroll
+      for (int kt = 0; kt < nt; ++kt) {
+        const char* kr = kb + ((c + kt) * 16 + lr) * 128;
+        f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+        acc = mfma16(*reinterpret_cast<const bf16x8*>(kr + ((g ^ (lr & 7)) << 4)), qf0, acc);
+        acc = mfma16(*reinterpret_cast<const bf16x8*>(kr + (((4 + g) ^ (lr & 7)) << 4)), qf1, acc);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[kt][i] = acc[i] * a.scale_log2;
+      }
+      if (key0 + (c + nt) * 16 > a.Lk) {
+#pragma unroll
+        for (int kt = 0; kt < nt; ++kt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (key0 + (c + kt) * 16 + 4 * g + i >= a.Lk) s[kt][i] = -INFINITY;
+      }
+#pragma unroll
+      for (int kt = 0; kt < nt; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[kt][i]);
+      mx = max_xor32(max_xor16(mx));
+      const float m_new = fmaxf(m, mx), m_use = m_new == -INFINITY ? 0.f : m_new;
+      const float alpha = __builtin_amdgcn_exp2f(m - m_use);
+      m = m_new;
+#pragma unroll
+      for (int kt = 0; kt < nt; ++kt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[kt][i] = __builtin_amdgcn_exp2f(s[kt][i] - m_use);
+#pragma unroll
+      for (int dt = 0; dt < 5; ++dt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[dt][i] *= alpha;
+      // O^T += V^T P^T over pairs of key tiles (of an odd count's last pair one): k-slot j of lane group g is key
+      // 4g + j (j < 4) of the first tile and 4g + j - 4 of the second
+#pragma unroll
+      for (int kp = 0; kp < (nt + 1) / 2; ++kp) {
+        typedef short i16x4 __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(3))) i16x4* lds4;
+        const bool two = 2 * kp + 1 < nt;
+        bf16x8 pb;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          pb[i] = f2bf(s[2 * kp][i]);
+          pb[4 + i] = two ? f2bf(s[two ? 2 * kp + 1 : 0][i]) : f2bf(0.f);
+        }
+        o[4] = mfma16(ones, pb, o[4]);
+        bf16x8 pl;  // FINE: what the rounding to pb left
+        if constexpr (FINE) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            pl[i] = f2bf(s[2 * kp][i] - bf2f(pb[i]));
+            pl[4 + i] = two ? f2bf(s[two ? 2 * kp + 1 : 0][i] - bf2f(pb[4 + i])) : f2bf(0.f);
+          }
+          o[4] = mfma16(ones, pl, o[4]);
+        }
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+          const int r = (c + 2 * kp) * 16 + 4 * g + (lr >> 2);  // 16 rows on: the same swizzle
+          const char* vr = vb + r * 128 + ((dt ^ ((r >> 1) & 3)) << 5) + (lr & 3) * 8;
+          const i16x4 t0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)vr);
+          i16x4 t1 = i16x4{0, 0, 0, 0};
+          if (two) t1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(vr + 16 * 128));
+          const bf16x8 va = __builtin_bit_cast(bf16x8, __builtin_shufflevector(t0, t1, 0, 1, 2, 3, 4, 5, 6, 7));
+          o[dt] = mfma16(va, pb, o[dt]);
+          if constexpr (FINE) ol[dt] = mfma16(va, pl, ol[dt]);
+        }
+      }
+    }
+  }
+  if constexpr (KSPLIT > 1) {
+    // lane-wise merge: both waves of a query block hold query lr's state in the same lanes
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();  // no load into the stages is in flight, every wave is done with them
+    float* slot = reinterpret_cast<float*>(smem) + (wq * 64 + lane) * 18;
+    if (wk == 1) {
+      slot[0] = m;
+      slot[1] = o[4][0];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) slot[2 + j] = o[j / 4][j % 4];
+    }
+    __syncthreads();
+    if (wk == 1) return;
+    const float m2 = slot[0], m_new = fmaxf(m, m2), m_use = m_new == -INFINITY ? 0.f : m_new;
+    const float a1 = __builtin_amdgcn_exp2f(m - m_use), a2 = __builtin_amdgcn_exp2f(m2 - m_use);
+    o[4][0] = o[4][0] * a1 + slot[1] * a2;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) o[j / 4][j % 4] = o[j / 4][j % 4] * a1 + slot[2 + j] * a2;
+  }
+  if (my_q >= a.Lq) return;  // the 4 lanes of a query leave together
+  if constexpr (FINE)
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      if (fabsf(ol[j / 4][j % 4]) < INFINITY) o[j / 4][j % 4] += ol[j / 4][j % 4];
+  const int f = bh / a.H, h = bh - f * a.H;
+  const int fo = f / a.f_inner, fi = f - fo * a.f_inner;
+  const int64_t off = fo * a.o_sfo + fi * a.o_sf + h * a.o_sh + (int64_t)my_q * a.o_si;
+  store_head<bf16>(O, off, o, 1.0f / o[4][0], g, a.frag_ks, a.o8, a.o8s);
+}
+
+template <int NW, int KSPLIT, int KS, int ST, int CT, bool FINE = false>
+int ring_go(const bf16* q, const bf16* k, const bf16* v, bf16* o, int64_t n_bh, const AttnArgs& a, hipStream_t s) {
+  const dim3 grid((unsigned)((a.Lq + NW * 16 - 1) / (NW * 16)), (unsigned)n_bh, oasis::prefetch_any(&a.pf) ? 2 : 1);
+  hipLaunchKernelGGL((flash_ring_kernel<NW, KSPLIT, KS, ST, CT, FINE>), grid, dim3(NW * KSPLIT * 64), 0, s, q, k, v, o, a);
+  return oasis::check_launch("attention");
 }
 
 template <typename T>
@@ -344,13 +534,10 @@ int flash_launch(const T* q, const T* k, const T* v, T* o, int64_t n_bh, const A
   OASIS_REQUIRE(a.Lq > 0 && a.Lk > 0, OASIS_ERR_SHAPE, "attention: empty sequence");
   // K and V rows are addressed by 32-bit offsets within a (frame, head) block
   OASIS_REQUIRE(a.Lk < (1 << 24), OASIS_ERR_SHAPE, "attention: Lk=%d must be below 2^24", a.Lk);
-  // staging: short sequences (up to 32 or 64 keys: the temporal windows) and whole frames (up
-  // to 160 keys, 144 per DiT frame; up to 192) in one chunk; up to 576 keys (the VAE) staged at
-  // once (158 KB of LDS) and consumed in 64-key chunks by two waves per query block; longer
-  // sequences in 576-key stages.
-  // 144-query frames take 48 queries per workgroup (each 16-query block on two waves taking
-  // alternate 32-key chunks), or with 256+ (frame, head) pairs all 144 (9 waves share one K/V
-  // staging).
+  // With a bias, a causal mask or fp32 operands, and up to 64 queries and keys: one chunk for up to 32, 64, 160 and
+  // 192 keys, beyond that 576-key stages (158 KB of LDS) consumed in 64-key chunks by two waves per query block.
+  // 48-row query counts take 48 queries per workgroup (each 16-query block on two waves taking alternate 32-key
+  // chunks), or with 256+ heads of 144 queries all 144 (9 waves share one K/V staging).
   const unsigned nb = (unsigned)n_bh;
   if (a.Lq <= 32 && a.Lk <= 32) {
     flash_go<2, 32, 32>(dim3(1, nb), q, k, v, o, a, s);
@@ -359,6 +546,24 @@ int flash_launch(const T* q, const T* k, const T* v, T* o, int64_t n_bh, const A
   if (a.Lq <= 64 && a.Lk <= 64) {
     flash_go<4, 64, 64>(dim3(1, nb), q, k, v, o, a, s);
     return oasis::check_launch("attention");
+  }
+  if constexpr (std::is_same<T, bf16>::value) {
+    if (!a.bias && !a.causal) {
+      // The smallest single stage that takes the sequence, beyond 192 keys a ring. Where 32-key chunks ran before
+      // (fewer than 256 heads, or 48-query workgroups) the probabilities keep their remainders; without them 64
+      // frames take 23.7 us instead of 25.4 and 160 keys x 160 queries x 512 heads 12.8 instead of 17.9. A ring with
+      // one workgroup per CU at most stages 128 keys (96 KB; 16 x 1000 x 1000 13.2 us, with 64 15.3), with more of
+      // them 64 (48 KB, three per CU; 3 latents 14.8, with 128 18.3).
+      if (a.Lk <= 144)
+        return n_bh >= 256 && a.Lq % 144 == 0 ? ring_go<3, 1, 144, 1, 9>(q, k, v, o, n_bh, a, s)
+                                              : ring_go<3, 1, 144, 1, 9, true>(q, k, v, o, n_bh, a, s);
+      if (a.Lk <= 160)
+        return n_bh >= 256 && (a.Lq % 64 == 0 || a.Lq % 48 != 0) ? ring_go<4, 1, 160, 1, 10>(q, k, v, o, n_bh, a, s)
+                                                                 : ring_go<3, 1, 160, 1, 10, true>(q, k, v, o, n_bh, a, s);
+      if (a.Lk <= 192) return ring_go<4, 1, 192, 1, 12>(q, k, v, o, n_bh, a, s);
+      if ((a.Lq + 63) / 64 * n_bh <= 256) return ring_go<4, 2, 128, 3, 4>(q, k, v, o, n_bh, a, s);
+      return ring_go<4, 2, 64, 3, 2>(q, k, v, o, n_bh, a, s);
+    }
   }
   const int kind = a.Lk <= 160 ? 0 : (a.Lk <= 192 ? 1 : 2);
   if (a.Lq % 64 != 0 && a.Lq % 48 == 0) {

@@ -1,0 +1,55 @@
+"""Attention without bias or causal mask: every staging variant at its edges, and non-finite values, against fp64."""
+import pytest
+import torch
+
+from helpers import L, cuda, stream, sync
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(n, sq, sk):
+    g = torch.Generator().manual_seed(n + 3 * sq + 7 * sk)
+    return [cuda(torch.randn(n, r, 64, generator=g) * 2, torch.bfloat16) for r in (sq, sk, sk)]
+
+
+def _run(q, k, v):
+    n, sq, _ = q.shape
+    out = torch.full((n, sq, 64), float("nan"), device="cuda", dtype=torch.bfloat16)
+    L.call("oasis_sdpa", L.ptr(q), L.ptr(k), L.ptr(v), L.ptr(out), n, sq, k.shape[1], 64, 0.125, None, 0, L.BF16,
+           stream())
+    sync()
+    return out.double()
+
+
+def _ref(q, k, v):
+    s = torch.matmul(q.double(), k.double().transpose(-1, -2).contiguous()) * 0.125
+    p = s.softmax(-1)
+    return torch.matmul(p, v.double()), torch.matmul(p, v.double().abs())
+
+
+# one stage of 144, 160 or 192 keys with and without the probabilities' remainders, the two rings on either side of
+# 256 workgroups; one key past a stage, one short of it, one key in the last stage, and partial query tiles
+@pytest.mark.parametrize("n,sq,sk", [(1, 1, 65), (3, 144, 143), (256, 144, 144), (255, 144, 144), (257, 65, 1),
+                                     (2, 49, 144), (2, 47, 145), (3, 48, 160), (256, 128, 160), (256, 33, 159),
+                                     (256, 48, 152), (2, 70, 161), (5, 200, 192), (2, 65, 193), (1, 16, 256),
+                                     (3, 100, 257), (4, 4096, 385), (129, 100, 193), (128, 65, 320), (300, 1, 576),
+                                     (30, 576, 576), (28, 576, 576), (300, 20, 641)])
+def test_attention_variants(n, sq, sk):
+    q, k, v = _inputs(n, sq, sk)
+    out = _run(q, k, v)
+    ref, mass = _ref(q, k, v)
+    # bf16 rounds to within 2^-8: each probability, the sum of them, and the output; 1.02 covers the fp32 scores
+    bound = 1.02 * 2.0 ** -8 * (mass + 2 * ref.abs())
+    assert torch.isfinite(out).all() and ((out - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("n,sq,sk", [(2, 144, 144), (256, 144, 144), (2, 96, 160), (2, 70, 192), (2, 64, 576)])
+def test_attention_keeps_infinite_values(n, sq, sk):
+    """An infinite value gives infinity in its dim, whatever rounding left of its probability, and in no other."""
+    q, k, v = _inputs(n, sq, sk)
+    q = q * 0.25  # no probability underflows
+    v[1, sk // 2, 9] = float("inf")
+    out = _run(q, k, v)
+    assert (out[1, :, 9] == float("inf")).all()
+    out[1, :, 9] = 0
+    assert torch.isfinite(out).all()
