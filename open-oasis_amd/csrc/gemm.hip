@@ -10,8 +10,8 @@
 //     (global_load_lds_dwordx4) into a ring of STAGES tiles; small tiles for the split-K slices
 //     and the QKV + RoPE product at 144 / 288 tokens.
 //   - gemm_big_kernel: the same ring with a grouped tile order and a per-wave staged epilogue, on
-//     4-, 6- and 8-wave tiles: the MLP products, every VAE projection, and the 8-wave 288-row
-//     tiles from 2048 tokens up.
+//     4- to 16-wave tiles: most products above 320 tokens, the VAE's among them, by measured cost
+//     (kCosts).
 //   - gemm_wave_kernel: 4 waves split each workgroup's K slice four ways, each over its own LDS
 //     ring with no workgroup barrier in the K loop; the default below 320 tokens (QKV + RoPE, O,
 //     FC1, FC2) and for the VAE's O projection.
@@ -372,7 +372,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_big_kernel(const bf16* __re
   }
 }
 
-// Wave-split K (below 2048 tokens): the 4 waves of a workgroup share one BM x BN output tile and
+// Wave-split K (few rows): the 4 waves of a workgroup share one BM x BN output tile and
 // split its K slice four ways. Each wave stages its own K tiles (global_load_lds into the same
 // swizzled 128-byte rows as above) in a private STG-deep LDS ring and multiplies them, so the K
 // loop waits only on the wave's own loads (no workgroup barrier) and every staged byte is read
@@ -1124,12 +1124,12 @@ const TileCfg kTiles[] = {
     {32, 64, launch_lds<32, 64, 1, 4, 4>},                  // 0: 4 K tiles in flight
     {32, 64, launch_lds<32, 64, 1, 4, 3>},                  // 1: 3 K tiles in flight
     // the 8-wave kernel's grouped tile order and per-wave staged epilogue on 4- and 6-wave tiles:
-    // FC1 / FC2 below 2048 tokens and every VAE projection
+    // products above 320 tokens where kCosts finds them cheapest
     {96, 64, launch_big<96, 64, 2, 2, 4>},                  // 2
     {64, 64, launch_big<64, 64, 2, 2, 4, 6>},               // 3: groups of 6 n tiles (576 tokens: an XCD's 54 tiles
                                                             //    are 6 whole weight slices)
     {144, 64, launch_big<144, 64, 3, 2, 4>},                // 4: 6 waves
-    // 8-wave large-token tiles (2048+ tokens)
+    // 8-wave large-token tiles
     {288, 256, launch_big<288, 256, 2, 4, 2>},              // 5
     {288, 192, launch_big<288, 192, 2, 4, 2>, 1},           // 6
     {288, 128, launch_big<288, 128, 2, 4, 2>},              // 7
