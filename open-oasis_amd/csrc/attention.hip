@@ -346,12 +346,12 @@ void flash_go(dim3 g, const T* q, const T* k, const T* v, T* o, const AttnArgs& 
 // three workgroups per CU: flash_kernel stages K and V^T at once (158 KB at 576 keys, one workgroup per CU) and
 // its time stepped with rounds of 256 workgroups. Rows are XOR-swizzled against bank repeats: a K row's 16-byte
 // units by row % 8, a V row's 32-byte groups by (row / 2) % 4. A stage is consumed in chunks of CT 16-key tiles;
-// KSPLIT = 2: two waves per query block, each half of every stage. The sum of the probabilities is a product with
-// ones on the matrix cores: the sum of what the products take, so that rounding to bf16 largely cancels.
-// FINE: what that rounding leaves goes through the products as a second bf16 (one stage, one chunk): chunks of 9 or
-// 10 tiles round more probabilities than the 32-key chunks of flash_kernel did, where every chunk's largest is 1.
-// Relative rms error against fp64 at 144 keys: 1.70e-3 there, 1.75e-3 without FINE, 1.66e-3 (the output's own
-// rounding) with it, for 0.3-0.9 us.
+// KSPLIT = 2: two waves per query block, each half of every stage. The sum of the probabilities is of the fp32 ones.
+// FINE: what rounding the probabilities to bf16 leaves goes through the products as a second bf16 (one stage, one
+// chunk), and their sum is a product with ones of both parts: chunks of 9 or 10 tiles round more probabilities than the
+// 32-key chunks of flash_kernel did, where every chunk's largest is 1. Relative rms error against fp64, standard normal
+// operands: at 144 keys 2.07e-3 there, 2.17e-3 without FINE, 1.66e-3 (the output's own rounding) with it, for 0.3-0.9
+// us; at 576 keys 2.16e-3 there and 2.15e-3 here.
 // Measured, before -> now: 576 tokens x 1, 2, 3, 4, 8 latents 9.9, 19.3, 20.1, 28.2, 44.8 -> 9.3, 14.3, 14.8, 18.7,
 // 29.2 us; 144 tokens x 1, 8, 12, 32, 64 frames 5.1, 8.1, 11.7, 15.8, 33.1 -> 4.8, 7.0, 8.5, 11.5, 23.7 (64 frames: 75 MB,
 // 3.2 TB/s).
@@ -400,14 +400,16 @@ __global__ __launch_bounds__(NW * KSPLIT * 64) void flash_ring_kernel(const bf16
   for (int st = 0; st < (ST > 1 ? ST - 1 : 1); ++st) issue(min(st, n - 1), st);
 
   float m = -INFINITY;
-  f32x4 o[5];  // o[4]: the sum of the probabilities as the products take them (ones in V's place)
+  float lsum = 0.f;  // of this lane's keys only (4 of 16); the 4 lanes of a query add up at the end
+  f32x4 o[4];
 #pragma unroll
-  for (int dt = 0; dt < 5; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int dt = 0; dt < 4; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  f32x4 osum = f32x4{0.f, 0.f, 0.f, 0.f};  // FINE: the sum, as a product with ones of both bf16 parts
+  const bf16 one = f2bf(1.f);
+  const bf16x8 ones = {one, one, one, one, one, one, one, one};
   f32x4 ol[4];  // FINE: the products of the remainders, apart: against an infinite value they are not finite
 #pragma unroll
   for (int dt = 0; dt < 4; ++dt) ol[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const bf16 one = f2bf(1.f);
-  const bf16x8 ones = {one, one, one, one, one, one, one, one};
   for (int st = 0; st < n; ++st) {
     __builtin_amdgcn_s_waitcnt(WAIT);
     __builtin_amdgcn_s_barrier();
@@ -445,12 +447,17 @@ __global__ __launch_bounds__(NW * KSPLIT * 64) void flash_ring_kernel(const bf16
       const float m_new = fmaxf(m, mx), m_use = m_new == -INFINITY ? 0.f : m_new;
       const float alpha = __builtin_amdgcn_exp2f(m - m_use);
       m = m_new;
+      float ps[4] = {0.f, 0.f, 0.f, 0.f};  // four chains: one of up to 48 adds takes longer than the products
 #pragma unroll
       for (int kt = 0; kt < nt; ++kt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s[kt][i] = __builtin_amdgcn_exp2f(s[kt][i] - m_use);
+        for (int i = 0; i < 4; ++i) {
+          s[kt][i] = __builtin_amdgcn_exp2f(s[kt][i] - m_use);
+          if constexpr (!FINE) ps[i] += s[kt][i];
+        }
+      lsum = lsum * alpha + ((ps[0] + ps[1]) + (ps[2] + ps[3]));
 #pragma unroll
-      for (int dt = 0; dt < 5; ++dt)
+      for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[dt][i] *= alpha;
       // O^T += V^T P^T over pairs of key tiles (of an odd count's last pair one): k-slot j of lane group g is key
@@ -466,7 +473,6 @@ __global__ __launch_bounds__(NW * KSPLIT * 64) void flash_ring_kernel(const bf16
           pb[i] = f2bf(s[2 * kp][i]);
           pb[4 + i] = two ? f2bf(s[two ? 2 * kp + 1 : 0][i]) : f2bf(0.f);
         }
-        o[4] = mfma16(ones, pb, o[4]);
         bf16x8 pl;  // FINE: what the rounding to pb left
         if constexpr (FINE) {
 #pragma unroll
@@ -474,7 +480,8 @@ __global__ __launch_bounds__(NW * KSPLIT * 64) void flash_ring_kernel(const bf16
             pl[i] = f2bf(s[2 * kp][i] - bf2f(pb[i]));
             pl[4 + i] = two ? f2bf(s[two ? 2 * kp + 1 : 0][i] - bf2f(pb[4 + i])) : f2bf(0.f);
           }
-          o[4] = mfma16(ones, pl, o[4]);
+          osum = mfma16(ones, pb, osum);
+          osum = mfma16(ones, pl, osum);
         }
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt) {
@@ -497,7 +504,7 @@ __global__ __launch_bounds__(NW * KSPLIT * 64) void flash_ring_kernel(const bf16
     float* slot = reinterpret_cast<float*>(smem) + (wq * 64 + lane) * 18;
     if (wk == 1) {
       slot[0] = m;
-      slot[1] = o[4][0];
+      slot[1] = lsum;
 #pragma unroll
       for (int j = 0; j < 16; ++j) slot[2 + j] = o[j / 4][j % 4];
     }
@@ -505,10 +512,11 @@ __global__ __launch_bounds__(NW * KSPLIT * 64) void flash_ring_kernel(const bf16
     if (wk == 1) return;
     const float m2 = slot[0], m_new = fmaxf(m, m2), m_use = m_new == -INFINITY ? 0.f : m_new;
     const float a1 = __builtin_amdgcn_exp2f(m - m_use), a2 = __builtin_amdgcn_exp2f(m2 - m_use);
-    o[4][0] = o[4][0] * a1 + slot[1] * a2;
+    lsum = lsum * a1 + slot[1] * a2;
 #pragma unroll
     for (int j = 0; j < 16; ++j) o[j / 4][j % 4] = o[j / 4][j % 4] * a1 + slot[2 + j] * a2;
   }
+  const float inv = 1.0f / (FINE ? osum[0] : sum_xor32(sum_xor16(lsum)));
   if (my_q >= a.Lq) return;  // the 4 lanes of a query leave together
   if constexpr (FINE)
 #pragma unroll
@@ -517,7 +525,7 @@ __global__ __launch_bounds__(NW * KSPLIT * 64) void flash_ring_kernel(const bf16
   const int f = bh / a.H, h = bh - f * a.H;
   const int fo = f / a.f_inner, fi = f - fo * a.f_inner;
   const int64_t off = fo * a.o_sfo + fi * a.o_sf + h * a.o_sh + (int64_t)my_q * a.o_si;
-  store_head<bf16>(O, off, o, 1.0f / o[4][0], g, a.frag_ks, a.o8, a.o8s);
+  store_head<bf16>(O, off, o, inv, g, a.frag_ks, a.o8, a.o8s);
 }
 
 template <int NW, int KSPLIT, int KS, int ST, int CT, bool FINE = false>

@@ -38,8 +38,9 @@ def test_attention_variants(n, sq, sk):
     q, k, v = _inputs(n, sq, sk)
     out = _run(q, k, v)
     ref, mass = _ref(q, k, v)
-    # bf16 rounds to within 2^-8: each probability, the sum of them, and the output; 1.02 covers the fp32 scores
-    bound = 1.02 * 2.0 ** -8 * (mass + 2 * ref.abs())
+    # bf16 rounds to within 2^-8: each probability (the sum divided by is of the unrounded ones) and the output;
+    # 1.02 covers the fp32 scores and sums
+    bound = 1.02 * 2.0 ** -8 * (mass + ref.abs())
     assert torch.isfinite(out).all() and ((out - ref).abs() <= bound).all()
 
 
@@ -53,3 +54,28 @@ def test_attention_keeps_infinite_values(n, sq, sk):
     assert (out[1, :, 9] == float("inf")).all()
     out[1, :, 9] = 0
     assert torch.isfinite(out).all()
+
+
+# every staging variant, each chunk of keys holding both kinds of rounded key
+@pytest.mark.parametrize("n,sq,sk", [(2, 144, 144), (256, 144, 144), (2, 48, 160), (256, 128, 160), (2, 70, 192),
+                                     (3, 100, 257), (2, 64, 576), (300, 20, 640)])
+def test_attention_divides_by_the_unrounded_sum(n, sq, sk):
+    """Keys whose probability bf16 rounds by nearly half a step, all in one direction, and whose values are zero
+    reach the output through the softmax sum alone: the sum is of the fp32 probabilities."""
+    s = torch.arange(-1.0, 0.0, 2.0 ** -8, dtype=torch.float64)   # scores that bf16 holds
+    p = s.exp()
+    off = (p.float().bfloat16().double() / p - 1)
+    s = s[off.argmax()].item()
+    assert off.max() > 0.003
+    scores = torch.full((sk,), s, dtype=torch.float64)
+    scores[::16] = 0                            # the largest score of every chunk: a probability of 1
+    q, k, v = (torch.zeros(n, r, 64) for r in (sq, sk, sk))
+    q[:, :, 0], k[:, :, 0] = 8, scores.float()  # q . k / 8
+    v[:, sk - sk % 16 - 16] = torch.rand(n, 64, generator=torch.Generator().manual_seed(sk)).bfloat16().float() + 1
+    v = v.bfloat16().float()
+    out = _run(*(cuda(t, torch.bfloat16) for t in (q, k, v)))
+    ref = (v.double().sum(1) / scores.exp().sum()).unsqueeze(1).cuda().expand_as(out)
+    # one value with probability 1: exact but for fp32 (1e-5) and the output's rounding, to within 2^-8 of the
+    # power of two below it (half a step of 2^-7)
+    half_step = torch.exp2(torch.floor(torch.log2(ref))) * 2.0 ** -8
+    assert ((out - ref).abs() <= half_step + 1e-5 * ref).all()
