@@ -348,7 +348,7 @@ void flash_go(dim3 g, const T* q, const T* k, const T* v, T* o, const AttnArgs& 
 // units by row % 8, a V row's 32-byte groups by (row / 2) % 4. A stage is consumed in chunks of CT 16-key tiles;
 // KSPLIT = 2: two waves per query block, each half of every stage. The sum of the probabilities is of the fp32 ones.
 // FINE: what rounding the probabilities to bf16 leaves goes through the products as a second bf16 (one stage, one
-// chunk), and their sum is a product with ones of both parts: chunks of 9 or 10 tiles round more probabilities than the
+// chunk), and their sum is a product with ones of both parts: chunks of 6 to 10 tiles round more probabilities than the
 // 32-key chunks of flash_kernel did, where every chunk's largest is 1. Relative rms error against fp64, standard normal
 // operands: at 144 keys 2.07e-3 there, 2.17e-3 without FINE, 1.66e-3 (the output's own rounding) with it, for 0.3-0.9
 // us; at 576 keys 2.16e-3 there and 2.15e-3 here.
@@ -557,17 +557,26 @@ int flash_launch(const T* q, const T* k, const T* v, T* o, int64_t n_bh, const A
   }
   if constexpr (std::is_same<T, bf16>::value) {
     if (!a.bias && !a.causal) {
-      // The smallest single stage that takes the sequence, beyond 192 keys a ring. Where 32-key chunks ran before
-      // (fewer than 256 heads, or 48-query workgroups) the probabilities keep their remainders; without them 64
-      // frames take 23.7 us instead of 25.4 and 160 keys x 160 queries x 512 heads 12.8 instead of 17.9. A ring with
-      // one workgroup per CU at most stages 128 keys (96 KB; 16 x 1000 x 1000 13.2 us, with 64 15.3), with more of
-      // them 64 (48 KB, three per CU; 3 latents 14.8, with 128 18.3).
+      // The smallest single stage that takes the sequence, beyond 192 keys a ring. Up to 160 keys the probabilities
+      // keep their remainders, but with 256 heads of whole-frame or 64-row queries, which flash_kernel took in one
+      // chunk: there 64 frames take 23.7 us without, 25.4 with them. 96- and 128-key stages keep short sequences
+      // from computing 144 (255 heads of 128 x 128: 8.0 us on flash_kernel, 8.8 on 144 keys, 6.9 on 128). At 160
+      // keys 64-query workgroups where 48-query ones would be more than two per CU, or one if 64 divides the
+      // queries (200 heads of 160 x 160: 48 9.2 us, 64 8.5; 64 x 160: 6.9, 5.7), else 48 (32 heads of 160 x 160:
+      // 5.3, with 64 5.4). A ring with one workgroup per CU at most stages 128 keys (96 KB; 16 x 1000 x
+      // 1000 13.2 us, with 64 15.3), with more of them 64 (48 KB, three per CU; 3 latents 14.6, with 128 18.3).
+      if (a.Lk <= 96) return ring_go<3, 1, 96, 1, 6, true>(q, k, v, o, n_bh, a, s);
+      if (a.Lk <= 128) return ring_go<4, 1, 128, 1, 8, true>(q, k, v, o, n_bh, a, s);
       if (a.Lk <= 144)
         return n_bh >= 256 && a.Lq % 144 == 0 ? ring_go<3, 1, 144, 1, 9>(q, k, v, o, n_bh, a, s)
                                               : ring_go<3, 1, 144, 1, 9, true>(q, k, v, o, n_bh, a, s);
-      if (a.Lk <= 160)
-        return n_bh >= 256 && (a.Lq % 64 == 0 || a.Lq % 48 != 0) ? ring_go<4, 1, 160, 1, 10>(q, k, v, o, n_bh, a, s)
-                                                                 : ring_go<3, 1, 160, 1, 10, true>(q, k, v, o, n_bh, a, s);
+      if (a.Lk <= 160) {
+        const bool q64 = a.Lq % 64 == 0 || a.Lq % 48 != 0;
+        if (q64 && n_bh >= 256) return ring_go<4, 1, 160, 1, 10>(q, k, v, o, n_bh, a, s);
+        if (q64 && (a.Lq + 47) / 48 * n_bh > (a.Lq % 64 == 0 ? 256 : 512))
+          return ring_go<4, 1, 160, 1, 10, true>(q, k, v, o, n_bh, a, s);
+        return ring_go<3, 1, 160, 1, 10, true>(q, k, v, o, n_bh, a, s);
+      }
       if (a.Lk <= 192) return ring_go<4, 1, 192, 1, 12>(q, k, v, o, n_bh, a, s);
       if ((a.Lq + 63) / 64 * n_bh <= 256) return ring_go<4, 2, 128, 3, 4>(q, k, v, o, n_bh, a, s);
       return ring_go<4, 2, 64, 3, 2>(q, k, v, o, n_bh, a, s);

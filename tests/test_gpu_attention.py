@@ -27,9 +27,11 @@ def _ref(q, k, v):
     return torch.matmul(p, v.double()), torch.matmul(p, v.double().abs())
 
 
-# one stage of 144, 160 or 192 keys with and without the probabilities' remainders, the two rings on either side of
-# 256 workgroups; one key past a stage, one short of it, one key in the last stage, and partial query tiles
-@pytest.mark.parametrize("n,sq,sk", [(1, 1, 65), (3, 144, 143), (256, 144, 144), (255, 144, 144), (257, 65, 1),
+# one stage of 96 to 192 keys with and without the probabilities' remainders, the two rings on either side of 256
+# workgroups; one key past a stage, one short of it, one key in the last stage, and partial query tiles
+@pytest.mark.parametrize("n,sq,sk", [(1, 1, 65), (2, 97, 96), (300, 48, 95), (3, 64, 97), (2, 65, 128), (260, 130, 127),
+                                     (1, 1, 129), (200, 160, 160), (171, 150, 146), (129, 64, 145), (3, 144, 143),
+                                     (256, 144, 144), (255, 144, 144), (257, 65, 1),
                                      (2, 49, 144), (2, 47, 145), (3, 48, 160), (256, 128, 160), (256, 33, 159),
                                      (256, 48, 152), (2, 70, 161), (5, 200, 192), (2, 65, 193), (1, 16, 256),
                                      (3, 100, 257), (4, 4096, 385), (129, 100, 193), (128, 65, 320), (300, 1, 576),
@@ -44,7 +46,8 @@ def test_attention_variants(n, sq, sk):
     assert torch.isfinite(out).all() and ((out - ref).abs() <= bound).all()
 
 
-@pytest.mark.parametrize("n,sq,sk", [(2, 144, 144), (256, 144, 144), (2, 96, 160), (2, 70, 192), (2, 64, 576)])
+@pytest.mark.parametrize("n,sq,sk", [(2, 144, 144), (256, 144, 144), (2, 96, 160), (2, 70, 192), (2, 64, 576),
+                                     (2, 96, 96), (2, 100, 128), (200, 160, 160)])
 def test_attention_keeps_infinite_values(n, sq, sk):
     """An infinite value gives infinity in its dim, whatever rounding left of its probability, and in no other."""
     q, k, v = _inputs(n, sq, sk)
@@ -58,7 +61,8 @@ def test_attention_keeps_infinite_values(n, sq, sk):
 
 # every staging variant, each chunk of keys holding both kinds of rounded key
 @pytest.mark.parametrize("n,sq,sk", [(2, 144, 144), (256, 144, 144), (2, 48, 160), (256, 128, 160), (2, 70, 192),
-                                     (3, 100, 257), (2, 64, 576), (300, 20, 640)])
+                                     (3, 100, 257), (2, 64, 576), (300, 20, 640), (2, 96, 96), (2, 100, 128),
+                                     (200, 160, 160)])
 def test_attention_divides_by_the_unrounded_sum(n, sq, sk):
     """Keys whose probability bf16 rounds by nearly half a step, all in one direction, and whose values are zero
     reach the output through the softmax sum alone: the sum is of the fp32 probabilities."""
