@@ -750,7 +750,7 @@ __global__ __launch_bounds__(256) void temporal_tile_kernel(const bf16* __restri
   }
   const int lane = threadIdx.x & 63, lr = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t r0 = ((int64_t)blockIdx.x * 4 + wave) * tile_rows;
+  const int64_t r0 = ((int64_t)blockIdx.x * (blockDim.x >> 6) + wave) * tile_rows;
   if (r0 >= rows) return;
   const int n = (int)(rows - r0 < tile_rows ? rows - r0 : tile_rows);
   char* vs = vs_all + wave * NT * 2048;
@@ -976,12 +976,17 @@ int temporal_attention(const void* q, const void* k, const void* v, void* out, i
     if (T <= 32) {
       const int tile_rows = T <= 16 ? (int)(16 / T * T) : (int)T;
       const int64_t tiles = (G * T + tile_rows - 1) / tile_rows;
-      const dim3 grid((unsigned)((tiles + 3) / 4), 1, gz);
+      // up to 12 tiles per CU a workgroup each: four waves in one leave CUs idle (256 groups of 24 frames 4.2 us on
+      // flash_kernel, 4.9 with four waves, 4.3 with one; 2304 groups of 16: 7.1, 5.6, 5.2); beyond, four start faster
+      // (9216 groups of 32: 25.8 us, 27.2 with one). As fp8 blocks 256 groups of 24 take 5.0 us, 4.3 on flash_kernel,
+      // which lets a masked frame's infinite value into the earlier ones.
+      const int waves = tiles <= 12 * 256 ? 1 : 4;
+      const dim3 grid((unsigned)((tiles + waves - 1) / waves), 1, gz), block(waves * 64);
       if (T <= 16)
-        hipLaunchKernelGGL((temporal_tile_kernel<1>), grid, dim3(256), 0, stream, qp, kp, vp, op, G * T, (int)T, tile_rows,
+        hipLaunchKernelGGL((temporal_tile_kernel<1>), grid, block, 0, stream, qp, kp, vp, op, G * T, (int)T, tile_rows,
                            (int)P, (int)n_heads, sl, fks, out8, out8_scale, pfv);
       else
-        hipLaunchKernelGGL((temporal_tile_kernel<2>), grid, dim3(256), 0, stream, qp, kp, vp, op, G * T, (int)T, tile_rows,
+        hipLaunchKernelGGL((temporal_tile_kernel<2>), grid, block, 0, stream, qp, kp, vp, op, G * T, (int)T, tile_rows,
                            (int)P, (int)n_heads, sl, fks, out8, out8_scale, pfv);
       return check_launch("temporal_attention");
     }

@@ -20,9 +20,10 @@ def _inputs(B, P, H, T):
     return [cuda(torch.randn(B, P, H, T, 64, generator=g) * 2, torch.bfloat16) for _ in range(3)]
 
 
-# every window length; 5 x 7 x 3 = 105 groups leave the last tile, the last wave and the last block partly empty
-@pytest.mark.parametrize("B,P,H", [(1, 1, 1), (5, 7, 3)])
-@pytest.mark.parametrize("T", list(range(3, 34)))
+# every window length; 5 x 7 x 3 = 105 groups leave the last tile, the last wave and the last block partly empty.
+# Above 3072 tiles a workgroup takes four of them: 6201 groups two to a tile, 3101 one to a tile
+@pytest.mark.parametrize("B,P,H,T", [(B, P, H, T) for T in range(3, 34) for B, P, H in ((1, 1, 1), (5, 7, 3))]
+                         + [(3, 689, 3, 8), (7, 443, 1, 11), (7, 443, 1, 16), (7, 443, 1, 17), (7, 443, 1, 24)])
 def test_temporal_windows(B, P, H, T):
     q, k, v = _inputs(B, P, H, T)
     out = _run(q, k, v).double()
