@@ -1,7 +1,8 @@
-// Skinny GEMM for up to 32 conditioning rows per pass (adaLN projections and the conditioning
-// MLP): out[r, n] = act_out(sum_k act_in(x[r, k]) W[n, k] + b[n]).
+// Skinny GEMM for conditioning rows (adaLN projections and the conditioning MLP):
+// out[r, n] = act_out(sum_k act_in(x[r, k]) W[n, k] + b[n]). gemv_kernel takes up to 32 rows per pass over W,
+// gemv_rows_kernel up to 96 of tile-order weights, gemv_f32_kernel and gemm_f32_kernel fp32 weights.
 //
-// This is pure weight streaming (the adaLN matrices of all sub-blocks are 406 MB of
+// gemv_kernel is pure weight streaming (the adaLN matrices of all sub-blocks are 406 MB of
 // bf16 per DiT step against ~0.8 GFLOP), so the kernel is shaped around HBM:
 //   - W rows are read as 16-byte streaming vectors straight into MFMA A operands
 //     (v_mfma_f32_16x16x32_bf16, 16 weight rows x 32 k per instruction), two k-steps
@@ -23,7 +24,7 @@ namespace {
 constexpr int KSTEP = 64;   // k per pipeline step (two MFMAs)
 // pipeline steps whose loads are issued together (gemv_tiles' UNROLL): 4 with one 16-row group of
 // x; 8 with two, whose staged x (132 KB at 32 rows) leaves one workgroup per CU, so each wave keeps
-// more in flight (the config-4 adaLN pass over 32 rows 180 -> 171 us)
+// more in flight (32 rows over 196608 x 1024 row-major weights 180 -> 171 us)
 
 // TILED: W in 16-row MFMA tile order (for tile t and 32-wide K step s, the 64 lanes' 16-byte
 // pieces back to back, lane l holding row 16t + (l & 15), columns 32s + 8(l >> 4) .. +7), so a
@@ -158,7 +159,7 @@ __global__ __launch_bounds__(256) void gemv_kernel(const float* __restrict__ x, 
   gemv_tiles<RG, KS, TILED>(x, ldx, R, W, N, K, b, out, ld_out, act_in, act_out, accumulate, blockIdx.x, gridDim.x);
 }
 
-// Many conditioning rows over tile-order weights (9 rows up: a longer window, several streams, a video
+// Many conditioning rows over tile-order weights (rows_min up: a longer window, several streams, a video
 // batch) in one pass over W per 96 rows. A workgroup's 4 waves take 3 weight tiles each (48 output
 // columns a wave) and walk K in 64-wide chunks: the chunk of x (RG groups of 16 rows, activation applied,
 // hi + lo bf16 halves in MFMA fragment order) is staged in LDS, double-buffered, while the weights
@@ -301,10 +302,14 @@ __global__ __launch_bounds__(256) void gemv_rows_kernel(const float* __restrict_
 
 namespace {
 
-// rows of x per pass of gemv_rows_kernel, and the fewest it takes (9 rows: 76 us against 81 on gemv_kernel;
-// up to 8 rows the step's pair kernel, whose workgroups stage x once)
-// and the fewest outputs: below 512 weight tiles gemv_kernel splits K over the waves instead
-constexpr int64_t kRowsPass = 96, kRowsMin = 9, kRowsMinN = 512 * 16;
+// rows of x per pass of gemv_rows_kernel, and the fewest outputs: below 512 weight tiles gemv_kernel splits K over
+// the waves instead
+constexpr int64_t kRowsPass = 96, kRowsMinN = 512 * 16;
+// The fewest rows: its waves cross a barrier per 64-wide chunk of K, which few rows or few chunks do not repay. At
+// 12288 outputs, gemv_kernel and here: K = 64 x 16 rows 3.9 and 4.5 us, x 32 5.5 and 5.7; K = 256 x 9 5.5 and 7.1,
+// x 16 7.3 and 6.9; K = 1024 x 9 15.9 and 17.2, x 12 19.0 and 17.2. From 24576 outputs one row less (196608 x 1024,
+// 9 rows: 81 and 76). Up to 8 rows the step's pair kernel, whose workgroups stage x once, or gemv_kernel.
+int64_t rows_min(int64_t N, int64_t K) { return std::max<int64_t>(9, 9 + 1536 / K - (N >= 24576 ? 1 : 0)); }
 
 int gemv_rows(const float* x, int64_t ldx, int64_t R, const bf16* W, int64_t N, int64_t K, const float* b, float* out,
               int64_t ld_out, int act_in, int act_out, int accumulate, hipStream_t s) {
@@ -347,7 +352,7 @@ int gemv_bf16(const float* x, int64_t ldx, int64_t R, const void* W, int64_t N, 
   OASIS_REQUIRE((act_in == OASIS_ACT_NONE || act_in == OASIS_ACT_SILU) &&
                     (act_out == OASIS_ACT_NONE || act_out == OASIS_ACT_SILU),
                 OASIS_ERR_ARG, "gemv: bad activation");
-  if (tiled && R >= kRowsMin && N >= kRowsMinN)
+  if (tiled && N >= kRowsMinN && R >= rows_min(N, K))
     return gemv_rows(x, ldx, R, static_cast<const bf16*>(W), N, K, b, out, ld_out, act_in, act_out, accumulate,
                      static_cast<hipStream_t>(stream));
   // one pass over W per 32 rows (two 16-row groups) while x fits in LDS, else per 16 rows

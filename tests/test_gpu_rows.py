@@ -16,10 +16,12 @@ def _silu(x):
 @pytest.mark.parametrize("R,N,K,off,act_in,act_out,acc", [(9, 8192, 64, 0, 1, 0, 0), (16, 8208, 320, 0, 0, 1, 0),
                                                           (33, 9216, 1024, 0, 1, 0, 1), (80, 8224, 1024, 0, 1, 0, 0),
                                                           (96, 8400, 192, 1, 1, 0, 0), (97, 8400, 448, 0, 1, 1, 1),
-                                                          (200, 8192, 2048, 3, 0, 0, 0), (40, 8176, 128, 0, 1, 0, 0)])
+                                                          (200, 8192, 2048, 3, 0, 0, 0), (40, 8176, 128, 0, 1, 0, 0),
+                                                          (33, 8192, 64, 0, 1, 0, 0), (10, 8192, 1024, 2, 1, 0, 1),
+                                                          (9, 24592, 1024, 0, 1, 0, 0), (9, 8192, 2048, 0, 0, 1, 0)])
 def test_tiled_rows(R, N, K, off, act_in, act_out, acc):
-    """off: x rows that start `off` floats past a 16-byte boundary. N = 8176 is below the kernel's range. In it
-    the row-major kernel gives the same bits."""
+    """off: x rows that start `off` floats past a 16-byte boundary. N = 8176 and 9 rows of K = 64 are below the
+    kernel's range, the last four shapes its fewest rows. The row-major kernel gives the same bits."""
     g = torch.Generator().manual_seed(R + N)
     W = (torch.randn(N, K, generator=g) * 0.05).to(torch.bfloat16)
     x, b, o0 = torch.randn(R, K, generator=g) * 2, torch.randn(N, generator=g), torch.randn(R, N + 4, generator=g)
@@ -69,14 +71,16 @@ def test_f32_rows(R, N, K, act_in, act_out, acc):
     assert (out.cpu().double() - y).norm() <= (1e-4 if act_in == 2 else 2e-6) * y.norm()
 
 
-def test_conditioning_rows_do_not_depend_on_the_batch():
-    """The rows of a 41-row conditioning call (the MFMA kernels, [hid | action] side by side) against the same
-    rows 8 at a time (the step's kernels): fp32 sums in another order."""
+@pytest.mark.parametrize("R", [9, 41, 96, 97])
+def test_conditioning_rows_do_not_depend_on_the_batch(R):
+    """The rows of one conditioning call (the MFMA kernels, [hid | action] side by side, and the adaLN rows kernel
+    from its fewest rows to a second pass) against the same rows 8 at a time (the step's kernels): fp32 sums in
+    another order."""
     dr = pkg.synth.Draw(3)
-    w = pkg.synth.dit_weights(dr, n_blocks=1, d=256, n_heads=4, d_mlp=1024)
+    # 4 sub-blocks of D = 1024: 24576 stacked adaLN outputs
+    w = pkg.synth.dit_weights(dr, n_blocks=2, d=1024, n_heads=16, d_mlp=1024)
     dit = pkg.DiT(w, "cuda")
-    R = 41
-    ws = dit.workspace(144, max_cond=48)
+    ws = dit.workspace(144, max_cond=112)
     t, a = dr.randint(0, 1000, (R,)).float().cuda(), pkg.synth.one_hot_actions(dr, R).cuda()
     many = dit.conditioning(t, a, ws).clone()
     few = torch.cat([dit.conditioning(t[i:i + 8], a[i:i + 8], ws).clone() for i in range(0, R, 8)])
