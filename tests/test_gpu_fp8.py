@@ -186,11 +186,14 @@ def test_quantize_act_fp8_matches_oracle():
 
 
 @pytest.mark.parametrize("kind,F,T,H", [("spatial", 2, 1, 16), ("spatial", 1, 1, 4), ("temporal", 2, 2, 4),
-                                         ("temporal", 2, 4, 4), ("temporal", 1, 13, 4), ("temporal", 1, 32, 2)])
+                                         ("temporal", 2, 4, 4), ("temporal", 1, 13, 4), ("temporal", 1, 32, 2),
+                                         ("spatial", 16, 1, 16), ("temporal", 3, 1, 4), ("temporal", 1, 7, 4),
+                                         ("temporal", 2, 16, 16), ("temporal", 1, 33, 2), ("temporal", 2, 48, 1)])
 def test_attention_fp8_output_equals_quantized_bf16(kind, F, T, H):
     """The attention kernels' fp8-block output (the fp8 step's O operand, written in the attention
-    launch) is bit for bit oasis_quantize_act_fp8 of their bf16 output: the spatial flash kernel,
-    the temporal VALU kernel (T = 2 and its general loop) and the causal flash kernel (T >= 8)."""
+    launch) is bit for bit oasis_quantize_act_fp8 of their bf16 output: the spatial ring kernel with and without
+    remainders, the temporal VALU kernel (its general loop at T = 1, T = 2, and the rows loaded ahead at 4 and 7),
+    the tile kernel (8 to 32, one wave and four to a workgroup) and the causal flash kernel (33 and up)."""
     P = 144
     rows = F * T * P
     D = H * 64
