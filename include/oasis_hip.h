@@ -235,6 +235,11 @@ int oasis_gemm_bf16_config(const void* A, int64_t lda, const void* B, int64_t ld
                            int64_t N, int64_t K, const oasis_epilogue_t* epi, int tile, int splits,
                            oasis_stream_t stream);
 
+/* The tile configuration that -1 stands for: of oasis_gemm_bf16_config, or (fp8 != 0) of oasis_gemm_fp8_a8;
+ * a negative error code for shapes or epilogue kinds that neither takes. Host only.
+ * No counterpart in the reference (a tuning query, for benchmarks and tests). */
+int oasis_gemm_tile(int64_t M, int64_t N, int64_t K, int kind, int splits, int fp8);
+
 /* acc[M,N] = A[M,K] @ B[N,K]^T with both operands in MFMA fragment order: A [a_rows, K] (a_rows
  * >= M rounded up to the tile: 48 rows for M <= 160, else 80; rows past M are read and their
  * results dropped), B [N, K]. Each workgroup's 8 waves split its K slice, every load issued

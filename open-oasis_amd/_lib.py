@@ -115,6 +115,7 @@ SIGNATURES = {
     "oasis_sdpa": [c_p, c_p, c_p, c_p, c_i64, c_i64, c_i64, c_i64, c_f, c_p, c_i, c_i, c_p],
     "oasis_gemm_bf16": [c_p, c_i64, c_p, c_i64, c_i64, c_i64, c_i64, P(Epilogue), c_p],
     "oasis_gemm_bf16_config": [c_p, c_i64, c_p, c_i64, c_i64, c_i64, c_i64, P(Epilogue), c_i, c_i, c_p],
+    "oasis_gemm_tile": [c_i64, c_i64, c_i64, c_i, c_i, c_i],
     "oasis_gemm_bf16_frag": [c_p, c_i64, c_p, c_i64, c_i64, c_i64, P(Epilogue), c_i, c_p],
     "oasis_dit_frag_plan": [c_i64],
     "oasis_gemm_fp8": [c_p, c_i64, c_p, c_i64, c_p, c_i64, c_i64, c_i64, P(Epilogue), c_i, c_i, c_p],

@@ -1167,28 +1167,30 @@ const TileCfg kTiles[] = {
 };
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
-// Fitted costs (tile_cost) of the tiles used above 320 tokens: c, a and b for the plain and GELU
-// stores, QKV + RoPE, and the fp32 residual and partial-sum epilogues.
-const TileCost kCosts[] = {
-    {2, {{0.25f, 0.374f, 0.00f}, {3.80f, 0.300f, 0.00f}, {3.71f, 0.235f, 1.04f}}},  // 96 x 64
-    {3, {{1.35f, 0.287f, 0.00f}, {0.20f, 0.298f, 0.00f}, {3.45f, 0.181f, 0.79f}}},  // 64 x 64
-    {4, {{2.48f, 0.555f, 0.00f}, {2.15f, 0.722f, 0.00f}, {1.48f, 0.375f, 3.43f}}},  // 144 x 64
-    {9, {{0.00f, 0.173f, 0.00f}, {3.31f, 0.129f, 0.00f}, {1.26f, 0.090f, 1.12f}}},  // 48 x 32
-    {10, {{2.85f, 0.271f, 0.00f}, {2.44f, 0.279f, 0.00f}, {1.48f, 0.147f, 2.28f}}},  // 48 x 64
-    {11, {{2.53f, 0.319f, 0.00f}, {1.89f, 0.324f, 0.00f}, {1.47f, 0.172f, 2.71f}}},  // 64 x 64
-    {12, {{-3.05f, 0.287f, 0.00f}, {2.48f, 0.211f, 0.00f}, {1.45f, 0.113f, 1.86f}}},  // 32 x 64
-    {18, {{2.19f, 0.787f, 0.00f}, {1.10f, 0.811f, 0.00f}, {0.79f, 0.528f, 5.23f}}},  // 144 x 128
-    {19, {{8.94f, 0.644f, 0.00f}, {6.75f, 0.668f, 0.00f}, {3.35f, 0.684f, 3.14f}}},  // 192 x 128
-    {20, {{0.78f, 1.029f, 0.00f}, {0.37f, 1.208f, 0.00f}, {0.74f, 0.626f, 6.26f}}},  // 192 x 128
-    {21, {{-0.16f, 1.402f, 0.00f}, {-0.84f, 1.527f, 0.00f}, {-0.86f, 0.838f, 9.16f}}},  // 144 x 256
-    {22, {{2.68f, 1.270f, 0.00f}, {-0.48f, 1.319f, 0.00f}, {-0.25f, 0.866f, 7.63f}}},  // 192 x 192
-    {23, {{2.59f, 0.602f, 0.00f}, {3.17f, 0.724f, 0.00f}, {1.61f, 0.429f, 3.57f}}},  // 96 x 128
-    {24, {{8.86f, 0.396f, 0.00f}, {6.93f, 0.372f, 0.00f}, {5.18f, 0.459f, 0.89f}}},  // 96 x 128
-    {25, {{1.63f, 0.753f, 0.00f}, {1.38f, 0.918f, 0.00f}, {1.14f, 0.490f, 4.60f}}},  // 128 x 128
-    {26, {{-2.32f, 2.061f, 0.00f}, {-1.76f, 1.971f, 0.00f}, {-2.81f, 1.197f, 13.58f}}},  // 256 x 256
-    {27, {{-1.88f, 2.319f, 0.00f}, {-1.23f, 2.289f, 0.00f}, {-4.66f, 1.369f, 16.58f}}},  // 288 x 256
-    {28, {{-0.66f, 1.286f, 0.00f}, {-0.80f, 1.360f, 0.00f}, {-0.57f, 0.702f, 9.04f}}},  // 256 x 128
-    {29, {{2.27f, 0.703f, 0.00f}, {2.06f, 0.813f, 0.00f}, {1.31f, 0.467f, 4.25f}}},  // 144 x 96
+// Fitted costs (tile_cost) of the tiles used above 320 tokens: c, lat, a and b for the plain and GELU
+// stores, QKV + RoPE, the fp32 residual, and split-K slices of 512 and longer (with which split counts
+// are chosen: fitted to the DiT's O and FC2 products; shorter slices cost as residuals).
+const TileCost<4> kCosts[] = {
+    {1, {{2.498f, 0.29f, 0.146f, 0.359f}, {2.861f, 0.196f, 0.131f, 0.519f}, {2.739f, 0.295f, 0.143f, 0.758f}, {kNever, 0, 0, 0}}},  // 32 x 64
+    {2, {{3.144f, 0.289f, 0.221f, 1.341f}, {3.801f, 0.247f, 0.233f, 1.393f}, {2.357f, 0.327f, 0.243f, 1.835f}, {3.71f, 0.0f, 0.235f, 1.04f}}},  // 96 x 64
+    {3, {{2.788f, 0.281f, 0.177f, 0.919f}, {3.13f, 0.574f, 0.179f, 1.07f}, {3.073f, 0.283f, 0.145f, 1.087f}, {3.45f, 0.0f, 0.181f, 0.79f}}},  // 64 x 64
+    {4, {{1.588f, 0.365f, 0.433f, 2.857f}, {1.924f, 0.823f, 0.451f, 6.63f}, {2.42f, 0.087f, 0.333f, 3.211f}, {1.48f, 0.0f, 0.375f, 3.43f}}},  // 144 x 64
+    {9, {{1.79f, 0.07f, 0.108f, 0.763f}, {3.51f, 0.368f, 0.07f, 0.92f}, {1.782f, 0.153f, 0.095f, 0.892f}, {1.26f, 0.0f, 0.09f, 1.12f}}},  // 48 x 32
+    {10, {{1.5f, 0.009f, 0.136f, 2.527f}, {2.694f, 0.591f, 0.082f, 3.536f}, {1.943f, 0.036f, 0.08f, 4.271f}, {1.48f, 0.0f, 0.147f, 2.28f}}},  // 48 x 64
+    {11, {{1.5f, 0.244f, 0.158f, 2.355f}, {1.854f, 0.202f, 0.133f, 3.704f}, {1.888f, 0.242f, 0.142f, 2.944f}, {1.47f, 0.0f, 0.172f, 2.71f}}},  // 64 x 64
+    {12, {{1.819f, 0.12f, 0.099f, 1.441f}, {3.391f, 0.188f, 0.126f, 1.767f}, {1.688f, 0.011f, 0.154f, 1.716f}, {1.45f, 0.0f, 0.113f, 1.86f}}},  // 32 x 64
+    {18, {{1.5f, 0.422f, 0.597f, 3.811f}, {2.933f, 0.191f, 0.581f, 3.193f}, {1.5f, 0.557f, 0.558f, 5.961f}, {0.79f, 0.0f, 0.528f, 5.23f}}},  // 144 x 128
+    {19, {{3.741f, 0.83f, 0.551f, 2.403f}, {4.851f, 1.1f, 0.57f, 2.678f}, {2.474f, 0.871f, 0.568f, 6.12f}, {3.35f, 0.0f, 0.684f, 3.14f}}},  // 192 x 128
+    {20, {{1.631f, 0.346f, 0.625f, 4.644f}, {2.921f, 0.192f, 0.68f, 6.32f}, {2.926f, 0.539f, 0.626f, 5.845f}, {0.74f, 0.0f, 0.626f, 6.26f}}},  // 192 x 128
+    {21, {{1.5f, 0.809f, 0.847f, 6.038f}, {8.498f, 0.345f, 1.113f, 2.543f}, {5.977f, 0.098f, 0.801f, 5.207f}, {-0.86f, 0.0f, 0.838f, 9.16f}}},  // 144 x 256
+    {22, {{1.656f, 1.03f, 0.843f, 5.323f}, {2.705f, 0.291f, 1.051f, 3.816f}, {7.087f, 0.657f, 0.935f, 4.547f}, {-0.25f, 0.0f, 0.866f, 7.63f}}},  // 192 x 192
+    {23, {{1.524f, 0.487f, 0.444f, 3.192f}, {5.548f, 0.433f, 0.422f, 2.181f}, {1.956f, 0.406f, 0.385f, 4.377f}, {1.61f, 0.0f, 0.429f, 3.57f}}},  // 96 x 128
+    {24, {{3.319f, 0.861f, 0.48f, 1.492f}, {4.583f, 0.755f, 0.401f, 0.861f}, {2.414f, 0.762f, 0.456f, 3.735f}, {5.18f, 0.0f, 0.459f, 0.89f}}},  // 96 x 128
+    {25, {{2.413f, 0.187f, 0.539f, 2.632f}, {6.803f, 0.256f, 0.71f, 1.42f}, {1.5f, 0.072f, 0.459f, 5.717f}, {1.14f, 0.0f, 0.49f, 4.6f}}},  // 128 x 128
+    {26, {{1.55f, 1.584f, 1.229f, 7.698f}, {1.915f, 1.107f, 1.327f, 8.819f}, {1.5f, 0.467f, 1.336f, 20.787f}, {-2.81f, 0.0f, 1.197f, 13.58f}}},  // 256 x 256
+    {27, {{2.18f, 0.439f, 1.51f, 8.421f}, {2.032f, 1.354f, 1.419f, 9.658f}, {5.463f, 0.352f, 1.482f, 10.243f}, {-4.66f, 0.0f, 1.369f, 16.58f}}},  // 288 x 256
+    {28, {{1.899f, 0.478f, 0.801f, 4.431f}, {1.97f, 0.725f, 0.848f, 8.612f}, {2.365f, 0.613f, 0.746f, 7.688f}, {-0.57f, 0.0f, 0.702f, 9.04f}}},  // 256 x 128
+    {29, {{1.5f, 0.167f, 0.497f, 3.339f}, {1.699f, 0.528f, 0.61f, 6.397f}, {1.5f, 0.67f, 0.415f, 5.085f}, {1.31f, 0.0f, 0.467f, 4.25f}}},  // 144 x 96
 };
 
 // the K / splits a tile can run (as gemm_launch_cfg checks it)
@@ -1201,10 +1203,11 @@ bool tile_takes_k(const TileCfg& t, int64_t kslice) {
 int cheapest_tile(int64_t M, int64_t N, int64_t K, int splits, int kind, float* us) {
   int best = 2;
   float best_us = kNever;
-  for (const TileCost& c : kCosts) {
+  const int cls = kind == OASIS_EPI_PARTIAL_F32 && K / splits >= 512 ? COST_PART : cost_class(kind);
+  for (const TileCost<4>& c : kCosts) {
     const TileCfg& t = kTiles[c.tile];
     if (!tile_takes_k(t, K / splits) || (t.no_fp8_epi && kind == OASIS_EPI_GELU_TANH_FP8)) continue;
-    const float cost = tile_cost(c, t.bm, t.bn, M, N, K / splits / 64, splits, kind);
+    const float cost = tile_cost(c, t.bm, t.bn, M, N, K / splits / 64, splits, cls);
     if (cost < best_us) {
       best_us = cost;
       best = c.tile;
@@ -1374,6 +1377,15 @@ extern "C" int oasis_gemm_bf16_config(const void* A, int64_t lda, const void* B,
   OASIS_REQUIRE(epi, OASIS_ERR_NULL, "gemm: null epilogue");
   return oasis::gemm_launch_cfg(static_cast<const bf16*>(A), lda, static_cast<const bf16*>(B), ldb, M, N, K,
                                 *epi, tile, splits, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int oasis_gemm_tile(int64_t M, int64_t N, int64_t K, int kind, int splits, int fp8) {
+  const int gran = fp8 ? 128 : BK;
+  OASIS_REQUIRE(M > 0 && N > 0 && K > 0 && K % gran == 0 && splits >= 1 && (K / gran) % splits == 0, OASIS_ERR_SHAPE,
+                "gemm_tile: bad shape M=%lld N=%lld K=%lld splits=%d", (long long)M, (long long)N, (long long)K, splits);
+  OASIS_REQUIRE(kind >= OASIS_EPI_STORE_F32 && kind <= OASIS_EPI_GELU_TANH_FRAG, OASIS_ERR_ARG,
+                "gemm_tile: epilogue kind %d does not run on a tile table", kind);
+  return fp8 ? oasis::gemm_fp8_auto_tile(M, N, K, splits, kind) : oasis::auto_tile(M, N, K, splits, kind);
 }
 
 extern "C" int oasis_gemm_bf16(const void* A, int64_t lda, const void* B, int64_t ldb, int64_t M,

@@ -87,30 +87,36 @@ __device__ __forceinline__ void grouped_tile(int pid, int Mt, int Nt, int GN, in
 
 // Tile choice by measured cost. A launch of `tiles` workgroups puts W = ceil(tiles / 256) of them on
 // the busiest CU, one after another or side by side, and takes about
-//     c + W * (a * nk + b)  microseconds,  nk = K tiles of a workgroup's K slice,
-// with c, a and b of a tile and an epilogue class fitted (least squares of the relative error) to
-// hipGraphs of 32 launches over cold weights at 24 row counts from 432 to 9216 (fp8: from 144) and the
-// DiT's four projections. It is what the width alone could not say: 1440 x 4096 in 144 x 64 tiles is
-// 640 workgroups, three rounds of 256 of which the last is half empty (29.8 us), in 192 x 128 tiles
-// 256 workgroups (19.0 us). Over those shapes the tile it picks takes 1.02 times the fastest of all
-// tiles (mean; 1.2 at worst).
-enum { COST_STORE = 0, COST_QKV = 1, COST_RES = 2 };  // plain and GELU stores; QKV + RoPE; fp32 residual / partials
+//     c + max(lat * nk, W * (a * nk + b))  microseconds,  nk = K tiles of a workgroup's K slice,
+// lat the time of a K tile of a workgroup that has its CU to itself. c, lat, a and b of a tile and an
+// epilogue class are fitted to hipGraphs of 16 launches over cold weights at 14 row counts from 321 to
+// 9216 (fp8: 20 from 1), N = 64 to 4096 and K = 64 (fp8: 128) to 4096: a least-squares start, then a
+// descent on the time of the picked tile over that of the fastest. It is what the width alone could not
+// say: 1440 x 4096 in 144 x 64 tiles is 640 workgroups, three rounds of 256 of which the last is half
+// empty (29.8 us), in 192 x 128 tiles 256 workgroups (19.0 us). Over those 1848 (fp8: 2044) shapes the
+// tile it picks takes 1.018 (fp8: 1.007) times the fastest of all tiles in the mean, 1.31 (1.17) at
+// worst, where K = 4096; fitted at K = 1024 alone it took up to 3.2 (2.9) times at K = 64 (128).
+enum { COST_STORE = 0, COST_QKV = 1, COST_RES = 2, COST_PART = 3 };
+template <int CLASSES>
 struct TileCost {
   int tile;
   struct {
-    float c, a, b;
-  } k[3];
+    float c, lat, a, b;
+  } k[CLASSES];
 };
 constexpr float kNever = 1e9f;  // class not run on this tile
+// plain and GELU stores; QKV + RoPE; fp32 residuals and partial sums
 inline int cost_class(int kind) {
   if (kind == OASIS_EPI_QKV_ROPE) return COST_QKV;
   return kind == OASIS_EPI_PARTIAL_F32 || kind == OASIS_EPI_GATED_RES || kind == OASIS_EPI_RESIDUAL ? COST_RES : COST_STORE;
 }
 // microseconds of an M x N product in bm x bn tiles and nk K tiles per workgroup
-inline float tile_cost(const TileCost& t, int bm, int bn, int64_t M, int64_t N, int64_t nk, int splits, int kind) {
-  const auto& k = t.k[cost_class(kind)];
+template <int CLASSES>
+inline float tile_cost(const TileCost<CLASSES>& t, int bm, int bn, int64_t M, int64_t N, int64_t nk, int splits, int cls) {
+  const auto& k = t.k[cls];
   const int64_t tiles = (M + bm - 1) / bm * ((N + bn - 1) / bn) * splits;
-  return k.c + (float)((tiles + 255) / 256) * (k.a * (float)nk + k.b);
+  const float lone = k.lat * (float)nk, busy = (float)((tiles + 255) / 256) * (k.a * (float)nk + k.b);
+  return k.c + (lone > busy ? lone : busy);
 }
 // What a split-K product's slices cost the residual_ln that adds them: its reads of M x N fp32
 // slices against a residual added in the GEMM's epilogue (measured at 288 to 4608 rows, N = 1024).

@@ -526,7 +526,7 @@ const Tile8 kTiles8[] = {
     OASIS_T8_BIG(288, 64, 2, 4, 1, 2),     // 9
     OASIS_T8_BIG(144, 128, 3, 2, 0, 3),    // 10 (three stages)
     OASIS_T8_BIG(144, 128, 3, 2, 0, 4),    // 11 (four stages)
-    // with 5, 10 and 4 what kCosts8 picks from (fp8 A): 32 x 32 to 96 x 64 wave tiles on 4 to 16 waves
+    // with 0, 2 to 5 and 10 what kCosts8 picks from (fp8 A): 32 x 32 to 96 x 64 wave tiles on 4 to 16 waves
     OASIS_T8_BIG(64, 64, 2, 2, 0, 4),      // 12
     OASIS_T8_BIG(96, 64, 2, 2, 0, 3),      // 13
     OASIS_T8_BIG(96, 128, 2, 4, 0, 3),     // 14
@@ -544,33 +544,36 @@ const Tile8 kTiles8[] = {
 #undef OASIS_T8_BIG
 constexpr int kNumTiles8 = sizeof(kTiles8) / sizeof(kTiles8[0]);
 
-// Fitted costs (tile_cost, 128-wide K tiles) of the tiles for fp8 A: c, a and b for the plain and
+// Fitted costs (tile_cost, 128-wide K tiles) of the tiles for fp8 A: c, lat, a and b for the plain and
 // GELU stores, QKV + RoPE, and the fp32 residual and partial-sum epilogues.
-const TileCost kCosts8[] = {
-    {4, {{2.96f, 0.254f, 0.00f}, {4.03f, 0.224f, 0.00f}, {3.33f, 0.212f, 0.36f}}},  // 32 x 64
-    {5, {{0.04f, 3.364f, 0.00f}, {0.22f, 3.304f, 0.00f}, {-5.24f, 1.520f, 15.95f}}},  // 288 x 256
-    {10, {{1.81f, 1.299f, 0.00f}, {2.19f, 1.551f, 0.00f}, {0.33f, 0.719f, 5.47f}}},  // 144 x 128
-    {12, {{3.15f, 0.405f, 0.00f}, {3.61f, 0.419f, 0.00f}, {2.63f, 0.365f, 1.09f}}},  // 64 x 64
-    {13, {{4.28f, 0.414f, 0.00f}, {4.56f, 0.437f, 0.00f}, {3.44f, 0.409f, 1.09f}}},  // 96 x 64
-    {14, {{1.50f, 0.960f, 0.00f}, {1.70f, 0.971f, 0.00f}, {0.37f, 0.698f, 3.96f}}},  // 96 x 128
-    {15, {{0.82f, 1.270f, 0.00f}, {1.05f, 1.412f, 0.00f}, {-0.94f, 0.821f, 6.04f}}},  // 144 x 128
-    {16, {{1.87f, 0.881f, 0.00f}, {1.92f, 0.886f, 0.00f}, {0.78f, 0.578f, 3.62f}}},  // 144 x 64
-    {17, {{1.21f, 1.412f, 0.00f}, {1.13f, 1.630f, 0.00f}, {-0.86f, 0.786f, 6.93f}}},  // 192 x 128
-    {18, {{0.61f, 1.918f, 0.00f}, {-0.26f, 1.928f, 0.00f}, {-1.76f, 1.109f, 8.54f}}},  // 192 x 192
-    {19, {{3.06f, 0.598f, 0.00f}, {3.08f, 0.622f, 0.00f}, {kNever, 0.0f, 0.0f}}},  // 64 x 128
-    {20, {{0.63f, 1.949f, 0.00f}, {-0.03f, 2.121f, 0.00f}, {-2.70f, 1.183f, 9.80f}}},  // 144 x 256
-    {21, {{-1.13f, 2.549f, 0.00f}, {-0.65f, 2.346f, 0.00f}, {-3.86f, 1.419f, 11.80f}}},  // 192 x 256
-    {22, {{kNever, 0.0f, 0.0f}, {-0.31f, 3.001f, 0.00f}, {-2.06f, 1.362f, 11.77f}}},  // 288 x 192
-    {23, {{1.01f, 1.758f, 0.00f}, {0.44f, 1.971f, 0.00f}, {-1.64f, 0.870f, 8.72f}}},  // 256 x 128
+const TileCost<3> kCosts8[] = {
+    {0, {{5.138f, 0.875f, 0.884f, 2.769f}, {2.308f, 0.908f, 0.69f, 7.947f}, {kNever, 0, 0, 0}}},  // 128 x 128
+    {2, {{5.413f, 0.135f, 0.37f, 1.596f}, {4.748f, 0.752f, 0.319f, 3.142f}, {kNever, 0, 0, 0}}},  // 64 x 128
+    {3, {{3.496f, 0.394f, 0.285f, 0.475f}, {3.62f, 0.487f, 0.343f, 0.436f}, {kNever, 0, 0, 0}}},  // 64 x 64
+    {4, {{2.904f, 0.14f, 0.204f, 0.215f}, {2.945f, 0.362f, 0.219f, 0.244f}, {3.33f, 0.0f, 0.212f, 0.36f}}},  // 32 x 64
+    {5, {{1.5f, 1.455f, 1.507f, 10.538f}, {2.537f, 2.09f, 1.783f, 12.188f}, {-5.24f, 0.0f, 1.52f, 15.95f}}},  // 288 x 256
+    {10, {{1.5f, 0.634f, 0.696f, 4.631f}, {3.041f, 1.246f, 0.751f, 6.223f}, {0.33f, 0.0f, 0.719f, 5.47f}}},  // 144 x 128
+    {12, {{2.784f, 0.416f, 0.335f, 1.13f}, {4.55f, 0.419f, 0.234f, 0.854f}, {2.63f, 0.0f, 0.365f, 1.09f}}},  // 64 x 64
+    {13, {{3.665f, 0.405f, 0.402f, 1.51f}, {3.495f, 0.848f, 0.364f, 1.543f}, {3.44f, 0.0f, 0.409f, 1.09f}}},  // 96 x 64
+    {14, {{1.642f, 0.633f, 0.676f, 2.935f}, {1.5f, 0.502f, 0.694f, 3.173f}, {0.37f, 0.0f, 0.698f, 3.96f}}},  // 96 x 128
+    {15, {{1.5f, 0.385f, 0.758f, 3.518f}, {2.652f, 0.152f, 0.684f, 5.673f}, {-0.94f, 0.0f, 0.821f, 6.04f}}},  // 144 x 128
+    {16, {{1.649f, 0.254f, 0.466f, 3.172f}, {1.519f, 0.607f, 0.608f, 3.097f}, {0.78f, 0.0f, 0.578f, 3.62f}}},  // 144 x 64
+    {17, {{1.5f, 0.258f, 0.83f, 4.92f}, {4.223f, 0.231f, 0.947f, 3.597f}, {-0.86f, 0.0f, 0.786f, 6.93f}}},  // 192 x 128
+    {18, {{1.741f, 0.821f, 1.079f, 5.008f}, {1.5f, 1.628f, 1.118f, 5.436f}, {-1.76f, 0.0f, 1.109f, 8.54f}}},  // 192 x 192
+    {19, {{2.943f, 0.301f, 0.476f, 1.5f}, {3.576f, 0.17f, 0.48f, 1.0f}, {kNever, 0, 0, 0}}},  // 64 x 128
+    {20, {{1.516f, 1.613f, 1.142f, 5.466f}, {1.5f, 2.058f, 1.095f, 6.065f}, {-2.7f, 0.0f, 1.183f, 9.8f}}},  // 144 x 256
+    {21, {{1.507f, 1.948f, 1.394f, 5.467f}, {4.432f, 1.603f, 1.527f, 3.674f}, {-3.86f, 0.0f, 1.419f, 11.8f}}},  // 192 x 256
+    {22, {{2.158f, 1.981f, 1.291f, 9.226f}, {2.403f, 0.268f, 1.342f, 11.432f}, {-2.06f, 0.0f, 1.362f, 11.77f}}},  // 288 x 192
+    {23, {{1.652f, 0.481f, 0.827f, 5.867f}, {3.725f, 1.373f, 0.588f, 8.479f}, {-1.64f, 0.0f, 0.87f, 8.72f}}},  // 256 x 128
 };
 
 int cheapest_tile8(int64_t M, int64_t N, int64_t K, int splits, int kind, float* us) {
   int best = 4;
   float best_us = kNever;
-  for (const TileCost& c : kCosts8) {
+  for (const TileCost<3>& c : kCosts8) {
     const Tile8& t = kTiles8[c.tile];
     if (t.no_fp8_epi && kind == OASIS_EPI_GELU_TANH_FP8) continue;
-    const float cost = tile_cost(c, t.bm, t.bn, M, N, K / splits / BK8, splits, kind);
+    const float cost = tile_cost(c, t.bm, t.bn, M, N, K / splits / BK8, splits, cost_class(kind));
     if (cost < best_us) {
       best_us = cost;
       best = c.tile;
@@ -637,6 +640,10 @@ __global__ __launch_bounds__(256) void quant_act_kernel(const bf16* __restrict__
 }  // namespace
 
 namespace oasis {
+
+int gemm_fp8_auto_tile(int64_t M, int64_t N, int64_t K, int splits, int kind) {
+  return auto_tile8(M, N, K, splits, true, kind);
+}
 
 int gemm_fp8_auto_splits(int64_t M, int64_t N, int64_t K, int max_splits) {
   int best = 1;

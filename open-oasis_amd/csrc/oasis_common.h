@@ -65,6 +65,8 @@ int gemm_launch_cfg(const __bf16* A, int64_t lda, const __bf16* B, int64_t ldb, 
 // the residual in its epilogue); the same with e4m3 weights and fp8 A, at any M
 int gemm_auto_splits(int64_t M, int64_t N, int64_t K, int max_splits);
 int gemm_fp8_auto_splits(int64_t M, int64_t N, int64_t K, int max_splits);
+// the default tile of gemm_fp8_launch with fp8 A
+int gemm_fp8_auto_tile(int64_t M, int64_t N, int64_t K, int splits, int kind);
 // acc = A[M,K] @ (Bq[N,K] (e4m3) * w_scale[N])^T with the given epilogue (gemm_fp8.hip).
 // A_scale == nullptr: A is bf16; else A is e4m3 blocks with e8m0 scales A_scale[M, lds].
 int gemm_fp8_launch(const void* A, int64_t lda, const uint8_t* A_scale, int64_t lds, const uint8_t* B, int64_t ldb,
