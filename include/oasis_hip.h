@@ -95,6 +95,11 @@ int oasis_layernorm(const void* x, const void* weight, const void* bias, int64_t
 int oasis_linear(const void* x, const void* w, void* out, int64_t M, int64_t K, int64_t N,
                  int w_layout, int out_dtype, oasis_stream_t stream);
 
+/* The kernel that oasis_linear runs for [K,N] weights: its place in linear.hip's kLinear table, or past its end
+ * for rows beyond 32-bit byte offsets; a negative error code for shapes it refuses. Host only.
+ * No counterpart in the reference (a tuning query, for tests). */
+int oasis_linear_tile(int64_t M, int64_t K, int64_t N);
+
 /* out[r, :] = silu_cond[0, :] @ w[K,N] + b[N] for r in [0, out_rows) (row expansion).
  * All fp32 except w (bf16).
  * Replaces make_adaln_matmul_expand_kernel(k_tiles, n_repeat)(silu_cond, adaln_w,

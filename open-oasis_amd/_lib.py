@@ -109,6 +109,7 @@ SIGNATURES = {
     "oasis_bias_gated_residual": [c_p, c_p, c_p, c_p, c_p, c_i64, c_i, c_p],
     "oasis_layernorm": [c_p, c_p, c_p, c_i64, c_p, c_i64, c_i64, c_f, c_i, c_p],
     "oasis_linear": [c_p, c_p, c_p, c_i64, c_i64, c_i64, c_i, c_i, c_p],
+    "oasis_linear_tile": [c_i64, c_i64, c_i64],
     "oasis_adaln_matmul_expand": [c_p, c_p, c_p, c_p, c_i64, c_i64, c_i64, c_p],
     "oasis_rope_layout": [c_p, c_i64, c_p, c_p, c_i64, c_i64, c_i64, c_i64, c_p, c_p, c_p,
                           c_i64, c_i64, c_i64, c_i64, c_i, c_i, c_p],

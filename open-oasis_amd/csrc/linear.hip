@@ -349,7 +349,17 @@ const LinearTile& linear_tile(int64_t M, int64_t N, int64_t K) {
   return *best;
 }
 
+// a K tile's 64 rows, or a tile's rows of x, beyond 32-bit byte offsets (2^32 / 2 / 192 rows)
+bool linear_wide(int64_t K, int64_t N) { return N >= (1ll << 24) || K >= (1ll << 23); }
+
 }  // namespace
+
+extern "C" int oasis_linear_tile(int64_t M, int64_t K, int64_t N) {
+  OASIS_REQUIRE(M > 0 && N > 0 && K > 0 && K % 64 == 0 && N % 8 == 0 && M < (1ll << 31) && N < (1ll << 31),
+                OASIS_ERR_SHAPE, "linear_tile: need K %% 64 == 0 and N %% 8 == 0");
+  if (linear_wide(K, N)) return (int)(sizeof(kLinear) / sizeof(kLinear[0]));
+  return (int)(&linear_tile(M, N, K) - kLinear);
+}
 
 extern "C" int oasis_linear(const void* x, const void* w, void* out, int64_t M, int64_t K, int64_t N,
                             int w_layout, int out_dtype, oasis_stream_t stream) {
@@ -370,8 +380,7 @@ extern "C" int oasis_linear(const void* x, const void* w, void* out, int64_t M, 
     ex.ld_out = N;
     return oasis::gemm_launch(static_cast<const bf16*>(x), K, static_cast<const bf16*>(w), K, M, N, K, ex, s);
   }
-  // a K tile's 64 rows, or a tile's rows of x, beyond 32-bit byte offsets (2^32 / 2 / 192 rows)
-  if (N >= (1ll << 24) || K >= (1ll << 23)) {
+  if (linear_wide(K, N)) {
     launch_linear<64, 64, 2, 2, 4, true>(static_cast<const bf16*>(x), K, static_cast<const bf16*>(w), N, (int)M, (int)N,
                                          (int)K, out, out_dtype == OASIS_F32, s);
     return oasis::check_launch("linear");

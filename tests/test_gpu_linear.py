@@ -16,12 +16,16 @@ def _linear(x, w, dtype):
     return out
 
 
-# one wave-split tile height after the other, then the ring tiles; partial last tiles on both sides, N below a
-# tile and below a 16-column group, K of one ring stage, of fewer K tiles than the ring and of odd counts
-@pytest.mark.parametrize("M,K,N", [(1, 256, 8), (17, 1024, 1000), (64, 4096, 72), (300, 1024, 1000), (150, 512, 3048),
-                                   (630, 1024, 1016), (321, 1024, 3064), (1, 64, 8), (5, 64, 64), (500, 320, 3064),
-                                   (70, 128, 200), (640, 1024, 4088), (1290, 1024, 3064), (1281, 192, 3064),
-                                   (2561, 1024, 4088), (2500, 64, 4072), (577, 832, 1208)])
+# every kernel of the table (the shapes' kernels are checked without a GPU beside the other tile choices); partial
+# last tiles on both sides, N below a tile and below a 16-column group, K of one ring stage, of fewer K tiles than
+# the ring and of odd counts
+SHAPES = [(1, 256, 8), (17, 1024, 1000), (64, 4096, 72), (300, 1024, 1000), (150, 512, 3048), (250, 1024, 3064),
+          (243, 4096, 3048), (630, 1024, 1016), (321, 1024, 3064), (1, 64, 8), (5, 64, 64), (500, 320, 3064),
+          (70, 128, 200), (640, 1024, 4088), (1030, 1024, 3064), (1057, 960, 3048), (1290, 1024, 3064),
+          (1281, 192, 3064), (2561, 1024, 4088), (2500, 64, 4072), (577, 832, 1208), (643, 1024, 3064)]
+
+
+@pytest.mark.parametrize("M,K,N", SHAPES)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_linear_kn_tiles(M, K, N, dtype):
     g = torch.Generator().manual_seed(M + N)

@@ -3,6 +3,7 @@ that the DiT runs, the tile picked is among those measured within 12 % of the fa
 import pytest
 
 from helpers import L
+from test_gpu_linear import SHAPES as LINEAR_SHAPES
 
 # (epilogue, M, N, K, tiles within 12 % of the fastest), MI355X, weights not in cache
 BF16 = [
@@ -35,3 +36,13 @@ def test_default_tile_is_among_the_fastest(fp8, kind, M, N, K, good):
                                        ((64, 64, 128, 12, 1, 0), -5), ((64, 64, 128, -1, 1, 0), -5)])
 def test_tile_query_errors(args, code):
     assert L.lib().oasis_gemm_tile(*args) == code
+
+
+def test_linear_shapes_reach_every_kernel():
+    """The [K, N] linear layer's GPU test runs each kernel of its table, on at least one shape with partial last
+    tiles of rows and of columns."""
+    tile = L.lib().oasis_linear_tile
+    assert {tile(*s) for s in LINEAR_SHAPES} == set(range(8))
+    assert {tile(M, K, N) for M, K, N in LINEAR_SHAPES if M % 16 and N % 64} == set(range(8))
+    assert tile(3, 64, (1 << 24) + 8) == tile(3, 1 << 23, 64) == 8
+    assert tile(0, 64, 64) == tile(1, 96, 64) == tile(1, 64, 60) == -2
