@@ -1171,26 +1171,26 @@ constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 // stores, QKV + RoPE, the fp32 residual, and split-K slices of 512 and longer (with which split counts
 // are chosen: fitted to the DiT's O and FC2 products; shorter slices cost as residuals).
 const TileCost<4> kCosts[] = {
-    {1, {{2.498f, 0.29f, 0.146f, 0.359f}, {2.861f, 0.196f, 0.131f, 0.519f}, {2.739f, 0.295f, 0.143f, 0.758f}, {kNever, 0, 0, 0}}},  // 32 x 64
-    {2, {{3.144f, 0.289f, 0.221f, 1.341f}, {3.801f, 0.247f, 0.233f, 1.393f}, {2.357f, 0.327f, 0.243f, 1.835f}, {3.71f, 0.0f, 0.235f, 1.04f}}},  // 96 x 64
-    {3, {{2.788f, 0.281f, 0.177f, 0.919f}, {3.13f, 0.574f, 0.179f, 1.07f}, {3.073f, 0.283f, 0.145f, 1.087f}, {3.45f, 0.0f, 0.181f, 0.79f}}},  // 64 x 64
-    {4, {{1.588f, 0.365f, 0.433f, 2.857f}, {1.924f, 0.823f, 0.451f, 6.63f}, {2.42f, 0.087f, 0.333f, 3.211f}, {1.48f, 0.0f, 0.375f, 3.43f}}},  // 144 x 64
-    {9, {{1.79f, 0.07f, 0.108f, 0.763f}, {3.51f, 0.368f, 0.07f, 0.92f}, {1.782f, 0.153f, 0.095f, 0.892f}, {1.26f, 0.0f, 0.09f, 1.12f}}},  // 48 x 32
-    {10, {{1.5f, 0.009f, 0.136f, 2.527f}, {2.694f, 0.591f, 0.082f, 3.536f}, {1.943f, 0.036f, 0.08f, 4.271f}, {1.48f, 0.0f, 0.147f, 2.28f}}},  // 48 x 64
-    {11, {{1.5f, 0.244f, 0.158f, 2.355f}, {1.854f, 0.202f, 0.133f, 3.704f}, {1.888f, 0.242f, 0.142f, 2.944f}, {1.47f, 0.0f, 0.172f, 2.71f}}},  // 64 x 64
-    {12, {{1.819f, 0.12f, 0.099f, 1.441f}, {3.391f, 0.188f, 0.126f, 1.767f}, {1.688f, 0.011f, 0.154f, 1.716f}, {1.45f, 0.0f, 0.113f, 1.86f}}},  // 32 x 64
-    {18, {{1.5f, 0.422f, 0.597f, 3.811f}, {2.933f, 0.191f, 0.581f, 3.193f}, {1.5f, 0.557f, 0.558f, 5.961f}, {0.79f, 0.0f, 0.528f, 5.23f}}},  // 144 x 128
-    {19, {{3.741f, 0.83f, 0.551f, 2.403f}, {4.851f, 1.1f, 0.57f, 2.678f}, {2.474f, 0.871f, 0.568f, 6.12f}, {3.35f, 0.0f, 0.684f, 3.14f}}},  // 192 x 128
-    {20, {{1.631f, 0.346f, 0.625f, 4.644f}, {2.921f, 0.192f, 0.68f, 6.32f}, {2.926f, 0.539f, 0.626f, 5.845f}, {0.74f, 0.0f, 0.626f, 6.26f}}},  // 192 x 128
-    {21, {{1.5f, 0.809f, 0.847f, 6.038f}, {8.498f, 0.345f, 1.113f, 2.543f}, {5.977f, 0.098f, 0.801f, 5.207f}, {-0.86f, 0.0f, 0.838f, 9.16f}}},  // 144 x 256
-    {22, {{1.656f, 1.03f, 0.843f, 5.323f}, {2.705f, 0.291f, 1.051f, 3.816f}, {7.087f, 0.657f, 0.935f, 4.547f}, {-0.25f, 0.0f, 0.866f, 7.63f}}},  // 192 x 192
-    {23, {{1.524f, 0.487f, 0.444f, 3.192f}, {5.548f, 0.433f, 0.422f, 2.181f}, {1.956f, 0.406f, 0.385f, 4.377f}, {1.61f, 0.0f, 0.429f, 3.57f}}},  // 96 x 128
-    {24, {{3.319f, 0.861f, 0.48f, 1.492f}, {4.583f, 0.755f, 0.401f, 0.861f}, {2.414f, 0.762f, 0.456f, 3.735f}, {5.18f, 0.0f, 0.459f, 0.89f}}},  // 96 x 128
-    {25, {{2.413f, 0.187f, 0.539f, 2.632f}, {6.803f, 0.256f, 0.71f, 1.42f}, {1.5f, 0.072f, 0.459f, 5.717f}, {1.14f, 0.0f, 0.49f, 4.6f}}},  // 128 x 128
-    {26, {{1.55f, 1.584f, 1.229f, 7.698f}, {1.915f, 1.107f, 1.327f, 8.819f}, {1.5f, 0.467f, 1.336f, 20.787f}, {-2.81f, 0.0f, 1.197f, 13.58f}}},  // 256 x 256
-    {27, {{2.18f, 0.439f, 1.51f, 8.421f}, {2.032f, 1.354f, 1.419f, 9.658f}, {5.463f, 0.352f, 1.482f, 10.243f}, {-4.66f, 0.0f, 1.369f, 16.58f}}},  // 288 x 256
-    {28, {{1.899f, 0.478f, 0.801f, 4.431f}, {1.97f, 0.725f, 0.848f, 8.612f}, {2.365f, 0.613f, 0.746f, 7.688f}, {-0.57f, 0.0f, 0.702f, 9.04f}}},  // 256 x 128
-    {29, {{1.5f, 0.167f, 0.497f, 3.339f}, {1.699f, 0.528f, 0.61f, 6.397f}, {1.5f, 0.67f, 0.415f, 5.085f}, {1.31f, 0.0f, 0.467f, 4.25f}}},  // 144 x 96
+    {1, {{2.504f, 0.29f, 0.145f, 0.359f}, {2.412f, 0.218f, 0.145f, 0.493f}, {2.765f, 0.289f, 0.154f, 0.694f}, {kNever, 0, 0, 0}}},  // 32 x 64
+    {2, {{3.152f, 0.287f, 0.226f, 1.353f}, {3.662f, 0.378f, 0.241f, 1.172f}, {2.64f, 0.304f, 0.219f, 1.952f}, {3.71f, 0.0f, 0.235f, 1.04f}}},  // 96 x 64
+    {3, {{2.772f, 0.282f, 0.179f, 0.919f}, {3.031f, 0.549f, 0.181f, 1.043f}, {3.123f, 0.275f, 0.172f, 1.036f}, {3.45f, 0.0f, 0.181f, 0.79f}}},  // 64 x 64
+    {4, {{1.749f, 0.425f, 0.443f, 2.687f}, {3.641f, 0.574f, 0.328f, 5.242f}, {2.076f, 0.223f, 0.356f, 3.334f}, {1.48f, 0.0f, 0.375f, 3.43f}}},  // 144 x 64
+    {9, {{1.919f, 0.064f, 0.091f, 0.8f}, {2.629f, 0.445f, 0.058f, 0.992f}, {2.447f, 0.054f, 0.096f, 0.686f}, {1.26f, 0.0f, 0.09f, 1.12f}}},  // 48 x 32
+    {10, {{1.5f, 0.21f, 0.08f, 3.342f}, {1.813f, 0.067f, 0.094f, 3.399f}, {1.5f, 0.21f, 0.15f, 2.985f}, {1.48f, 0.0f, 0.147f, 2.28f}}},  // 48 x 64
+    {11, {{1.5f, 0.036f, 0.16f, 2.339f}, {3.168f, 0.573f, 0.106f, 3.004f}, {1.668f, 0.302f, 0.125f, 3.622f}, {1.47f, 0.0f, 0.172f, 2.71f}}},  // 64 x 64
+    {12, {{1.556f, 0.058f, 0.089f, 1.749f}, {1.813f, 0.027f, 0.05f, 2.823f}, {1.952f, 0.196f, 0.133f, 1.509f}, {1.45f, 0.0f, 0.113f, 1.86f}}},  // 32 x 64
+    {18, {{2.122f, 0.152f, 0.609f, 3.053f}, {1.5f, 0.255f, 0.537f, 4.321f}, {1.89f, 0.26f, 0.653f, 5.017f}, {0.79f, 0.0f, 0.528f, 5.23f}}},  // 144 x 128
+    {19, {{3.867f, 0.84f, 0.59f, 2.345f}, {4.914f, 1.145f, 0.549f, 3.759f}, {1.5f, 0.542f, 0.751f, 5.884f}, {3.35f, 0.0f, 0.684f, 3.14f}}},  // 192 x 128
+    {20, {{1.657f, 0.065f, 0.633f, 4.694f}, {1.5f, 0.651f, 0.717f, 9.372f}, {1.72f, 0.163f, 0.67f, 6.956f}, {0.74f, 0.0f, 0.626f, 6.26f}}},  // 192 x 128
+    {21, {{1.5f, 0.259f, 0.93f, 5.683f}, {8.243f, 0.13f, 1.233f, 0.627f}, {5.071f, 0.294f, 0.904f, 5.261f}, {-0.86f, 0.0f, 0.838f, 9.16f}}},  // 144 x 256
+    {22, {{1.57f, 0.146f, 0.938f, 5.12f}, {3.154f, 0.74f, 1.094f, 3.435f}, {4.166f, 0.961f, 1.088f, 5.718f}, {-0.25f, 0.0f, 0.866f, 7.63f}}},  // 192 x 192
+    {23, {{1.727f, 0.429f, 0.454f, 2.995f}, {2.153f, 0.586f, 0.458f, 4.664f}, {1.5f, 0.505f, 0.33f, 4.663f}, {1.61f, 0.0f, 0.429f, 3.57f}}},  // 96 x 128
+    {24, {{3.129f, 0.866f, 0.472f, 1.725f}, {4.713f, 0.676f, 0.451f, 1.0f}, {2.004f, 0.671f, 0.517f, 3.636f}, {5.18f, 0.0f, 0.459f, 0.89f}}},  // 96 x 128
+    {25, {{2.183f, 0.052f, 0.585f, 2.819f}, {2.934f, 0.253f, 0.522f, 4.9f}, {1.5f, 0.054f, 0.529f, 4.747f}, {1.14f, 0.0f, 0.49f, 4.6f}}},  // 128 x 128
+    {26, {{2.203f, 0.618f, 1.199f, 7.655f}, {4.581f, 0.271f, 1.422f, 6.115f}, {5.864f, 0.314f, 0.983f, 22.77f}, {-2.81f, 0.0f, 1.197f, 13.58f}}},  // 256 x 256
+    {27, {{2.153f, 1.067f, 1.642f, 8.275f}, {8.992f, 0.38f, 1.672f, 2.623f}, {2.062f, 0.101f, 1.327f, 9.789f}, {-4.66f, 0.0f, 1.369f, 16.58f}}},  // 288 x 256
+    {28, {{1.721f, 0.58f, 0.87f, 4.712f}, {1.938f, 0.55f, 0.891f, 8.982f}, {4.356f, 0.44f, 0.718f, 5.532f}, {-0.57f, 0.0f, 0.702f, 9.04f}}},  // 256 x 128
+    {29, {{1.5f, 0.295f, 0.472f, 3.381f}, {4.784f, 0.466f, 0.587f, 3.758f}, {1.616f, 0.167f, 0.498f, 5.141f}, {1.31f, 0.0f, 0.467f, 4.25f}}},  // 144 x 96
 };
 
 // the K / splits a tile can run (as gemm_launch_cfg checks it)

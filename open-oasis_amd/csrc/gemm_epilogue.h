@@ -90,11 +90,12 @@ __device__ __forceinline__ void grouped_tile(int pid, int Mt, int Nt, int GN, in
 //     c + max(lat * nk, W * (a * nk + b))  microseconds,  nk = K tiles of a workgroup's K slice,
 // lat the time of a K tile of a workgroup that has its CU to itself. c, lat, a and b of a tile and an
 // epilogue class are fitted to hipGraphs of 16 launches over cold weights at 14 row counts from 321 to
-// 9216 (fp8: 20 from 1), N = 64 to 4096 and K = 64 (fp8: 128) to 4096: a least-squares start, then a
-// descent on the time of the picked tile over that of the fastest. It is what the width alone could not
+// 9216 (fp8: 20 from 1), N = 64 to 4096 and K = 64 (fp8: 128) to 4096, and at every whole number of frames
+// of the DiT's products up to 64: a least-squares start, then a descent on the time of the picked tile
+// over that of the fastest. It is what the width alone could not
 // say: 1440 x 4096 in 144 x 64 tiles is 640 workgroups, three rounds of 256 of which the last is half
-// empty (29.8 us), in 192 x 128 tiles 256 workgroups (19.0 us). Over those 1848 (fp8: 2044) shapes the
-// tile it picks takes 1.018 (fp8: 1.007) times the fastest of all tiles in the mean, 1.31 (1.17) at
+// empty (29.8 us), in 192 x 128 tiles 256 workgroups (19.0 us). Over 2048 (fp8: 2244) such shapes the
+// tile it picks takes 1.017 (fp8: 1.007) times the fastest of all tiles in the mean, 1.31 (1.18) at
 // worst, where K = 4096; fitted at K = 1024 alone it took up to 3.2 (2.9) times at K = 64 (128).
 enum { COST_STORE = 0, COST_QKV = 1, COST_RES = 2, COST_PART = 3 };
 template <int CLASSES>

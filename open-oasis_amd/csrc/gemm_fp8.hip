@@ -547,24 +547,24 @@ constexpr int kNumTiles8 = sizeof(kTiles8) / sizeof(kTiles8[0]);
 // Fitted costs (tile_cost, 128-wide K tiles) of the tiles for fp8 A: c, lat, a and b for the plain and
 // GELU stores, QKV + RoPE, and the fp32 residual and partial-sum epilogues.
 const TileCost<3> kCosts8[] = {
-    {0, {{5.138f, 0.875f, 0.884f, 2.769f}, {2.308f, 0.908f, 0.69f, 7.947f}, {kNever, 0, 0, 0}}},  // 128 x 128
-    {2, {{5.413f, 0.135f, 0.37f, 1.596f}, {4.748f, 0.752f, 0.319f, 3.142f}, {kNever, 0, 0, 0}}},  // 64 x 128
-    {3, {{3.496f, 0.394f, 0.285f, 0.475f}, {3.62f, 0.487f, 0.343f, 0.436f}, {kNever, 0, 0, 0}}},  // 64 x 64
-    {4, {{2.904f, 0.14f, 0.204f, 0.215f}, {2.945f, 0.362f, 0.219f, 0.244f}, {3.33f, 0.0f, 0.212f, 0.36f}}},  // 32 x 64
-    {5, {{1.5f, 1.455f, 1.507f, 10.538f}, {2.537f, 2.09f, 1.783f, 12.188f}, {-5.24f, 0.0f, 1.52f, 15.95f}}},  // 288 x 256
-    {10, {{1.5f, 0.634f, 0.696f, 4.631f}, {3.041f, 1.246f, 0.751f, 6.223f}, {0.33f, 0.0f, 0.719f, 5.47f}}},  // 144 x 128
-    {12, {{2.784f, 0.416f, 0.335f, 1.13f}, {4.55f, 0.419f, 0.234f, 0.854f}, {2.63f, 0.0f, 0.365f, 1.09f}}},  // 64 x 64
-    {13, {{3.665f, 0.405f, 0.402f, 1.51f}, {3.495f, 0.848f, 0.364f, 1.543f}, {3.44f, 0.0f, 0.409f, 1.09f}}},  // 96 x 64
-    {14, {{1.642f, 0.633f, 0.676f, 2.935f}, {1.5f, 0.502f, 0.694f, 3.173f}, {0.37f, 0.0f, 0.698f, 3.96f}}},  // 96 x 128
-    {15, {{1.5f, 0.385f, 0.758f, 3.518f}, {2.652f, 0.152f, 0.684f, 5.673f}, {-0.94f, 0.0f, 0.821f, 6.04f}}},  // 144 x 128
-    {16, {{1.649f, 0.254f, 0.466f, 3.172f}, {1.519f, 0.607f, 0.608f, 3.097f}, {0.78f, 0.0f, 0.578f, 3.62f}}},  // 144 x 64
-    {17, {{1.5f, 0.258f, 0.83f, 4.92f}, {4.223f, 0.231f, 0.947f, 3.597f}, {-0.86f, 0.0f, 0.786f, 6.93f}}},  // 192 x 128
-    {18, {{1.741f, 0.821f, 1.079f, 5.008f}, {1.5f, 1.628f, 1.118f, 5.436f}, {-1.76f, 0.0f, 1.109f, 8.54f}}},  // 192 x 192
-    {19, {{2.943f, 0.301f, 0.476f, 1.5f}, {3.576f, 0.17f, 0.48f, 1.0f}, {kNever, 0, 0, 0}}},  // 64 x 128
-    {20, {{1.516f, 1.613f, 1.142f, 5.466f}, {1.5f, 2.058f, 1.095f, 6.065f}, {-2.7f, 0.0f, 1.183f, 9.8f}}},  // 144 x 256
-    {21, {{1.507f, 1.948f, 1.394f, 5.467f}, {4.432f, 1.603f, 1.527f, 3.674f}, {-3.86f, 0.0f, 1.419f, 11.8f}}},  // 192 x 256
-    {22, {{2.158f, 1.981f, 1.291f, 9.226f}, {2.403f, 0.268f, 1.342f, 11.432f}, {-2.06f, 0.0f, 1.362f, 11.77f}}},  // 288 x 192
-    {23, {{1.652f, 0.481f, 0.827f, 5.867f}, {3.725f, 1.373f, 0.588f, 8.479f}, {-1.64f, 0.0f, 0.87f, 8.72f}}},  // 256 x 128
+    {0, {{5.138f, 0.875f, 0.884f, 2.769f}, {5.363f, 0.864f, 1.094f, 6.275f}, {kNever, 0, 0, 0}}},  // 128 x 128
+    {2, {{5.413f, 0.135f, 0.37f, 1.596f}, {6.008f, 0.487f, 0.477f, 1.483f}, {kNever, 0, 0, 0}}},  // 64 x 128
+    {3, {{3.496f, 0.394f, 0.285f, 0.475f}, {3.167f, 0.737f, 0.205f, 1.08f}, {kNever, 0, 0, 0}}},  // 64 x 64
+    {4, {{2.904f, 0.14f, 0.204f, 0.215f}, {3.102f, 0.455f, 0.209f, 0.255f}, {3.33f, 0.0f, 0.212f, 0.36f}}},  // 32 x 64
+    {5, {{1.5f, 1.455f, 1.507f, 10.538f}, {6.886f, 1.487f, 1.482f, 7.142f}, {-5.24f, 0.0f, 1.52f, 15.95f}}},  // 288 x 256
+    {10, {{1.5f, 0.634f, 0.696f, 4.631f}, {5.032f, 1.323f, 0.731f, 5.684f}, {0.33f, 0.0f, 0.719f, 5.47f}}},  // 144 x 128
+    {12, {{2.784f, 0.416f, 0.335f, 1.13f}, {3.308f, 0.29f, 0.364f, 1.226f}, {2.63f, 0.0f, 0.365f, 1.09f}}},  // 64 x 64
+    {13, {{3.665f, 0.405f, 0.402f, 1.51f}, {5.016f, 0.324f, 0.394f, 0.469f}, {3.44f, 0.0f, 0.409f, 1.09f}}},  // 96 x 64
+    {14, {{1.642f, 0.633f, 0.676f, 2.935f}, {2.626f, 0.364f, 0.618f, 2.389f}, {0.37f, 0.0f, 0.698f, 3.96f}}},  // 96 x 128
+    {15, {{1.5f, 0.385f, 0.758f, 3.518f}, {2.798f, 0.71f, 0.439f, 6.12f}, {-0.94f, 0.0f, 0.821f, 6.04f}}},  // 144 x 128
+    {16, {{1.649f, 0.254f, 0.466f, 3.172f}, {1.813f, 0.885f, 0.521f, 3.108f}, {0.78f, 0.0f, 0.578f, 3.62f}}},  // 144 x 64
+    {17, {{1.5f, 0.258f, 0.83f, 4.92f}, {1.5f, 0.914f, 0.533f, 7.483f}, {-0.86f, 0.0f, 0.786f, 6.93f}}},  // 192 x 128
+    {18, {{1.741f, 0.821f, 1.079f, 5.008f}, {2.813f, 0.527f, 1.18f, 3.73f}, {-1.76f, 0.0f, 1.109f, 8.54f}}},  // 192 x 192
+    {19, {{2.943f, 0.301f, 0.476f, 1.5f}, {3.728f, 0.193f, 0.454f, 1.02f}, {kNever, 0, 0, 0}}},  // 64 x 128
+    {20, {{1.516f, 1.613f, 1.142f, 5.466f}, {2.319f, 1.885f, 0.857f, 7.036f}, {-2.7f, 0.0f, 1.183f, 9.8f}}},  // 144 x 256
+    {21, {{1.507f, 1.948f, 1.394f, 5.467f}, {1.5f, 1.756f, 0.958f, 7.636f}, {-3.86f, 0.0f, 1.419f, 11.8f}}},  // 192 x 256
+    {22, {{2.158f, 1.981f, 1.291f, 9.226f}, {1.5f, 0.283f, 1.017f, 13.191f}, {-2.06f, 0.0f, 1.362f, 11.77f}}},  // 288 x 192
+    {23, {{1.652f, 0.481f, 0.827f, 5.867f}, {2.509f, 0.208f, 0.587f, 9.679f}, {-1.64f, 0.0f, 0.87f, 8.72f}}},  // 256 x 128
 };
 
 int cheapest_tile8(int64_t M, int64_t N, int64_t K, int splits, int kind, float* us) {
