@@ -258,7 +258,7 @@ int oasis_gemm_bf16_frag(const void* A, int64_t a_rows, const void* B, int64_t M
 /* fp8 weight GEMM: acc[M,N] = A[M,K] @ (Bq[N,K] * w_scale[N])^T, then the epilogue.
  * A bf16 (quantized per 32-wide K block to e4m3 with a power-of-two scale inside the kernel),
  * Bq OCP fp8 e4m3 bytes, w_scale fp32 per output channel. K % 128 == 0, N % 8 == 0,
- * lda % 8 == 0, ldb % 16 == 0, both below 2^22. tile: 0..23 (gemm_fp8.hip's kTiles8), -1 = default;
+ * lda % 8 == 0, ldb % 16 == 0, both below 2^22. tile: 0..4 (gemm_fp8.hip's kTiles8), -1 = default;
  * splits divides K/128 (> 1 requires OASIS_EPI_PARTIAL_F32).
  * No counterpart in the reference: it has no sub-fp32 weight path (the config-4 serving
  * case of the build's benchmark plan). */
@@ -268,7 +268,7 @@ int oasis_gemm_fp8(const void* A, int64_t lda, const void* Bq, int64_t ldb, cons
 
 /* Same product with the A operand already in fp8 activation blocks: A8 e4m3 bytes [M, lda]
  * (lda % 16 == 0) and A_scale e8m0 bytes [M, lds] (lds >= K/32, lds % 4 == 0), one scale per
- * 32-wide K block (as oasis_quantize_act_fp8 and OASIS_EPI_GELU_TANH_FP8 write them).
+ * 32-wide K block (as oasis_quantize_act_fp8 and OASIS_EPI_GELU_TANH_FP8 write them). tile: 0..23, -1 = default.
  * No counterpart in the reference (see oasis_gemm_fp8). */
 int oasis_gemm_fp8_a8(const void* A8, int64_t lda, const void* A_scale, int64_t lds, const void* Bq,
                       int64_t ldb, const float* w_scale, int64_t M, int64_t N, int64_t K,
@@ -358,7 +358,7 @@ int oasis_temporal_qkv_attention(const void* h, int64_t ldh, const void* w_qkv, 
 
 enum { OASIS_ACT_NONE = 0, OASIS_ACT_SILU = 1, OASIS_ACT_TEMB = 2 };
 
-/* Skinny GEMM for R <= 1024 rows (one pass over W per 16 rows):
+/* Skinny GEMM for R <= 1024 rows (one pass over W per 32 rows, or 16 where 32 do not fit in LDS):
  * out[r, n] (+)= act_out(sum_k act_in(x[r, k]) W[n, k] + b[n]).
  * x fp32 [R, ldx], W bf16 [N, K] (K % 64 == 0), b fp32 [N] or NULL, out fp32 [R, ld_out].
  * x is split into bf16 hi + lo parts, so the product keeps ~16 mantissa bits of x.
@@ -371,7 +371,8 @@ int oasis_gemv_bf16(const float* x, int64_t ldx, int64_t R, const void* W, int64
 /* Same product with W in 16-row MFMA tile order: for tile t (rows 16t..16t+15) and each
  * 32-wide K step s, 64 pieces of 8 bf16 back to back, piece l holding row 16t + (l & 15),
  * columns 32s + 8(l >> 4) .. +7 (tile t, step s at element offset (t*K/32 + s)*512). Each
- * wave's weight loads are then 1 KB contiguous. The DiT's stacked adaLN weights (ada_w of
+ * wave's weight loads are then 1 KB contiguous, and many rows (from 9, more where K is short) over 8192 outputs
+ * and up take one pass over W per 96. The DiT's stacked adaLN weights (ada_w of
  * oasis_dit_weights_t) are kept in this order. No counterpart in the reference: a storage
  * order of the adaLN projections' weights (oasis_inference.py:983-993). */
 int oasis_gemv_bf16_tiled(const float* x, int64_t ldx, int64_t R, const void* W, int64_t N,

@@ -7,8 +7,8 @@
 //
 // Kernels (v_mfma_f32_16x16x32_bf16 throughout; K in 64-wide tiles):
 //   - gemm_lds_kernel: 4 waves, the K tiles copied global -> LDS by the memory pipeline itself
-//     (global_load_lds_dwordx4) into a ring of STAGES tiles; small tiles for the split-K slices
-//     and the QKV + RoPE product at 144 / 288 tokens.
+//     (global_load_lds_dwordx4) into a ring of STAGES tiles; small tiles for K slices the wave-split
+//     kernel does not take, and for short K above 320 tokens.
 //   - gemm_big_kernel: the same ring with a grouped tile order and a per-wave staged epilogue, on
 //     4- to 16-wave tiles: most products above 320 tokens, the VAE's among them, by measured cost
 //     (kCosts).
@@ -1108,8 +1108,9 @@ hipError_t launch_lds(const bf16* A, int64_t lda, const bf16* B, int64_t ldb, in
   return hipGetLastError();
 }
 
-// Tile configurations (id -> BM x BN, wave grid, prefetch depth): the ones the default choice
-// below uses, for the shapes of the DiT step, the frame, the VAE and the large-token batches.
+// Tile configurations (id -> BM x BN, wave grid, prefetch depth). The default choice below uses 0-4, 8-12
+// and 18-29; 5-7 and 13-17, the large-token tiles before it went by measured cost, run by explicit id and
+// the OASIS_GEMM_PLAN, OASIS_O_UNSPLIT and OASIS_FC2_UNSPLIT overrides.
 typedef hipError_t (*launch_fn)(const bf16*, int64_t, const bf16*, int64_t, int, int, int, int, const Epi&,
                                 hipStream_t);
 struct TileCfg {
@@ -1120,7 +1121,7 @@ struct TileCfg {
   int k_max = 1 << 30;  // and at most this long
 };
 const TileCfg kTiles[] = {
-    // direct-to-LDS, 4 waves: split-K slices of the O projection, QKV + RoPE at 144 / 288 tokens
+    // direct-to-LDS, 4 waves: K slices the wave-split tiles do not take, short K above 320 tokens
     {32, 64, launch_lds<32, 64, 1, 4, 4>},                  // 0: 4 K tiles in flight
     {32, 64, launch_lds<32, 64, 1, 4, 3>},                  // 1: 3 K tiles in flight
     // the 8-wave kernel's grouped tile order and per-wave staged epilogue on 4- and 6-wave tiles:
@@ -1129,7 +1130,7 @@ const TileCfg kTiles[] = {
     {64, 64, launch_big<64, 64, 2, 2, 4, 6>},               // 3: groups of 6 n tiles (576 tokens: an XCD's 54 tiles
                                                             //    are 6 whole weight slices)
     {144, 64, launch_big<144, 64, 3, 2, 4>},                // 4: 6 waves
-    // 8-wave large-token tiles
+    // 8-wave large-token tiles (by explicit id)
     {288, 256, launch_big<288, 256, 2, 4, 2>},              // 5
     {288, 192, launch_big<288, 192, 2, 4, 2>, 1},           // 6
     {288, 128, launch_big<288, 128, 2, 4, 2>},              // 7
@@ -1142,14 +1143,13 @@ const TileCfg kTiles[] = {
     {48, 64, launch_wave<48, 64, 2>, 1, 256, 2048},                       // 10
     {64, 64, launch_wave<64, 64, 2>, 1, 256, 2048},                       // 11
     {32, 64, launch_wave<32, 64, 2>, 1, 256, 2048},                       // 12
-    // large-token products of N = 1024 run unsplit (the O projection with its gated residual in
-    // the epilogue): 256 workgroups at 4608 tokens, 6 waves of 48 x 64 or 8 of 144 x 16
+    // 256 workgroups for an unsplit product of 4608 x 1024, 6 waves of 48 x 64 or 8 of 144 x 16 (by explicit id)
     {144, 128, launch_big<144, 128, 3, 2, 2>},                            // 13
     {288, 64, launch_big<288, 64, 2, 4, 2>, 1},                           // 14
     {144, 128, launch_big<144, 128, 3, 2, 3>},                            // 15: 3 stages
     {144, 128, launch_big<144, 128, 3, 2, 4>},                            // 16: 4 stages
     {288, 128, launch_big<288, 128, 2, 4, 3>},                            // 17: 3 stages
-    // above 320 tokens (kCosts picks among these and tiles 2-4 and 9-12): wave tiles of 48 x 32 to
+    // above 320 tokens (kCosts picks among these and tiles 1-4 and 9-12): wave tiles of 48 x 32 to
     // 96 x 64 on 6 to 16 waves, sized so that some tile fills one round of 256 CUs at any row count;
     // the two-stage ones of 64 and 56 KB run two workgroups per CU
     {144, 128, launch_big<144, 128, 3, 4, 3>},                            // 18: 12 waves
@@ -1361,9 +1361,7 @@ int gemm_frag_launch(const bf16* A, int64_t a_rows, const bf16* B, int64_t M, in
   return OASIS_OK;
 }
 
-// Default tile choice. M is small (288 / 576 tokens) and the weights are streamed once,
-// so the tiles trade L2 re-reads of A and B against enough workgroups (and K-tiles in
-// flight per workgroup) to keep all 256 CUs issuing HBM loads.
+// unsplit on the default tile
 int gemm_launch(const bf16* A, int64_t lda, const bf16* B, int64_t ldb, int64_t M, int64_t N, int64_t K,
                 const oasis_epilogue_t& ex, hipStream_t s) {
   return gemm_launch_cfg(A, lda, B, ldb, M, N, K, ex, -1, 1, s);

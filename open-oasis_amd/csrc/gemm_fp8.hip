@@ -519,10 +519,12 @@ const Tile8 kTiles8[] = {
     OASIS_T8(64, 128, 2, 2),               // 2
     OASIS_T8(64, 64, 2, 2),                // 3
     OASIS_T8(32, 64, 1, 4),                // 4
-    OASIS_T8_BIG(288, 256, 2, 4, 0, 2),    // 5  (fp8 A only; two stages)
+    // fp8 A only from here on; 6-9 and 11 by explicit id (and the OASIS_GEMM_PLAN8, OASIS_O_UNSPLIT and
+    // OASIS_FC2_UNSPLIT overrides)
+    OASIS_T8_BIG(288, 256, 2, 4, 0, 2),    // 5  (two stages)
     OASIS_T8_BIG(288, 192, 2, 4, 1, 2),    // 6
     OASIS_T8_BIG(288, 128, 2, 4, 0, 2),    // 7
-    OASIS_T8_BIG(144, 128, 3, 2, 0, 2),    // 8  (N = 1024 unsplit at 4608 tokens: 256 tiles)
+    OASIS_T8_BIG(144, 128, 3, 2, 0, 2),    // 8  (256 tiles of an unsplit 4608 x 1024 product)
     OASIS_T8_BIG(288, 64, 2, 4, 1, 2),     // 9
     OASIS_T8_BIG(144, 128, 3, 2, 0, 3),    // 10 (three stages)
     OASIS_T8_BIG(144, 128, 3, 2, 0, 4),    // 11 (four stages)
