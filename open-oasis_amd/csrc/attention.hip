@@ -776,6 +776,10 @@ __global__ __launch_bounds__(256) void temporal_tile_kernel(const bf16* __restri
   float p[NT][NT][4], inv[NT];  // [query tile][key tile]
 #pragma unroll
   for (int qt = 0; qt < NT; ++qt) {
+    // score - max as written, so that the largest score gives exactly 0: fused into one multiply-add with the scale
+    // (only where a tile of keys needs no mask, the queries past the first 16) the maximum's rounding remains, which
+    // above 2^31 overflows exp2
+#pragma clang fp contract(off)
     const int my_q = qt * 16 + lr, first = NT == 1 ? my_q - my_q % T : 0;  // the query's group starts at row `first`
     float mx = -INFINITY;
 #pragma unroll

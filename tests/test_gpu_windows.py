@@ -51,3 +51,18 @@ def test_temporal_windows_keep_non_finite_values_apart(T, bad):
     # the finite elements may be summed in another order: one bf16 step
     assert torch.isfinite(out[~hit]).all()
     assert ((out - clean)[~hit].abs() <= 2.0 ** -7 * clean[~hit].abs() + 1e-4).all()
+
+
+@pytest.mark.parametrize("T", [8, 11, 16, 17, 24, 32, 33])
+@pytest.mark.parametrize("big", [2.0 ** 33, 2.0 ** 120])
+def test_temporal_windows_of_huge_scores(T, big):
+    """Scores beyond what exp2 holds, finite in fp32: the key of the largest score gets probability 1."""
+    q, k, v = _inputs(2, 5, 3, T)
+    k[..., T // 2, 9] = big
+    out = _run(q, k, v).double()
+    s = (q.double().unsqueeze(-2) * k.double().unsqueeze(-3)).sum(-1) * 0.125
+    p = s.masked_fill(~torch.ones(T, T, dtype=torch.bool, device="cuda").tril(), float("-inf")).softmax(-1)
+    ref = (p.unsqueeze(-1) * v.double().unsqueeze(-3)).sum(-2)
+    # as test_temporal_windows
+    bound = 1.02 * 2.0 ** -8 * ((p.unsqueeze(-1) * v.double().abs().unsqueeze(-3)).sum(-2) + ref.abs())
+    assert torch.isfinite(out).all() and ((out - ref).abs() <= bound).all()
