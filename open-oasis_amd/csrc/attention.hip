@@ -348,12 +348,12 @@ void flash_go(dim3 g, const T* q, const T* k, const T* v, T* o, const AttnArgs& 
 // units by row % 8, a V row's 32-byte groups by (row / 2) % 4. A stage is consumed in chunks of CT 16-key tiles;
 // KSPLIT = 2: two waves per query block, each half of every stage. The sum of the probabilities is of the fp32 ones.
 // FINE: what rounding the probabilities to bf16 leaves goes through the products as a second bf16 (one stage, one
-// chunk), and their sum is a product with ones of both parts: chunks of 6 to 10 tiles round more probabilities than the
+// chunk), and their sum is a product with ones of both parts: chunks of 4 to 10 tiles round more probabilities than the
 // 32-key chunks of flash_kernel did, where every chunk's largest is 1. Relative rms error against fp64, standard normal
 // operands: at 144 keys 2.07e-3 there, 2.17e-3 without FINE, 1.66e-3 (the output's own rounding) with it, for 0.3-0.9
 // us; at 576 keys 2.16e-3 there and 2.15e-3 here.
-// Measured, before -> now: 576 tokens x 1, 2, 3, 4, 8 latents 9.9, 19.3, 20.1, 28.2, 44.8 -> 9.3, 14.3, 14.8, 18.7,
-// 29.2 us; 144 tokens x 1, 8, 12, 32, 64 frames 5.1, 8.1, 11.7, 15.8, 33.1 -> 4.8, 7.0, 8.5, 11.5, 23.7 (64 frames: 75 MB,
+// Measured, before -> now: 576 tokens x 1, 2, 3, 4, 8 latents 9.9, 19.3, 20.1, 28.2, 44.8 -> 9.0, 13.2, 14.0, 18.4,
+// 29.1 us; 144 tokens x 1, 8, 12, 32, 64 frames 5.1, 8.1, 11.7, 15.8, 33.1 -> 4.8, 7.0, 8.5, 11.5, 23.7 (64 frames: 75 MB,
 // 3.2 TB/s).
 template <int NW, int KSPLIT, int KS, int ST, int CT, bool FINE = false>
 __global__ __launch_bounds__(NW * KSPLIT * 64) void flash_ring_kernel(const bf16* __restrict__ Q,
@@ -384,7 +384,7 @@ __global__ __launch_bounds__(NW * KSPLIT * 64) void flash_ring_kernel(const bf16
   const __amdgpu_buffer_rsrc_t Krs = buffer_rsrc(K + (int64_t)bh * a.kv_bh), Vrs = buffer_rsrc(V + (int64_t)bh * a.kv_bh);
 
   const int n = (a.Lk + KS - 1) / KS;
-  auto issue = [&](int st, int buf) {  // rows past Lk are the last key's; masked below
+  auto issue = [&](int st, int buf) {  // rows past Lk are the last key's; masked and zeroed below
     char* base = smem + buf * STAGE;
 #pragma unroll
     for (int u = 0; u < LPW; ++u) {
@@ -414,6 +414,12 @@ __global__ __launch_bounds__(NW * KSPLIT * 64) void flash_ring_kernel(const bf16
     __builtin_amdgcn_s_waitcnt(WAIT);
     __builtin_amdgcn_s_barrier();
     if constexpr (ST > 1) issue(min(st + ST - 1, n - 1), (st + ST - 1) % ST);  // into the buffer read at st - 1
+    if ((st + 1) * KS > a.Lk) {  // the last key's value once only: against the 0 of a masked key an infinite one is NaN
+      char* v0 = smem + (ST > 1 ? st % ST : 0) * STAGE + KS * 128;
+      for (int i = (a.Lk - st * KS) * 8 + threadIdx.x; i < KS * 8; i += W * 64)
+        *reinterpret_cast<f32x4*>(v0 + i * 16) = f32x4{0.f, 0.f, 0.f, 0.f};
+      __syncthreads();
+    }
     if (q0 >= a.Lq) continue;
     const char* kb = smem + (ST > 1 ? st % ST : 0) * STAGE + wk * KT * 16 * 128;
     const char* vb = kb + KS * 128;
@@ -559,12 +565,13 @@ int flash_launch(const T* q, const T* k, const T* v, T* o, int64_t n_bh, const A
     if (!a.bias && !a.causal) {
       // The smallest single stage that takes the sequence, beyond 192 keys a ring. Up to 160 keys the probabilities
       // keep their remainders, but with 256 heads of whole-frame or 64-row queries, which flash_kernel took in one
-      // chunk: there 64 frames take 23.7 us without, 25.4 with them. 96- and 128-key stages keep short sequences
-      // from computing 144 (255 heads of 128 x 128: 8.0 us on flash_kernel, 8.8 on 144 keys, 6.9 on 128). At 160
+      // chunk: there 64 frames take 23.7 us without, 25.4 with them. 64-, 96- and 128-key stages keep short sequences
+      // from computing 144 (200 heads of 144 x 64: 9.1 us on flash_kernel, 6.7 on 96 keys, 5.6 on 64; 255 heads of 128 x 128: 8.0 us on flash_kernel, 8.8 on 144 keys, 6.9 on 128). At 160
       // keys 64-query workgroups where 48-query ones would be more than two per CU, or one if 64 divides the
       // queries (200 heads of 160 x 160: 48 9.2 us, 64 8.5; 64 x 160: 6.9, 5.7), else 48 (32 heads of 160 x 160:
       // 5.3, with 64 5.4). A ring with one workgroup per CU at most stages 128 keys (96 KB; 16 x 1000 x
       // 1000 13.2 us, with 64 15.3), with more of them 64 (48 KB, three per CU; 3 latents 14.6, with 128 18.3).
+      if (a.Lk <= 64) return ring_go<3, 1, 64, 1, 4, true>(q, k, v, o, n_bh, a, s);
       if (a.Lk <= 96) return ring_go<3, 1, 96, 1, 6, true>(q, k, v, o, n_bh, a, s);
       if (a.Lk <= 128) return ring_go<4, 1, 128, 1, 8, true>(q, k, v, o, n_bh, a, s);
       if (a.Lk <= 144)

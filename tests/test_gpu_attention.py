@@ -31,7 +31,7 @@ def _ref(q, k, v):
 # workgroups; one key past a stage, one short of it, one key in the last stage, and partial query tiles
 @pytest.mark.parametrize("n,sq,sk", [(1, 1, 65), (2, 97, 96), (300, 48, 95), (3, 64, 97), (2, 65, 128), (260, 130, 127),
                                      (1, 1, 129), (200, 160, 160), (171, 150, 146), (129, 64, 145), (3, 144, 143),
-                                     (256, 144, 144), (255, 144, 144), (257, 65, 1),
+                                     (256, 144, 144), (255, 144, 144), (257, 65, 1), (3, 97, 64),
                                      (2, 49, 144), (2, 47, 145), (3, 48, 160), (256, 128, 160), (256, 33, 159),
                                      (256, 48, 152), (2, 70, 161), (5, 200, 192), (2, 65, 193), (1, 16, 256),
                                      (3, 100, 257), (4, 4096, 385), (129, 100, 193), (128, 65, 320), (300, 1, 576),
@@ -53,6 +53,21 @@ def test_attention_keeps_infinite_values(n, sq, sk):
     q, k, v = _inputs(n, sq, sk)
     q = q * 0.25  # no probability underflows
     v[1, sk // 2, 9] = float("inf")
+    out = _run(q, k, v)
+    assert (out[1, :, 9] == float("inf")).all()
+    out[1, :, 9] = 0
+    assert torch.isfinite(out).all()
+
+
+# every staging variant with keys past the sequence in its last stage
+@pytest.mark.parametrize("n,sq,sk", [(3, 96, 32), (3, 144, 64), (2, 70, 65), (2, 100, 97), (2, 48, 143), (256, 144, 129),
+                                     (2, 48, 159), (256, 64, 145), (2, 70, 161), (128, 65, 320), (16, 576, 576),
+                                     (2, 40, 448), (300, 20, 641)])
+def test_attention_keeps_an_infinite_last_value(n, sq, sk):
+    """The rows that fill up the last stage repeat the last key with probability 0, and 0 x inf is not finite."""
+    q, k, v = _inputs(n, sq, sk)
+    q = q * 0.25  # no probability underflows
+    v[1, sk - 1, 9] = float("inf")
     out = _run(q, k, v)
     assert (out[1, :, 9] == float("inf")).all()
     out[1, :, 9] = 0
