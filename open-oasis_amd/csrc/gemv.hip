@@ -572,7 +572,7 @@ __global__ __launch_bounds__(256) void gemv_f32_kernel(const float* __restrict__
 __device__ __forceinline__ float silu_rcp(float x) {
   const float d = 1.0f + __expf(-x);
   const float r = __builtin_amdgcn_rcpf(d);
-  return d < 3.0e38f ? x * fmaf(r, fmaf(-d, r, 1.0f), r) : x / d;  // past it the step is inf * 0
+  return d < 0x1p126f ? x * fmaf(r, fmaf(-d, r, 1.0f), r) : x / d;  // past it r is no normal number, given as 0
 }
 
 // The same product for more than F32_RP rows on v_mfma_f32_16x16x4_f32 (fp32 operands and sums): a

@@ -71,6 +71,18 @@ def test_f32_rows(R, N, K, act_in, act_out, acc):
     assert (out.cpu().double() - y).norm() <= (1e-4 if act_in == 2 else 2e-6) * y.norm()
 
 
+@pytest.mark.parametrize("R", [8, 9])
+@pytest.mark.parametrize("x", [-80.0, -87.0, -87.5, -88.0, -88.5])
+def test_f32_rows_of_tiny_silu(R, x):
+    """1 + exp(-x) from 2^126 up: its reciprocal is no normal number, x over it still is."""
+    xd, W, out = torch.full((R, 64), x, device="cuda"), torch.full((64, 64), 2.0 ** 100, device="cuda"), torch.zeros(R, 64, device="cuda")
+    L.call("oasis_gemv_f32", L.ptr(xd), 64, R, L.ptr(W), 64, 64, None, L.ptr(out), 64, 1, 0, 0, stream())
+    sync()
+    ref = 64 * 2.0 ** 100 * _silu(torch.tensor(x, dtype=torch.float64)).item()
+    # the fp32 exponent -x log2(e) = 127 holds 2^-18: 3e-6 of the exponential
+    assert ((out.double() - ref).abs() <= 1e-5 * abs(ref)).all()
+
+
 @pytest.mark.parametrize("R", [9, 41, 96, 97])
 def test_conditioning_rows_do_not_depend_on_the_batch(R):
     """The rows of one conditioning call (the MFMA kernels, [hid | action] side by side, and the adaLN rows kernel
