@@ -747,7 +747,7 @@ __global__ __launch_bounds__(256) void temporal_kernel(const bf16* __restrict__ 
 template <int NT>
 __global__ __launch_bounds__(256) void temporal_tile_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k,
                                                             const bf16* __restrict__ v, bf16* __restrict__ out,
-                                                            int64_t rows, int T, int tile_rows, int P, int H,
+                                                            int rows, int T, int groups, int P, int H,
                                                             float scale_log2, int fks, uint8_t* __restrict__ out8,
                                                             uint8_t* __restrict__ out8s, oasis::Prefetch pf) {
   __shared__ __attribute__((aligned(1024))) char vs_all[4 * NT * 2048];
@@ -757,11 +757,12 @@ __global__ __launch_bounds__(256) void temporal_tile_kernel(const bf16* __restri
   }
   const int lane = threadIdx.x & 63, lr = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int64_t r0 = ((int64_t)blockIdx.x * (blockDim.x >> 6) + wave) * tile_rows;
+  const int tile = blockIdx.x * (blockDim.x >> 6) + wave, r0 = tile * groups * T;
   if (r0 >= rows) return;
-  const int n = (int)(rows - r0 < tile_rows ? rows - r0 : tile_rows);
+  const int n = min(rows - r0, groups * T);
   char* vs = vs_all + wave * NT * 2048;
-  const __amdgpu_buffer_rsrc_t Qrs = buffer_rsrc(q + r0 * 64), Krs = buffer_rsrc(k + r0 * 64), Vrs = buffer_rsrc(v + r0 * 64);
+  const int64_t e0 = (int64_t)r0 * 64;
+  const __amdgpu_buffer_rsrc_t Qrs = buffer_rsrc(q + e0), Krs = buffer_rsrc(k + e0), Vrs = buffer_rsrc(v + e0);
   // rows past the tile read its last row; what they give is masked or not stored
 #pragma unroll
   for (int b = 0; b < NT * 2; ++b) {
@@ -869,10 +870,9 @@ __global__ __launch_bounds__(256) void temporal_tile_kernel(const bf16* __restri
           }
     }
     if (my_q >= n) continue;  // the 4 lanes of a query leave together
-    const int64_t row = r0 + my_q, grp = row / T;
-    const int t = (int)(row - grp * T), h = (int)(grp % H);
-    const int64_t bp = grp / H, b = bp / P, pos = bp - b * P;
-    store_head<bf16>(out, ((b * T + t) * P + pos) * (int64_t)(H * 64) + h * 64, o, inv[qt], g, fks, out8, out8s);
+    const unsigned gi = NT == 1 ? (unsigned)my_q / (unsigned)T : 0, grp = tile * groups + gi, t = my_q - gi * T;
+    const unsigned bp = grp / (unsigned)H, h = grp - bp * H, b = bp / (unsigned)P, pos = bp - b * P;
+    store_head<bf16>(out, (int64_t)((b * T + t) * P + pos) * (H * 64) + h * 64, o, inv[qt], g, fks, out8, out8s);
   }
 }
 
@@ -985,8 +985,8 @@ int temporal_attention(const void* q, const void* k, const void* v, void* out, i
     // token-major at row (b*T + t)*P + p. Up to 32 frames a wave per tile of rows, beyond on flash_kernel.
     OASIS_REQUIRE(G <= 65535, OASIS_ERR_SHAPE, "temporal_attention: too many (stream, position, head) groups");
     if (T <= 32) {
-      const int tile_rows = T <= 16 ? (int)(16 / T * T) : (int)T;
-      const int64_t tiles = (G * T + tile_rows - 1) / tile_rows;
+      const int groups = T <= 16 ? (int)(16 / T) : 1;
+      const int64_t tiles = (G + groups - 1) / groups;
       // up to 12 tiles per CU a workgroup each: four waves in one leave CUs idle (256 groups of 24 frames 4.2 us on
       // flash_kernel, 4.9 with four waves, 4.3 with one; 2304 groups of 16: 7.1, 5.6, 5.2); beyond, four start faster
       // (9216 groups of 32: 25.8 us, 27.2 with one). As fp8 blocks 256 groups of 24 take 5.0 us, 4.3 on flash_kernel,
@@ -994,10 +994,10 @@ int temporal_attention(const void* q, const void* k, const void* v, void* out, i
       const int waves = tiles <= 12 * 256 ? 1 : 4;
       const dim3 grid((unsigned)((tiles + waves - 1) / waves), 1, gz), block(waves * 64);
       if (T <= 16)
-        hipLaunchKernelGGL((temporal_tile_kernel<1>), grid, block, 0, stream, qp, kp, vp, op, G * T, (int)T, tile_rows,
+        hipLaunchKernelGGL((temporal_tile_kernel<1>), grid, block, 0, stream, qp, kp, vp, op, (int)(G * T), (int)T, groups,
                            (int)P, (int)n_heads, sl, fks, out8, out8_scale, pfv);
       else
-        hipLaunchKernelGGL((temporal_tile_kernel<2>), grid, block, 0, stream, qp, kp, vp, op, G * T, (int)T, tile_rows,
+        hipLaunchKernelGGL((temporal_tile_kernel<2>), grid, block, 0, stream, qp, kp, vp, op, (int)(G * T), (int)T, groups,
                            (int)P, (int)n_heads, sl, fks, out8, out8_scale, pfv);
       return check_launch("temporal_attention");
     }
