@@ -305,11 +305,14 @@ namespace {
 // rows of x per pass of gemv_rows_kernel, and the fewest outputs: below 512 weight tiles gemv_kernel splits K over
 // the waves instead
 constexpr int64_t kRowsPass = 96, kRowsMinN = 512 * 16;
-// The fewest rows: its waves cross a barrier per 64-wide chunk of K, which few rows or few chunks do not repay. At
-// 12288 outputs, gemv_kernel and here: K = 64 x 16 rows 3.9 and 4.5 us, x 32 5.5 and 5.7; K = 256 x 9 5.5 and 7.1,
-// x 16 7.3 and 6.9; K = 1024 x 9 15.9 and 17.2, x 12 19.0 and 17.2. From 24576 outputs one row less (196608 x 1024,
-// 9 rows: 81 and 76). Up to 8 rows the step's pair kernel, whose workgroups stage x once, or gemv_kernel.
-int64_t rows_min(int64_t N, int64_t K) { return std::max<int64_t>(9, 9 + 1536 / K - (N >= 24576 ? 1 : 0)); }
+// The fewest rows: its waves cross a barrier per 64-wide chunk of K, which few rows or few chunks do not repay.
+// gemv_kernel's time over this kernel's at 8192 outputs: K = 64 x 32 rows 0.96, x 33 (its second pass) 1.12; K = 128
+// x 20 0.94, x 24 1.02; K = 256 x 16 1.08, x 17 0.99, x 20 1.07; K = 512 x 11 0.96, x 13 1.05; K = 768 x 12 0.96, x 13
+// 1.03; K = 1024 x 9 0.95, x 12 1.12; K = 2048 x 9 0.93, x 11 1.07. From 24576 outputs and K = 1024 up, 9 rows take
+// 0.98 to 1.8 (196608 x 1024: 1.04). Up to 8 rows the step's pair kernel, whose workgroups stage x once, or gemv_kernel.
+int64_t rows_min(int64_t N, int64_t K) {
+  return N >= 24576 && K >= 1024 ? 9 : std::min<int64_t>(33, 10 + 2304 / K);
+}
 
 int gemv_rows(const float* x, int64_t ldx, int64_t R, const bf16* W, int64_t N, int64_t K, const float* b, float* out,
               int64_t ld_out, int act_in, int act_out, int accumulate, hipStream_t s) {

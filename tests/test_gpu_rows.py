@@ -13,12 +13,12 @@ def _silu(x):
     return x * torch.sigmoid(x)
 
 
-@pytest.mark.parametrize("R,N,K,off,act_in,act_out,acc", [(9, 8192, 64, 0, 1, 0, 0), (16, 8208, 320, 0, 0, 1, 0),
+@pytest.mark.parametrize("R,N,K,off,act_in,act_out,acc", [(9, 8192, 64, 0, 1, 0, 0), (17, 8208, 320, 0, 0, 1, 0),
                                                           (33, 9216, 1024, 0, 1, 0, 1), (80, 8224, 1024, 0, 1, 0, 0),
                                                           (96, 8400, 192, 1, 1, 0, 0), (97, 8400, 448, 0, 1, 1, 1),
                                                           (200, 8192, 2048, 3, 0, 0, 0), (40, 8176, 128, 0, 1, 0, 0),
-                                                          (33, 8192, 64, 0, 1, 0, 0), (10, 8192, 1024, 2, 1, 0, 1),
-                                                          (9, 24592, 1024, 0, 1, 0, 0), (9, 8192, 2048, 0, 0, 1, 0)])
+                                                          (33, 8192, 64, 0, 1, 0, 0), (12, 8192, 1024, 2, 1, 0, 1),
+                                                          (9, 24592, 1024, 0, 1, 0, 0), (11, 8192, 2048, 0, 0, 1, 0)])
 def test_tiled_rows(R, N, K, off, act_in, act_out, acc):
     """off: x rows that start `off` floats past a 16-byte boundary. N = 8176 and 9 rows of K = 64 are below the
     kernel's range, the last four shapes its fewest rows. The row-major kernel gives the same bits."""
