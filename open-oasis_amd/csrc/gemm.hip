@@ -1108,9 +1108,8 @@ hipError_t launch_lds(const bf16* A, int64_t lda, const bf16* B, int64_t ldb, in
   return hipGetLastError();
 }
 
-// Tile configurations (id -> BM x BN, wave grid, prefetch depth). The default choice below uses 0-4, 8-12
-// and 18-29; 5-7 and 13-17, the large-token tiles before it went by measured cost, run by explicit id and
-// the OASIS_GEMM_PLAN, OASIS_O_UNSPLIT and OASIS_FC2_UNSPLIT overrides.
+// Tile configurations (id -> BM x BN, wave grid, prefetch depth). The default choice below uses 0-12
+// and 18-29; 13-17 run by explicit id and the OASIS_GEMM_PLAN, OASIS_O_UNSPLIT and OASIS_FC2_UNSPLIT overrides.
 typedef hipError_t (*launch_fn)(const bf16*, int64_t, const bf16*, int64_t, int, int, int, int, const Epi&,
                                 hipStream_t);
 struct TileCfg {
@@ -1130,7 +1129,7 @@ const TileCfg kTiles[] = {
     {64, 64, launch_big<64, 64, 2, 2, 4, 6>},               // 3: groups of 6 n tiles (576 tokens: an XCD's 54 tiles
                                                             //    are 6 whole weight slices)
     {144, 64, launch_big<144, 64, 3, 2, 4>},                // 4: 6 waves
-    // 8-wave large-token tiles (by explicit id)
+    // 8-wave large-token tiles
     {288, 256, launch_big<288, 256, 2, 4, 2>},              // 5
     {288, 192, launch_big<288, 192, 2, 4, 2>, 1},           // 6
     {288, 128, launch_big<288, 128, 2, 4, 2>},              // 7
@@ -1149,7 +1148,7 @@ const TileCfg kTiles[] = {
     {144, 128, launch_big<144, 128, 3, 2, 3>},                            // 15: 3 stages
     {144, 128, launch_big<144, 128, 3, 2, 4>},                            // 16: 4 stages
     {288, 128, launch_big<288, 128, 2, 4, 3>},                            // 17: 3 stages
-    // above 320 tokens (kCosts picks among these and tiles 1-4 and 9-12): wave tiles of 48 x 32 to
+    // above 320 tokens (kCosts picks among these and tiles 1-7 and 9-12): wave tiles of 48 x 32 to
     // 96 x 64 on 6 to 16 waves, sized so that some tile fills one round of 256 CUs at any row count;
     // the two-stage ones of 64 and 56 KB run two workgroups per CU
     {144, 128, launch_big<144, 128, 3, 4, 3>},                            // 18: 12 waves
@@ -1167,30 +1166,32 @@ const TileCfg kTiles[] = {
 };
 constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 
-// Fitted costs (tile_cost) of the tiles used above 320 tokens: c, lat, a and b for the plain and GELU
-// stores, QKV + RoPE, the fp32 residual, and split-K slices of 512 and longer (with which split counts
-// are chosen: fitted to the DiT's O and FC2 products; shorter slices cost as residuals).
-const TileCost<4> kCosts[] = {
-    {1, {{2.504f, 0.29f, 0.145f, 0.359f}, {2.412f, 0.218f, 0.145f, 0.493f}, {2.765f, 0.289f, 0.154f, 0.694f}, {kNever, 0, 0, 0}}},  // 32 x 64
-    {2, {{3.152f, 0.287f, 0.226f, 1.353f}, {3.662f, 0.378f, 0.241f, 1.172f}, {2.64f, 0.304f, 0.219f, 1.952f}, {3.71f, 0.0f, 0.235f, 1.04f}}},  // 96 x 64
-    {3, {{2.772f, 0.282f, 0.179f, 0.919f}, {3.031f, 0.549f, 0.181f, 1.043f}, {3.123f, 0.275f, 0.172f, 1.036f}, {3.45f, 0.0f, 0.181f, 0.79f}}},  // 64 x 64
-    {4, {{1.749f, 0.425f, 0.443f, 2.687f}, {3.641f, 0.574f, 0.328f, 5.242f}, {2.076f, 0.223f, 0.356f, 3.334f}, {1.48f, 0.0f, 0.375f, 3.43f}}},  // 144 x 64
-    {9, {{1.919f, 0.064f, 0.091f, 0.8f}, {2.629f, 0.445f, 0.058f, 0.992f}, {2.447f, 0.054f, 0.096f, 0.686f}, {1.26f, 0.0f, 0.09f, 1.12f}}},  // 48 x 32
-    {10, {{1.5f, 0.21f, 0.08f, 3.342f}, {1.813f, 0.067f, 0.094f, 3.399f}, {1.5f, 0.21f, 0.15f, 2.985f}, {1.48f, 0.0f, 0.147f, 2.28f}}},  // 48 x 64
-    {11, {{1.5f, 0.036f, 0.16f, 2.339f}, {3.168f, 0.573f, 0.106f, 3.004f}, {1.668f, 0.302f, 0.125f, 3.622f}, {1.47f, 0.0f, 0.172f, 2.71f}}},  // 64 x 64
-    {12, {{1.556f, 0.058f, 0.089f, 1.749f}, {1.813f, 0.027f, 0.05f, 2.823f}, {1.952f, 0.196f, 0.133f, 1.509f}, {1.45f, 0.0f, 0.113f, 1.86f}}},  // 32 x 64
-    {18, {{2.122f, 0.152f, 0.609f, 3.053f}, {1.5f, 0.255f, 0.537f, 4.321f}, {1.89f, 0.26f, 0.653f, 5.017f}, {0.79f, 0.0f, 0.528f, 5.23f}}},  // 144 x 128
-    {19, {{3.867f, 0.84f, 0.59f, 2.345f}, {4.914f, 1.145f, 0.549f, 3.759f}, {1.5f, 0.542f, 0.751f, 5.884f}, {3.35f, 0.0f, 0.684f, 3.14f}}},  // 192 x 128
-    {20, {{1.657f, 0.065f, 0.633f, 4.694f}, {1.5f, 0.651f, 0.717f, 9.372f}, {1.72f, 0.163f, 0.67f, 6.956f}, {0.74f, 0.0f, 0.626f, 6.26f}}},  // 192 x 128
-    {21, {{1.5f, 0.259f, 0.93f, 5.683f}, {8.243f, 0.13f, 1.233f, 0.627f}, {5.071f, 0.294f, 0.904f, 5.261f}, {-0.86f, 0.0f, 0.838f, 9.16f}}},  // 144 x 256
-    {22, {{1.57f, 0.146f, 0.938f, 5.12f}, {3.154f, 0.74f, 1.094f, 3.435f}, {4.166f, 0.961f, 1.088f, 5.718f}, {-0.25f, 0.0f, 0.866f, 7.63f}}},  // 192 x 192
-    {23, {{1.727f, 0.429f, 0.454f, 2.995f}, {2.153f, 0.586f, 0.458f, 4.664f}, {1.5f, 0.505f, 0.33f, 4.663f}, {1.61f, 0.0f, 0.429f, 3.57f}}},  // 96 x 128
-    {24, {{3.129f, 0.866f, 0.472f, 1.725f}, {4.713f, 0.676f, 0.451f, 1.0f}, {2.004f, 0.671f, 0.517f, 3.636f}, {5.18f, 0.0f, 0.459f, 0.89f}}},  // 96 x 128
-    {25, {{2.183f, 0.052f, 0.585f, 2.819f}, {2.934f, 0.253f, 0.522f, 4.9f}, {1.5f, 0.054f, 0.529f, 4.747f}, {1.14f, 0.0f, 0.49f, 4.6f}}},  // 128 x 128
-    {26, {{2.203f, 0.618f, 1.199f, 7.655f}, {4.581f, 0.271f, 1.422f, 6.115f}, {5.864f, 0.314f, 0.983f, 22.77f}, {-2.81f, 0.0f, 1.197f, 13.58f}}},  // 256 x 256
-    {27, {{2.153f, 1.067f, 1.642f, 8.275f}, {8.992f, 0.38f, 1.672f, 2.623f}, {2.062f, 0.101f, 1.327f, 9.789f}, {-4.66f, 0.0f, 1.369f, 16.58f}}},  // 288 x 256
-    {28, {{1.721f, 0.58f, 0.87f, 4.712f}, {1.938f, 0.55f, 0.891f, 8.982f}, {4.356f, 0.44f, 0.718f, 5.532f}, {-0.57f, 0.0f, 0.702f, 9.04f}}},  // 256 x 128
-    {29, {{1.5f, 0.295f, 0.472f, 3.381f}, {4.784f, 0.466f, 0.587f, 3.758f}, {1.616f, 0.167f, 0.498f, 5.141f}, {1.31f, 0.0f, 0.467f, 4.25f}}},  // 144 x 96
+// Fitted costs (tile_cost) of the tiles used above 320 tokens: c, lat, a and b of each class. The gated residual
+// of 256 x 256 spills registers (48): no choice.
+const TileCost kCosts[] = {
+    {1, {{3.092f, 0.249f, 0.142f, 0.477f}, {3.036f, 0.297f, 0.136f, 0.528f}, {3.211f, 0.26f, 0.146f, 0.669f}, {2.751f, 0.283f, 0.133f, 0.632f}, {kNever, 0, 0, 0}}},  // 32 x 64
+    {2, {{5.701f, 0.265f, 0.251f, 0.806f}, {4.642f, 0.344f, 0.308f, 1.088f}, {3.954f, 0.342f, 0.223f, 1.357f}, {2.876f, 0.313f, 0.239f, 1.302f}, {3.71f, 0.0f, 0.235f, 1.04f}}},  // 96 x 64
+    {3, {{4.198f, 0.274f, 0.181f, 0.377f}, {3.621f, 0.369f, 0.158f, 0.958f}, {3.268f, 0.284f, 0.183f, 1.119f}, {3.471f, 0.278f, 0.178f, 0.987f}, {3.45f, 0.0f, 0.181f, 0.79f}}},  // 64 x 64
+    {4, {{1.617f, 0.138f, 0.37f, 3.374f}, {1.131f, 0.28f, 0.336f, 4.601f}, {1.0f, 0.439f, 0.367f, 4.555f}, {2.328f, 0.464f, 0.363f, 3.11f}, {1.48f, 0.0f, 0.375f, 3.43f}}},  // 144 x 64
+    {5, {{2.645f, 1.701f, 1.299f, 8.322f}, {1.0f, 1.657f, 1.388f, 11.903f}, {4.24f, 1.666f, 1.311f, 11.182f}, {2.681f, 1.66f, 1.366f, 9.391f}, {kNever, 0, 0, 0}}},  // 288 x 256
+    {6, {{1.029f, 1.374f, 1.104f, 11.282f}, {kNever, 0, 0, 0}, {6.254f, 1.364f, 1.253f, 6.675f}, {1.007f, 1.43f, 1.128f, 9.35f}, {kNever, 0, 0, 0}}},  // 288 x 192
+    {7, {{1.0f, 1.071f, 0.967f, 6.218f}, {kNever, 0, 0, 0}, {1.0f, 0.447f, 0.994f, 7.76f}, {1.0f, 1.229f, 0.969f, 7.123f}, {kNever, 0, 0, 0}}},  // 288 x 128
+    {9, {{1.741f, 0.158f, 0.079f, 1.404f}, {2.46f, 0.191f, 0.113f, 0.904f}, {2.186f, 0.159f, 0.082f, 1.101f}, {2.666f, 0.131f, 0.08f, 0.824f}, {1.26f, 0.0f, 0.09f, 1.12f}}},  // 48 x 32
+    {10, {{2.248f, 0.097f, 0.134f, 2.493f}, {2.265f, 0.226f, 0.124f, 2.819f}, {1.501f, 0.244f, 0.138f, 3.303f}, {2.158f, 0.215f, 0.122f, 2.308f}, {1.48f, 0.0f, 0.147f, 2.28f}}},  // 48 x 64
+    {11, {{1.872f, 0.249f, 0.156f, 2.893f}, {2.147f, 0.265f, 0.142f, 3.13f}, {1.145f, 0.055f, 0.182f, 3.25f}, {1.881f, 0.257f, 0.147f, 2.774f}, {1.47f, 0.0f, 0.172f, 2.71f}}},  // 64 x 64
+    {12, {{1.801f, 0.18f, 0.108f, 1.898f}, {1.665f, 0.289f, 0.099f, 2.162f}, {1.596f, 0.191f, 0.111f, 2.265f}, {1.618f, 0.261f, 0.105f, 1.876f}, {1.45f, 0.0f, 0.113f, 1.86f}}},  // 32 x 64
+    {18, {{1.0f, 0.264f, 0.47f, 4.945f}, {1.0f, 0.591f, 0.487f, 5.516f}, {1.0f, 0.257f, 0.461f, 6.464f}, {1.0f, 0.346f, 0.459f, 5.389f}, {0.79f, 0.0f, 0.528f, 5.23f}}},  // 144 x 128
+    {19, {{6.411f, 0.662f, 0.575f, 0.859f}, {5.758f, 0.761f, 0.573f, 2.272f}, {kNever, 0, 0, 0}, {4.758f, 1.125f, 0.551f, 2.192f}, {3.35f, 0.0f, 0.684f, 3.14f}}},  // 192 x 128
+    {20, {{2.151f, 0.774f, 0.656f, 4.377f}, {1.0f, 0.156f, 0.658f, 6.418f}, {1.0f, 0.855f, 0.668f, 7.057f}, {4.068f, 0.729f, 0.56f, 5.209f}, {0.74f, 0.0f, 0.626f, 6.26f}}},  // 192 x 128
+    {21, {{1.0f, 0.692f, 0.798f, 6.894f}, {1.0f, 0.944f, 0.821f, 7.778f}, {1.0f, 0.96f, 0.823f, 8.612f}, {1.0f, 1.039f, 0.794f, 7.839f}, {-0.86f, 0.0f, 0.838f, 9.16f}}},  // 144 x 256
+    {22, {{1.001f, 0.936f, 0.79f, 6.051f}, {1.0f, 1.039f, 0.839f, 7.202f}, {1.0f, 0.524f, 0.829f, 8.42f}, {1.0f, 1.039f, 0.74f, 7.581f}, {-0.25f, 0.0f, 0.866f, 7.63f}}},  // 192 x 192
+    {23, {{1.443f, 0.466f, 0.406f, 3.666f}, {1.235f, 0.504f, 0.419f, 4.305f}, {2.048f, 0.474f, 0.444f, 4.658f}, {2.088f, 0.902f, 0.413f, 3.533f}, {1.61f, 0.0f, 0.429f, 3.57f}}},  // 96 x 128
+    {24, {{4.714f, 0.576f, 0.331f, 0.846f}, {4.479f, 0.648f, 0.332f, 1.409f}, {5.866f, 0.647f, 0.335f, 1.075f}, {3.976f, 0.666f, 0.378f, 1.866f}, {5.18f, 0.0f, 0.459f, 0.89f}}},  // 96 x 128
+    {25, {{1.002f, 0.557f, 0.489f, 4.349f}, {1.504f, 0.088f, 0.504f, 4.74f}, {1.0f, 0.571f, 0.465f, 5.7f}, {1.424f, 0.625f, 0.479f, 4.376f}, {1.14f, 0.0f, 0.49f, 4.6f}}},  // 128 x 128
+    {26, {{3.027f, 1.243f, 1.276f, 6.532f}, {3.287f, 0.057f, 1.178f, 7.424f}, {kNever, 0, 0, 0}, {1.0f, 1.006f, 1.097f, 10.68f}, {-2.81f, 0.0f, 1.197f, 13.58f}}},  // 256 x 256
+    {27, {{4.511f, 1.135f, 1.488f, 4.944f}, {1.0f, 0.984f, 1.442f, 10.175f}, {4.601f, 1.534f, 1.374f, 8.986f}, {2.384f, 0.809f, 1.352f, 10.157f}, {-4.66f, 0.0f, 1.369f, 16.58f}}},  // 288 x 256
+    {28, {{1.0f, 0.76f, 0.712f, 6.364f}, {1.0f, 0.644f, 0.74f, 7.132f}, {1.142f, 0.865f, 0.638f, 8.68f}, {1.186f, 0.968f, 0.667f, 7.907f}, {-0.57f, 0.0f, 0.702f, 9.04f}}},  // 256 x 128
+    {29, {{1.346f, 0.535f, 0.465f, 4.389f}, {1.597f, 0.55f, 0.465f, 4.803f}, {kNever, 0, 0, 0}, {1.816f, 0.602f, 0.458f, 4.152f}, {1.31f, 0.0f, 0.467f, 4.25f}}},  // 144 x 96
 };
 
 // the K / splits a tile can run (as gemm_launch_cfg checks it)
@@ -1199,12 +1200,11 @@ bool tile_takes_k(const TileCfg& t, int64_t kslice) {
          (t.k_gran == 64 || ((kslice / t.k_gran) & (kslice / t.k_gran - 1)) == 0);
 }
 
-// the cheapest tile above 320 tokens; *us (optional) its cost
-int cheapest_tile(int64_t M, int64_t N, int64_t K, int splits, int kind, float* us) {
+// the cheapest tile above 320 tokens by the costs of class cls; *us (optional) its cost
+int cheapest_tile(int64_t M, int64_t N, int64_t K, int splits, int kind, int cls, float* us) {
   int best = 2;
   float best_us = kNever;
-  const int cls = kind == OASIS_EPI_PARTIAL_F32 && K / splits >= 512 ? COST_PART : cost_class(kind);
-  for (const TileCost<4>& c : kCosts) {
+  for (const TileCost& c : kCosts) {
     const TileCfg& t = kTiles[c.tile];
     if (!tile_takes_k(t, K / splits) || (t.no_fp8_epi && kind == OASIS_EPI_GELU_TANH_FP8)) continue;
     const float cost = tile_cost(c, t.bm, t.bn, M, N, K / splits / 64, splits, cls);
@@ -1234,7 +1234,7 @@ namespace oasis {
 //     else; split-K partials on 32 x 64 (tile 0) for short slices and tile 2 else; other epilogues on
 //     32 x 64 (tile 1).
 int auto_tile(int64_t M, int64_t N, int64_t K, int splits, int kind) {
-  if (M > 320) return cheapest_tile(M, N, K, splits, kind, nullptr);
+  if (M > 320) return cheapest_tile(M, N, K, splits, kind, cost_class(kind), nullptr);
   const int64_t Kslice = K / splits;
   const bool wave_k = Kslice % 256 == 0 && Kslice <= 2048 && ((Kslice / 256) & (Kslice / 256 - 1)) == 0;
   const bool gelu = kind == OASIS_EPI_GELU_TANH || kind == OASIS_EPI_GELU_ERF || kind == OASIS_EPI_GELU_TANH_FRAG;
@@ -1257,7 +1257,7 @@ int gemm_auto_splits(int64_t M, int64_t N, int64_t K, int max_splits) {
   for (int s = 1; s <= std::min(max_splits, 8); s *= 2) {
     if ((K / 64) % s != 0) break;
     float us;
-    cheapest_tile(M, N, K, s, OASIS_EPI_PARTIAL_F32, &us);
+    cheapest_tile(M, N, K, s, OASIS_EPI_PARTIAL_F32, COST_SPLIT, &us);
     if (s > 1) us += split_cost(M, N, s);
     if (us < best_us) {
       best_us = us;

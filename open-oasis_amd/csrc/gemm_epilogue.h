@@ -89,31 +89,31 @@ __device__ __forceinline__ void grouped_tile(int pid, int Mt, int Nt, int GN, in
 // the busiest CU, one after another or side by side, and takes about
 //     c + max(lat * nk, W * (a * nk + b))  microseconds,  nk = K tiles of a workgroup's K slice,
 // lat the time of a K tile of a workgroup that has its CU to itself. c, lat, a and b of a tile and an
-// epilogue class are fitted to hipGraphs of 16 launches over cold weights at 14 row counts from 321 to
-// 9216 (fp8: 20 from 1), N = 64 to 4096 and K = 64 (fp8: 128) to 4096, and at every whole number of frames
-// of the DiT's products up to 64: a least-squares start, then a descent on the time of the picked tile
-// over that of the fastest. It is what the width alone could not
-// say: 1440 x 4096 in 144 x 64 tiles is 640 workgroups, three rounds of 256 of which the last is half
-// empty (29.8 us), in 192 x 128 tiles 256 workgroups (19.0 us). Over 2048 (fp8: 2244) such shapes the
-// tile it picks takes 1.017 (fp8: 1.007) times the fastest of all tiles in the mean, 1.31 (1.18) at
-// worst, where K = 4096; fitted at K = 1024 alone it took up to 3.2 (2.9) times at K = 64 (128).
-enum { COST_STORE = 0, COST_QKV = 1, COST_RES = 2, COST_PART = 3 };
-template <int CLASSES>
+// epilogue class are fitted to hipGraphs of 6 to 12 launches of every tile over cold weights at 4514 (fp8: 4444)
+// shapes: 23 row counts from 321 (fp8: 28 from 64) to 9216 of 16 products, every whole number of frames up to 64 of
+// the DiT's, and 70 products of any N from 64 to 6144 and K from 64 (fp8: 128) to 4096. A descent on the time of the
+// picked tile over that of the fastest, and over that of the rule by width that came before. It is what the width
+// alone could not say: 1440 x 4096 in 144 x 64 tiles is 640 workgroups, three rounds of 256 of which the last is half
+// empty (29.8 us), in 192 x 128 tiles 256 workgroups (19.0 us). Over those shapes the tile it picks takes 1.004
+// times the fastest of all in the mean, 1.17 (fp8: 1.28) at worst. Over 4142 others drawn at random 1.4 % run more
+// than 2 % slower than by the width (0.83 at worst: 344 x 4800 x 3584 in fp8), all together 1.38 times as fast.
+// COST_SPLIT: partial sums by an earlier fit to the DiT's O and FC2 products, with which split-K counts are chosen.
+enum { COST_STORE = 0, COST_QKV = 1, COST_RES = 2, COST_PART = 3, COST_SPLIT = 4 };
 struct TileCost {
   int tile;
   struct {
     float c, lat, a, b;
-  } k[CLASSES];
+  } k[5];
 };
 constexpr float kNever = 1e9f;  // class not run on this tile
-// plain and GELU stores; QKV + RoPE; fp32 residuals and partial sums
+// plain and GELU stores; QKV + RoPE; fp32 residuals; partial sums
 inline int cost_class(int kind) {
   if (kind == OASIS_EPI_QKV_ROPE) return COST_QKV;
-  return kind == OASIS_EPI_PARTIAL_F32 || kind == OASIS_EPI_GATED_RES || kind == OASIS_EPI_RESIDUAL ? COST_RES : COST_STORE;
+  if (kind == OASIS_EPI_PARTIAL_F32) return COST_PART;
+  return kind == OASIS_EPI_GATED_RES || kind == OASIS_EPI_RESIDUAL ? COST_RES : COST_STORE;
 }
 // microseconds of an M x N product in bm x bn tiles and nk K tiles per workgroup
-template <int CLASSES>
-inline float tile_cost(const TileCost<CLASSES>& t, int bm, int bn, int64_t M, int64_t N, int64_t nk, int splits, int cls) {
+inline float tile_cost(const TileCost& t, int bm, int bn, int64_t M, int64_t N, int64_t nk, int splits, int cls) {
   const auto& k = t.k[cls];
   const int64_t tiles = (M + bm - 1) / bm * ((N + bn - 1) / bn) * splits;
   const float lone = k.lat * (float)nk, busy = (float)((tiles + 255) / 256) * (k.a * (float)nk + k.b);

@@ -519,7 +519,7 @@ const Tile8 kTiles8[] = {
     OASIS_T8(64, 128, 2, 2),               // 2
     OASIS_T8(64, 64, 2, 2),                // 3
     OASIS_T8(32, 64, 1, 4),                // 4
-    // fp8 A only from here on; 6-9 and 11 by explicit id (and the OASIS_GEMM_PLAN8, OASIS_O_UNSPLIT and
+    // fp8 A only from here on; 8, 9 and 11 by explicit id (and the OASIS_GEMM_PLAN8, OASIS_O_UNSPLIT and
     // OASIS_FC2_UNSPLIT overrides)
     OASIS_T8_BIG(288, 256, 2, 4, 0, 2),    // 5  (two stages)
     OASIS_T8_BIG(288, 192, 2, 4, 1, 2),    // 6
@@ -528,7 +528,7 @@ const Tile8 kTiles8[] = {
     OASIS_T8_BIG(288, 64, 2, 4, 1, 2),     // 9
     OASIS_T8_BIG(144, 128, 3, 2, 0, 3),    // 10 (three stages)
     OASIS_T8_BIG(144, 128, 3, 2, 0, 4),    // 11 (four stages)
-    // with 0, 2 to 5 and 10 what kCosts8 picks from (fp8 A): 32 x 32 to 96 x 64 wave tiles on 4 to 16 waves
+    // with 3 to 7 and 10 what kCosts8 picks from (fp8 A): 32 x 32 to 96 x 64 wave tiles on 4 to 16 waves
     OASIS_T8_BIG(64, 64, 2, 2, 0, 4),      // 12
     OASIS_T8_BIG(96, 64, 2, 2, 0, 3),      // 13
     OASIS_T8_BIG(96, 128, 2, 4, 0, 3),     // 14
@@ -546,36 +546,37 @@ const Tile8 kTiles8[] = {
 #undef OASIS_T8_BIG
 constexpr int kNumTiles8 = sizeof(kTiles8) / sizeof(kTiles8[0]);
 
-// Fitted costs (tile_cost, 128-wide K tiles) of the tiles for fp8 A: c, lat, a and b for the plain and
-// GELU stores, QKV + RoPE, and the fp32 residual and partial-sum epilogues.
-const TileCost<3> kCosts8[] = {
-    {0, {{5.138f, 0.875f, 0.884f, 2.769f}, {5.363f, 0.864f, 1.094f, 6.275f}, {kNever, 0, 0, 0}}},  // 128 x 128
-    {2, {{5.413f, 0.135f, 0.37f, 1.596f}, {6.008f, 0.487f, 0.477f, 1.483f}, {kNever, 0, 0, 0}}},  // 64 x 128
-    {3, {{3.496f, 0.394f, 0.285f, 0.475f}, {3.167f, 0.737f, 0.205f, 1.08f}, {kNever, 0, 0, 0}}},  // 64 x 64
-    {4, {{2.904f, 0.14f, 0.204f, 0.215f}, {3.102f, 0.455f, 0.209f, 0.255f}, {3.33f, 0.0f, 0.212f, 0.36f}}},  // 32 x 64
-    {5, {{1.5f, 1.455f, 1.507f, 10.538f}, {6.886f, 1.487f, 1.482f, 7.142f}, {-5.24f, 0.0f, 1.52f, 15.95f}}},  // 288 x 256
-    {10, {{1.5f, 0.634f, 0.696f, 4.631f}, {5.032f, 1.323f, 0.731f, 5.684f}, {0.33f, 0.0f, 0.719f, 5.47f}}},  // 144 x 128
-    {12, {{2.784f, 0.416f, 0.335f, 1.13f}, {3.308f, 0.29f, 0.364f, 1.226f}, {2.63f, 0.0f, 0.365f, 1.09f}}},  // 64 x 64
-    {13, {{3.665f, 0.405f, 0.402f, 1.51f}, {5.016f, 0.324f, 0.394f, 0.469f}, {3.44f, 0.0f, 0.409f, 1.09f}}},  // 96 x 64
-    {14, {{1.642f, 0.633f, 0.676f, 2.935f}, {2.626f, 0.364f, 0.618f, 2.389f}, {0.37f, 0.0f, 0.698f, 3.96f}}},  // 96 x 128
-    {15, {{1.5f, 0.385f, 0.758f, 3.518f}, {2.798f, 0.71f, 0.439f, 6.12f}, {-0.94f, 0.0f, 0.821f, 6.04f}}},  // 144 x 128
-    {16, {{1.649f, 0.254f, 0.466f, 3.172f}, {1.813f, 0.885f, 0.521f, 3.108f}, {0.78f, 0.0f, 0.578f, 3.62f}}},  // 144 x 64
-    {17, {{1.5f, 0.258f, 0.83f, 4.92f}, {1.5f, 0.914f, 0.533f, 7.483f}, {-0.86f, 0.0f, 0.786f, 6.93f}}},  // 192 x 128
-    {18, {{1.741f, 0.821f, 1.079f, 5.008f}, {2.813f, 0.527f, 1.18f, 3.73f}, {-1.76f, 0.0f, 1.109f, 8.54f}}},  // 192 x 192
-    {19, {{2.943f, 0.301f, 0.476f, 1.5f}, {3.728f, 0.193f, 0.454f, 1.02f}, {kNever, 0, 0, 0}}},  // 64 x 128
-    {20, {{1.516f, 1.613f, 1.142f, 5.466f}, {2.319f, 1.885f, 0.857f, 7.036f}, {-2.7f, 0.0f, 1.183f, 9.8f}}},  // 144 x 256
-    {21, {{1.507f, 1.948f, 1.394f, 5.467f}, {1.5f, 1.756f, 0.958f, 7.636f}, {-3.86f, 0.0f, 1.419f, 11.8f}}},  // 192 x 256
-    {22, {{2.158f, 1.981f, 1.291f, 9.226f}, {1.5f, 0.283f, 1.017f, 13.191f}, {-2.06f, 0.0f, 1.362f, 11.77f}}},  // 288 x 192
-    {23, {{1.652f, 0.481f, 0.827f, 5.867f}, {2.509f, 0.208f, 0.587f, 9.679f}, {-1.64f, 0.0f, 0.87f, 8.72f}}},  // 256 x 128
+// Fitted costs (tile_cost, 128-wide K tiles) of the tiles for fp8 A: c, lat, a and b of each class. The gated
+// residuals of 192 x 256 and 288 x 192 (tile 22) spill registers (24 and 74) and are no choice: 9216 x 3072 x 1024
+// took 98.2 us on them, 58.9 on 288 x 128.
+const TileCost kCosts8[] = {
+    {3, {{3.818f, 0.38f, 0.27f, 0.826f}, {2.697f, 0.584f, 0.216f, 1.606f}, {3.779f, 0.339f, 0.279f, 1.273f}, {3.429f, 0.401f, 0.309f, 1.017f}, {kNever, 0, 0, 0}}},  // 64 x 64
+    {4, {{2.277f, 0.361f, 0.203f, 0.46f}, {2.452f, 0.407f, 0.2f, 0.532f}, {3.081f, 0.317f, 0.229f, 0.31f}, {2.219f, 0.476f, 0.233f, 0.525f}, {3.33f, 0.0f, 0.212f, 0.36f}}},  // 32 x 64
+    {5, {{1.512f, 1.836f, 1.408f, 10.805f}, {1.0f, 0.806f, 1.561f, 11.0f}, {1.0f, 2.014f, 1.581f, 12.581f}, {1.0f, 2.167f, 1.395f, 10.167f}, {-5.24f, 0.0f, 1.52f, 15.95f}}},  // 288 x 256
+    {6, {{1.189f, 1.562f, 1.08f, 12.132f}, {1.0f, 1.702f, 1.17f, 13.696f}, {1.515f, 1.764f, 1.285f, 12.444f}, {2.932f, 1.749f, 0.939f, 8.957f}, {kNever, 0, 0, 0}}},  // 288 x 192
+    {7, {{4.266f, 1.173f, 1.03f, 3.701f}, {1.0f, 1.311f, 1.035f, 7.162f}, {2.467f, 1.408f, 1.159f, 5.741f}, {1.0f, 1.665f, 1.163f, 6.544f}, {kNever, 0, 0, 0}}},  // 288 x 128
+    {10, {{1.271f, 0.864f, 0.635f, 5.553f}, {1.147f, 0.847f, 0.658f, 5.886f}, {1.0f, 0.941f, 0.673f, 6.701f}, {1.874f, 1.027f, 0.661f, 4.993f}, {0.33f, 0.0f, 0.719f, 5.47f}}},  // 144 x 128
+    {12, {{2.776f, 0.426f, 0.29f, 1.229f}, {3.462f, 0.048f, 0.321f, 1.476f}, {3.124f, 0.366f, 0.297f, 1.543f}, {2.774f, 0.451f, 0.356f, 1.199f}, {2.63f, 0.0f, 0.365f, 1.09f}}},  // 64 x 64
+    {13, {{4.031f, 0.537f, 0.381f, 0.729f}, {3.821f, 0.548f, 0.347f, 1.801f}, {4.921f, 0.451f, 0.401f, 0.873f}, {2.687f, 0.657f, 0.417f, 1.396f}, {3.44f, 0.0f, 0.409f, 1.09f}}},  // 96 x 64
+    {14, {{1.424f, 0.86f, 0.578f, 3.513f}, {1.441f, 0.891f, 0.565f, 4.015f}, {1.0f, 0.953f, 0.668f, 4.312f}, {2.397f, 1.034f, 0.623f, 3.504f}, {0.37f, 0.0f, 0.698f, 3.96f}}},  // 96 x 128
+    {15, {{1.459f, 0.968f, 0.666f, 4.871f}, {1.234f, 1.02f, 0.697f, 4.891f}, {1.0f, 1.099f, 0.834f, 5.475f}, {1.165f, 1.168f, 0.76f, 5.306f}, {-0.94f, 0.0f, 0.821f, 6.04f}}},  // 144 x 128
+    {16, {{1.398f, 0.69f, 0.479f, 3.573f}, {1.281f, 0.632f, 0.462f, 4.148f}, {1.0f, 0.758f, 0.522f, 4.254f}, {1.077f, 0.912f, 0.528f, 3.646f}, {0.78f, 0.0f, 0.578f, 3.62f}}},  // 144 x 64
+    {17, {{1.0f, 0.906f, 0.678f, 5.915f}, {1.0f, 1.016f, 0.734f, 5.922f}, {1.0f, 1.081f, 0.798f, 6.17f}, {1.0f, 1.168f, 0.769f, 5.721f}, {-0.86f, 0.0f, 0.786f, 6.93f}}},  // 192 x 128
+    {18, {{1.0f, 1.467f, 0.957f, 7.04f}, {1.0f, 1.453f, 1.089f, 6.551f}, {1.312f, 1.59f, 1.086f, 6.975f}, {1.134f, 1.657f, 1.165f, 6.459f}, {-1.76f, 0.0f, 1.109f, 8.54f}}},  // 192 x 192
+    {19, {{2.574f, 0.641f, 0.488f, 1.568f}, {2.824f, 0.624f, 0.431f, 2.125f}, {3.259f, 0.664f, 0.558f, 1.278f}, {2.249f, 0.941f, 0.573f, 1.725f}, {kNever, 0, 0, 0}}},  // 64 x 128
+    {20, {{4.255f, 1.263f, 1.022f, 3.738f}, {1.0f, 1.477f, 1.067f, 6.726f}, {1.136f, 1.601f, 1.15f, 7.089f}, {1.0f, 1.701f, 1.085f, 7.385f}, {-2.7f, 0.0f, 1.183f, 9.8f}}},  // 144 x 256
+    {21, {{1.0f, 1.679f, 1.353f, 6.95f}, {1.0f, 1.773f, 1.434f, 7.36f}, {kNever, 0, 0, 0}, {1.0f, 1.968f, 1.218f, 8.807f}, {-3.86f, 0.0f, 1.419f, 11.8f}}},  // 192 x 256
+    {22, {{1.0f, 1.568f, 1.217f, 9.125f}, {1.0f, 1.705f, 1.269f, 11.32f}, {kNever, 0, 0, 0}, {1.003f, 1.871f, 1.093f, 9.805f}, {-2.06f, 0.0f, 1.362f, 11.77f}}},  // 288 x 192
+    {23, {{1.916f, 1.028f, 0.796f, 6.023f}, {1.0f, 1.175f, 0.89f, 6.749f}, {2.392f, 1.206f, 0.948f, 6.589f}, {1.0f, 1.381f, 0.94f, 6.301f}, {-1.64f, 0.0f, 0.87f, 8.72f}}},  // 256 x 128
 };
 
-int cheapest_tile8(int64_t M, int64_t N, int64_t K, int splits, int kind, float* us) {
+int cheapest_tile8(int64_t M, int64_t N, int64_t K, int splits, int kind, int cls, float* us) {
   int best = 4;
   float best_us = kNever;
-  for (const TileCost<3>& c : kCosts8) {
+  for (const TileCost& c : kCosts8) {
     const Tile8& t = kTiles8[c.tile];
     if (t.no_fp8_epi && kind == OASIS_EPI_GELU_TANH_FP8) continue;
-    const float cost = tile_cost(c, t.bm, t.bn, M, N, K / splits / BK8, splits, cost_class(kind));
+    const float cost = tile_cost(c, t.bm, t.bn, M, N, K / splits / BK8, splits, cls);
     if (cost < best_us) {
       best_us = cost;
       best = c.tile;
@@ -587,7 +588,7 @@ int cheapest_tile8(int64_t M, int64_t N, int64_t K, int splits, int kind, float*
 
 // Default tile: with fp8 A the cheapest by kCosts8, with bf16 A the 4-wave tiles.
 int auto_tile8(int64_t M, int64_t N, int64_t K, int splits, bool aq, int kind) {
-  if (aq) return cheapest_tile8(M, N, K, splits, kind, nullptr);
+  if (aq) return cheapest_tile8(M, N, K, splits, kind, cost_class(kind), nullptr);
   return M >= 2048 ? 2 : (M >= 256 ? 3 : 4);
 }
 
@@ -653,7 +654,7 @@ int gemm_fp8_auto_splits(int64_t M, int64_t N, int64_t K, int max_splits) {
   for (int s = 1; s <= (max_splits < 8 ? max_splits : 8); s *= 2) {
     if ((K / BK8) % s != 0) break;
     float us;
-    cheapest_tile8(M, N, K, s, OASIS_EPI_PARTIAL_F32, &us);
+    cheapest_tile8(M, N, K, s, OASIS_EPI_PARTIAL_F32, COST_SPLIT, &us);
     if (s > 1) us += split_cost(M, N, s);
     if (us < best_us) {
       best_us = us;
