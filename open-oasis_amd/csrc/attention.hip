@@ -355,7 +355,8 @@ void flash_go(dim3 g, const T* q, const T* k, const T* v, T* o, const AttnArgs& 
 // Measured, before -> now: 576 tokens x 1, 2, 3, 4, 8 latents 9.9, 19.3, 20.1, 28.2, 44.8 -> 9.0, 13.2, 14.0, 18.4,
 // 29.1 us; 144 tokens x 1, 8, 12, 32, 64 frames 5.1, 8.1, 11.7, 15.8, 33.1 -> 4.8, 7.0, 8.5, 11.5, 23.7 (64 frames: 75 MB,
 // 3.2 TB/s).
-template <int NW, int KSPLIT, int KS, int ST, int CT, bool FINE = false>
+// TAIL: keys past the sequence in the last stage; their value rows are cleared.
+template <int NW, int KSPLIT, int KS, int ST, int CT, bool FINE, bool TAIL>
 __global__ __launch_bounds__(NW * KSPLIT * 64) void flash_ring_kernel(const bf16* __restrict__ Q,
                                                                       const bf16* __restrict__ K,
                                                                       const bf16* __restrict__ V, bf16* __restrict__ O,
@@ -414,7 +415,7 @@ __global__ __launch_bounds__(NW * KSPLIT * 64) void flash_ring_kernel(const bf16
     __builtin_amdgcn_s_waitcnt(WAIT);
     __builtin_amdgcn_s_barrier();
     if constexpr (ST > 1) issue(min(st + ST - 1, n - 1), (st + ST - 1) % ST);  // into the buffer read at st - 1
-    if ((st + 1) * KS > a.Lk) {  // the last key's value once only: against the 0 of a masked key an infinite one is NaN
+    if (TAIL && (st + 1) * KS > a.Lk) {  // the last key's value once only: against the 0 of a masked key an infinite one is NaN
       char* v0 = smem + (ST > 1 ? st % ST : 0) * STAGE + KS * 128;
       for (int i = (a.Lk - st * KS) * 8 + threadIdx.x; i < KS * 8; i += W * 64)
         *reinterpret_cast<f32x4*>(v0 + i * 16) = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -537,7 +538,11 @@ __global__ __launch_bounds__(NW * KSPLIT * 64) void flash_ring_kernel(const bf16
 template <int NW, int KSPLIT, int KS, int ST, int CT, bool FINE = false>
 int ring_go(const bf16* q, const bf16* k, const bf16* v, bf16* o, int64_t n_bh, const AttnArgs& a, hipStream_t s) {
   const dim3 grid((unsigned)((a.Lq + NW * 16 - 1) / (NW * 16)), (unsigned)n_bh, oasis::prefetch_any(&a.pf) ? 2 : 1);
-  hipLaunchKernelGGL((flash_ring_kernel<NW, KSPLIT, KS, ST, CT, FINE>), grid, dim3(NW * KSPLIT * 64), 0, s, q, k, v, o, a);
+  // whole frames without the tail: the two-frame step 1553 us, 1560 with it compiled in; elsewhere it costs nothing
+  constexpr bool WHOLE = KS == 144;
+  const auto fn = !WHOLE || a.Lk % KS ? &flash_ring_kernel<NW, KSPLIT, KS, ST, CT, FINE, true>
+                                      : &flash_ring_kernel<NW, KSPLIT, KS, ST, CT, FINE, !WHOLE>;
+  hipLaunchKernelGGL(fn, grid, dim3(NW * KSPLIT * 64), 0, s, q, k, v, o, a);
   return oasis::check_launch("attention");
 }
 
@@ -566,8 +571,8 @@ int flash_launch(const T* q, const T* k, const T* v, T* o, int64_t n_bh, const A
       // The smallest single stage that takes the sequence, beyond 192 keys a ring. Up to 160 keys the probabilities
       // keep their remainders, but with 256 heads of whole-frame or 64-row queries, which flash_kernel took in one
       // chunk: there 64 frames take 23.7 us without, 25.4 with them. 64-, 96- and 128-key stages keep short sequences
-      // from computing 144 (200 heads of 144 x 64: 9.1 us on flash_kernel, 6.7 on 96 keys, 5.6 on 64; 255 heads of 128 x 128: 8.0 us on flash_kernel, 8.8 on 144 keys, 6.9 on 128). At 160
-      // keys 64-query workgroups where 48-query ones would be more than two per CU, or one if 64 divides the
+      // from computing 144 (200 heads of 144 x 64: 9.1 us on flash_kernel, 6.7 on 96 keys, 5.6 on 64; 255 heads of
+      // 128 x 128: 8.0 us on flash_kernel, 8.8 on 144 keys, 6.9 on 128). At 160 keys 64-query workgroups where 48-query ones would be more than two per CU, or one if 64 divides the
       // queries (200 heads of 160 x 160: 48 9.2 us, 64 8.5; 64 x 160: 6.9, 5.7), else 48 (32 heads of 160 x 160:
       // 5.3, with 64 5.4). A ring with one workgroup per CU at most stages 128 keys (96 KB; 16 x 1000 x
       // 1000 13.2 us, with 64 15.3), with more of them 64 (48 KB, three per CU; 3 latents 14.6, with 128 18.3).
