@@ -1169,29 +1169,29 @@ constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
 // Fitted costs (tile_cost) of the tiles used above 320 tokens: c, lat, a and b of each class. The gated residual
 // of 256 x 256 spills registers (48): no choice.
 const TileCost kCosts[] = {
-    {1, {{3.092f, 0.249f, 0.142f, 0.477f}, {3.036f, 0.297f, 0.136f, 0.528f}, {3.211f, 0.26f, 0.146f, 0.669f}, {2.751f, 0.283f, 0.133f, 0.632f}, {kNever, 0, 0, 0}}},  // 32 x 64
-    {2, {{5.701f, 0.265f, 0.251f, 0.806f}, {4.642f, 0.344f, 0.308f, 1.088f}, {3.954f, 0.342f, 0.223f, 1.357f}, {2.876f, 0.313f, 0.239f, 1.302f}, {3.71f, 0.0f, 0.235f, 1.04f}}},  // 96 x 64
-    {3, {{4.198f, 0.274f, 0.181f, 0.377f}, {3.621f, 0.369f, 0.158f, 0.958f}, {3.268f, 0.284f, 0.183f, 1.119f}, {3.471f, 0.278f, 0.178f, 0.987f}, {3.45f, 0.0f, 0.181f, 0.79f}}},  // 64 x 64
-    {4, {{1.617f, 0.138f, 0.37f, 3.374f}, {1.131f, 0.28f, 0.336f, 4.601f}, {1.0f, 0.439f, 0.367f, 4.555f}, {2.328f, 0.464f, 0.363f, 3.11f}, {1.48f, 0.0f, 0.375f, 3.43f}}},  // 144 x 64
-    {5, {{2.645f, 1.701f, 1.299f, 8.322f}, {1.0f, 1.657f, 1.388f, 11.903f}, {4.24f, 1.666f, 1.311f, 11.182f}, {2.681f, 1.66f, 1.366f, 9.391f}, {kNever, 0, 0, 0}}},  // 288 x 256
-    {6, {{1.029f, 1.374f, 1.104f, 11.282f}, {kNever, 0, 0, 0}, {6.254f, 1.364f, 1.253f, 6.675f}, {1.007f, 1.43f, 1.128f, 9.35f}, {kNever, 0, 0, 0}}},  // 288 x 192
-    {7, {{1.0f, 1.071f, 0.967f, 6.218f}, {kNever, 0, 0, 0}, {1.0f, 0.447f, 0.994f, 7.76f}, {1.0f, 1.229f, 0.969f, 7.123f}, {kNever, 0, 0, 0}}},  // 288 x 128
-    {9, {{1.741f, 0.158f, 0.079f, 1.404f}, {2.46f, 0.191f, 0.113f, 0.904f}, {2.186f, 0.159f, 0.082f, 1.101f}, {2.666f, 0.131f, 0.08f, 0.824f}, {1.26f, 0.0f, 0.09f, 1.12f}}},  // 48 x 32
-    {10, {{2.248f, 0.097f, 0.134f, 2.493f}, {2.265f, 0.226f, 0.124f, 2.819f}, {1.501f, 0.244f, 0.138f, 3.303f}, {2.158f, 0.215f, 0.122f, 2.308f}, {1.48f, 0.0f, 0.147f, 2.28f}}},  // 48 x 64
-    {11, {{1.872f, 0.249f, 0.156f, 2.893f}, {2.147f, 0.265f, 0.142f, 3.13f}, {1.145f, 0.055f, 0.182f, 3.25f}, {1.881f, 0.257f, 0.147f, 2.774f}, {1.47f, 0.0f, 0.172f, 2.71f}}},  // 64 x 64
-    {12, {{1.801f, 0.18f, 0.108f, 1.898f}, {1.665f, 0.289f, 0.099f, 2.162f}, {1.596f, 0.191f, 0.111f, 2.265f}, {1.618f, 0.261f, 0.105f, 1.876f}, {1.45f, 0.0f, 0.113f, 1.86f}}},  // 32 x 64
-    {18, {{1.0f, 0.264f, 0.47f, 4.945f}, {1.0f, 0.591f, 0.487f, 5.516f}, {1.0f, 0.257f, 0.461f, 6.464f}, {1.0f, 0.346f, 0.459f, 5.389f}, {0.79f, 0.0f, 0.528f, 5.23f}}},  // 144 x 128
-    {19, {{6.411f, 0.662f, 0.575f, 0.859f}, {5.758f, 0.761f, 0.573f, 2.272f}, {kNever, 0, 0, 0}, {4.758f, 1.125f, 0.551f, 2.192f}, {3.35f, 0.0f, 0.684f, 3.14f}}},  // 192 x 128
-    {20, {{2.151f, 0.774f, 0.656f, 4.377f}, {1.0f, 0.156f, 0.658f, 6.418f}, {1.0f, 0.855f, 0.668f, 7.057f}, {4.068f, 0.729f, 0.56f, 5.209f}, {0.74f, 0.0f, 0.626f, 6.26f}}},  // 192 x 128
-    {21, {{1.0f, 0.692f, 0.798f, 6.894f}, {1.0f, 0.944f, 0.821f, 7.778f}, {1.0f, 0.96f, 0.823f, 8.612f}, {1.0f, 1.039f, 0.794f, 7.839f}, {-0.86f, 0.0f, 0.838f, 9.16f}}},  // 144 x 256
-    {22, {{1.001f, 0.936f, 0.79f, 6.051f}, {1.0f, 1.039f, 0.839f, 7.202f}, {1.0f, 0.524f, 0.829f, 8.42f}, {1.0f, 1.039f, 0.74f, 7.581f}, {-0.25f, 0.0f, 0.866f, 7.63f}}},  // 192 x 192
-    {23, {{1.443f, 0.466f, 0.406f, 3.666f}, {1.235f, 0.504f, 0.419f, 4.305f}, {2.048f, 0.474f, 0.444f, 4.658f}, {2.088f, 0.902f, 0.413f, 3.533f}, {1.61f, 0.0f, 0.429f, 3.57f}}},  // 96 x 128
-    {24, {{4.714f, 0.576f, 0.331f, 0.846f}, {4.479f, 0.648f, 0.332f, 1.409f}, {5.866f, 0.647f, 0.335f, 1.075f}, {3.976f, 0.666f, 0.378f, 1.866f}, {5.18f, 0.0f, 0.459f, 0.89f}}},  // 96 x 128
-    {25, {{1.002f, 0.557f, 0.489f, 4.349f}, {1.504f, 0.088f, 0.504f, 4.74f}, {1.0f, 0.571f, 0.465f, 5.7f}, {1.424f, 0.625f, 0.479f, 4.376f}, {1.14f, 0.0f, 0.49f, 4.6f}}},  // 128 x 128
-    {26, {{3.027f, 1.243f, 1.276f, 6.532f}, {3.287f, 0.057f, 1.178f, 7.424f}, {kNever, 0, 0, 0}, {1.0f, 1.006f, 1.097f, 10.68f}, {-2.81f, 0.0f, 1.197f, 13.58f}}},  // 256 x 256
-    {27, {{4.511f, 1.135f, 1.488f, 4.944f}, {1.0f, 0.984f, 1.442f, 10.175f}, {4.601f, 1.534f, 1.374f, 8.986f}, {2.384f, 0.809f, 1.352f, 10.157f}, {-4.66f, 0.0f, 1.369f, 16.58f}}},  // 288 x 256
-    {28, {{1.0f, 0.76f, 0.712f, 6.364f}, {1.0f, 0.644f, 0.74f, 7.132f}, {1.142f, 0.865f, 0.638f, 8.68f}, {1.186f, 0.968f, 0.667f, 7.907f}, {-0.57f, 0.0f, 0.702f, 9.04f}}},  // 256 x 128
-    {29, {{1.346f, 0.535f, 0.465f, 4.389f}, {1.597f, 0.55f, 0.465f, 4.803f}, {kNever, 0, 0, 0}, {1.816f, 0.602f, 0.458f, 4.152f}, {1.31f, 0.0f, 0.467f, 4.25f}}},  // 144 x 96
+    {1, {{2.99f, 0.253f, 0.14f, 0.473f}, {3.036f, 0.297f, 0.136f, 0.528f}, {3.285f, 0.256f, 0.141f, 0.729f}, {2.565f, 0.307f, 0.134f, 0.671f}, {kNever, 0, 0, 0}}},  // 32 x 64
+    {2, {{5.114f, 0.274f, 0.246f, 1.04f}, {4.642f, 0.344f, 0.308f, 1.088f}, {3.953f, 0.341f, 0.232f, 1.316f}, {2.667f, 0.359f, 0.218f, 1.509f}, {3.71f, 0.0f, 0.235f, 1.04f}}},  // 96 x 64
+    {3, {{4.077f, 0.27f, 0.164f, 0.464f}, {3.621f, 0.369f, 0.158f, 0.958f}, {3.573f, 0.271f, 0.183f, 1.062f}, {3.314f, 0.286f, 0.177f, 1.053f}, {3.45f, 0.0f, 0.181f, 0.79f}}},  // 64 x 64
+    {4, {{1.623f, 0.075f, 0.37f, 3.371f}, {1.131f, 0.28f, 0.336f, 4.601f}, {1.076f, 0.059f, 0.366f, 4.621f}, {2.34f, 0.464f, 0.365f, 3.069f}, {1.48f, 0.0f, 0.375f, 3.43f}}},  // 144 x 64
+    {5, {{1.939f, 1.704f, 1.288f, 9.643f}, {1.0f, 1.657f, 1.388f, 11.903f}, {1.662f, 1.723f, 1.43f, 12.995f}, {3.672f, 1.593f, 1.233f, 8.63f}, {kNever, 0, 0, 0}}},  // 288 x 256
+    {6, {{1.714f, 1.353f, 1.065f, 10.648f}, {kNever, 0, 0, 0}, {4.511f, 0.386f, 1.259f, 9.797f}, {1.0f, 1.501f, 1.177f, 9.516f}, {kNever, 0, 0, 0}}},  // 288 x 192
+    {7, {{1.0f, 1.058f, 0.945f, 6.611f}, {kNever, 0, 0, 0}, {3.147f, 1.069f, 0.967f, 5.741f}, {1.629f, 1.209f, 0.951f, 7.001f}, {kNever, 0, 0, 0}}},  // 288 x 128
+    {9, {{1.783f, 0.175f, 0.083f, 1.285f}, {2.46f, 0.191f, 0.113f, 0.904f}, {2.173f, 0.16f, 0.081f, 1.116f}, {2.511f, 0.138f, 0.081f, 0.84f}, {1.26f, 0.0f, 0.09f, 1.12f}}},  // 48 x 32
+    {10, {{2.067f, 0.216f, 0.134f, 2.542f}, {2.265f, 0.226f, 0.124f, 2.819f}, {1.503f, 0.244f, 0.138f, 3.295f}, {1.945f, 0.22f, 0.115f, 2.436f}, {1.48f, 0.0f, 0.147f, 2.28f}}},  // 48 x 64
+    {11, {{1.878f, 0.198f, 0.157f, 2.884f}, {2.147f, 0.265f, 0.142f, 3.13f}, {1.019f, 0.287f, 0.165f, 3.759f}, {1.819f, 0.257f, 0.148f, 2.776f}, {1.47f, 0.0f, 0.172f, 2.71f}}},  // 64 x 64
+    {12, {{1.662f, 0.184f, 0.108f, 1.921f}, {1.665f, 0.289f, 0.099f, 2.162f}, {1.604f, 0.19f, 0.111f, 2.264f}, {2.014f, 0.236f, 0.104f, 1.84f}, {1.45f, 0.0f, 0.113f, 1.86f}}},  // 32 x 64
+    {18, {{1.0f, 0.544f, 0.466f, 4.94f}, {1.0f, 0.591f, 0.487f, 5.516f}, {1.0f, 0.189f, 0.466f, 6.334f}, {1.15f, 0.429f, 0.562f, 5.0f}, {0.79f, 0.0f, 0.528f, 5.23f}}},  // 144 x 128
+    {19, {{5.551f, 0.753f, 0.572f, 2.116f}, {5.758f, 0.761f, 0.573f, 2.272f}, {kNever, 0, 0, 0}, {3.859f, 0.889f, 0.528f, 4.053f}, {3.35f, 0.0f, 0.684f, 3.14f}}},  // 192 x 128
+    {20, {{1.0f, 0.402f, 0.617f, 5.595f}, {1.0f, 0.156f, 0.658f, 6.418f}, {1.0f, 0.743f, 0.632f, 6.833f}, {1.0f, 0.16f, 0.646f, 5.766f}, {0.74f, 0.0f, 0.626f, 6.26f}}},  // 192 x 128
+    {21, {{1.0f, 0.098f, 0.796f, 7.209f}, {1.0f, 0.944f, 0.821f, 7.778f}, {2.229f, 0.111f, 0.833f, 7.731f}, {1.0f, 0.452f, 0.828f, 8.122f}, {-0.86f, 0.0f, 0.838f, 9.16f}}},  // 144 x 256
+    {22, {{2.68f, 0.447f, 0.819f, 4.497f}, {1.0f, 1.039f, 0.839f, 7.202f}, {1.0f, 0.052f, 0.851f, 8.385f}, {1.927f, 1.054f, 0.728f, 7.352f}, {-0.25f, 0.0f, 0.866f, 7.63f}}},  // 192 x 192
+    {23, {{1.456f, 0.466f, 0.406f, 3.654f}, {1.235f, 0.504f, 0.419f, 4.305f}, {2.276f, 0.231f, 0.46f, 4.385f}, {2.118f, 0.882f, 0.399f, 3.641f}, {1.61f, 0.0f, 0.429f, 3.57f}}},  // 96 x 128
+    {24, {{3.947f, 0.684f, 0.37f, 1.772f}, {4.479f, 0.648f, 0.332f, 1.409f}, {4.813f, 0.668f, 0.456f, 2.043f}, {3.518f, 0.737f, 0.391f, 2.637f}, {5.18f, 0.0f, 0.459f, 0.89f}}},  // 96 x 128
+    {25, {{1.042f, 0.555f, 0.481f, 4.418f}, {1.504f, 0.088f, 0.504f, 4.74f}, {1.0f, 0.57f, 0.473f, 5.635f}, {1.323f, 0.326f, 0.47f, 4.482f}, {1.14f, 0.0f, 0.49f, 4.6f}}},  // 128 x 128
+    {26, {{3.5f, 0.611f, 1.235f, 6.144f}, {3.287f, 0.057f, 1.178f, 7.424f}, {kNever, 0, 0, 0}, {2.434f, 1.27f, 1.166f, 9.311f}, {-2.81f, 0.0f, 1.197f, 13.58f}}},  // 256 x 256
+    {27, {{2.778f, 1.136f, 1.365f, 8.189f}, {1.0f, 0.984f, 1.442f, 10.175f}, {1.518f, 1.015f, 1.46f, 12.182f}, {1.0f, 1.677f, 1.267f, 11.269f}, {-4.66f, 0.0f, 1.369f, 16.58f}}},  // 288 x 256
+    {28, {{1.411f, 0.559f, 0.74f, 6.083f}, {1.0f, 0.644f, 0.74f, 7.132f}, {1.07f, 0.773f, 0.766f, 8.413f}, {1.531f, 0.971f, 0.714f, 7.846f}, {-0.57f, 0.0f, 0.702f, 9.04f}}},  // 256 x 128
+    {29, {{1.521f, 0.318f, 0.462f, 4.243f}, {1.597f, 0.55f, 0.465f, 4.803f}, {kNever, 0, 0, 0}, {1.777f, 0.596f, 0.452f, 4.189f}, {1.31f, 0.0f, 0.467f, 4.25f}}},  // 144 x 96
 };
 
 // the K / splits a tile can run (as gemm_launch_cfg checks it)

@@ -95,8 +95,11 @@ __device__ __forceinline__ void grouped_tile(int pid, int Mt, int Nt, int GN, in
 // picked tile over that of the fastest, and over that of the rule by width that came before. It is what the width
 // alone could not say: 1440 x 4096 in 144 x 64 tiles is 640 workgroups, three rounds of 256 of which the last is half
 // empty (29.8 us), in 192 x 128 tiles 256 workgroups (19.0 us). Over those shapes the tile it picks takes 1.004
-// times the fastest of all in the mean, 1.17 (fp8: 1.28) at worst. Over 4142 others drawn at random 1.4 % run more
-// than 2 % slower than by the width (0.83 at worst: 344 x 4800 x 3584 in fp8), all together 1.38 times as fast.
+// times the fastest of all in the mean, 1.17 (fp8: 1.28) at worst. But for QKV the bf16 tiles of two workgroups per CU
+// count 10 % longer than launches of one product in a row take on them: between other kernels they do (FC1 of 1440
+// rows 17.8 us in a row on 96 x 128, 18.8 on 192 x 128, yet the step is 2.1 us a sub-block slower on the former). Over
+// 8924 shapes, half of them drawn at random, 1.2 % run more than 2 % slower than by the width (0.83 at worst: 344 x 4800 x
+// 3584 in fp8), all together 1.31 times as fast.
 // COST_SPLIT: partial sums by an earlier fit to the DiT's O and FC2 products, with which split-K counts are chosen.
 enum { COST_STORE = 0, COST_QKV = 1, COST_RES = 2, COST_PART = 3, COST_SPLIT = 4 };
 struct TileCost {
